@@ -552,8 +552,10 @@ static long long small_nodes_bound() {
 }
 
 // after a change of the level matrices: the FP32 lattice values of every
-// level (1/a_ii of the FP64 form is recomputed on its first use)
-static void refresh_f32(cd3d_problem &P) {
+// level (1/a_ii of the FP64 form is recomputed on its first use); values
+// false: no per-node FP32 values of affine levels (the FP64 form evaluates
+// the affine stencils)
+static void refresh_f32(cd3d_problem &P, bool values = true) {
   for (size_t l = 0; l < P.dl.size(); l++) {
     DevLevel &D = P.dl[l];
     D.invdiag_ok = false;  // only the FP64 smoother reads it: computed there on first use
@@ -570,7 +572,7 @@ static void refresh_f32(cd3d_problem &P) {
         }
       };
       const long long nn = D.nn;
-      if (D.lat_fresh == 2 && nn * nn * nn > small_nodes_bound()) {
+      if (D.lat_fresh == 2 && (!values || nn * nn * nn > small_nodes_bound())) {
         // affine class stencils evaluated by the sweeps node by node (a level
         // this large never runs in the one-workgroup program, which reads
         // per-node values)
@@ -752,69 +754,127 @@ void cycle64(VC &v, int i, bool zero_start) {
   if (x != L.sol) k_copy(P.stream, L.ndof, x, L.sol);
 }
 
-// mixed precision on the lattice-stencil form: the same cycle, with vectors
-// in node-lattice order whose boundary entries are zero (the Dirichlet part
-// of every preconditioner rhs and iterate vanishes)
+// The lattice-stencil form of the same cycle: FP32 in the mixed form, FP64 in
+// the plain form where every level's matrix is its class stencils
+// (lattice64_ok).  Vectors are in node-lattice order with zero boundary
+// entries (the Dirichlet part of every preconditioner rhs and iterate
+// vanishes).  The FP64 vectors live in the level's DOF-ordered work vectors
+// (every lattice node is a DOF); the coarsest level keeps sol and rhs for the
+// DOF-ordered coarse solve and takes tmp and aux.
+template <typename T>
+struct LatVecs {
+  T *x, *f, *a, *t;
+};
+template <typename T>
+LatVecs<T> lat_vecs(const DevLevel &L, int level);
+template <>
+LatVecs<float> lat_vecs<float>(const DevLevel &L, int) {
+  return {L.lx, L.lf, L.la, L.lt};
+}
+template <>
+LatVecs<double> lat_vecs<double>(const DevLevel &L, int level) {
+  if (level == 0) return {L.tmp, L.aux, nullptr, nullptr};
+  return {L.sol, L.rhs, L.aux, L.tmp};
+}
+
+template <typename T>
 void coarseL(VC &v, bool zero_start) {
   DevLevel &C = v.P.dl[0];
+  const LatVecs<T> c = lat_vecs<T>(C, 0);
   if (zero_start && v.sp.coarse_smoother == 17) {
     // inside the preconditioner the Dirichlet data are zero, so the defect of
     // the zero iterate is the rhs: one launch, same arithmetic as below
     coarse_join(v.P);
-    k_coarse_from_lattice(v.P.stream, C, v.P.cinv, C.lf, C.lx);
+    k_coarse_from_lattice<T>(v.P.stream, C, v.P.cinv, c.f, c.x);
     return;
   }
-  kl_to_dof(v.P.stream, C, C.lf, C.rhs);
-  if (!zero_start) kl_to_dof(v.P.stream, C, C.lx, C.sol);
+  kl_to_dof<T>(v.P.stream, C, c.f, C.rhs);
+  if (!zero_start) kl_to_dof<T>(v.P.stream, C, c.x, C.sol);
   coarse64(v, zero_start);
-  kl_from_dof(v.P.stream, C, C.sol, C.lx);
+  kl_from_dof<T>(v.P.stream, C, C.sol, c.x);
 }
 
-void cycleL(VC &v, int i, bool zero_start) {
+// ftop, ztop: the finest level's rhs and result when they are not the level's
+// own vectors
+template <typename T>
+void cycleL(VC &v, int i, bool zero_start, const T *ftop = nullptr, T *ztop = nullptr) {
   cd3d_problem &P = v.P;
   if (i == 0) {
-    coarseL(v, zero_start);
+    coarseL<T>(v, zero_start);
     return;
   }
-  if (v.small < 0) v.small = small_top(P, v.sp);
-  if (zero_start && i == v.small) {
-    coarse_join(P);
-    kl_small_vcycle(P.stream, P.dl.data(), i, P.mesh.order, v.sp.pre, v.sp.post, (float)v.sp.omega,
-                    (float)v.sp.gmg_damp, P.cinv);
-    return;
+  if constexpr (sizeof(T) == 4) {
+    if (v.small < 0) v.small = small_top(P, v.sp);
+    if (zero_start && i == v.small) {
+      coarse_join(P);
+      kl_small_vcycle(P.stream, P.dl.data(), i, P.mesh.order, v.sp.pre, v.sp.post, (float)v.sp.omega,
+                      (float)v.sp.gmg_damp, P.cinv);
+      return;
+    }
   }
   DevLevel &L = P.dl[i], &C = P.dl[i - 1];
   const int p = P.mesh.order;
-  float *x = L.lx, *t = L.lt;
-  const float om = (float)v.sp.omega;
+  const LatVecs<T> l = lat_vecs<T>(L, i), c = lat_vecs<T>(C, i - 1);
+  const T *f = ftop ? ftop : l.f;
+  T *x = l.x, *t = l.t;
+  const T om = (T)v.sp.omega;
   const bool ready = zero_start && (v.zero_ready >> i & 1u);
   v.zero_ready &= ~(1u << i);
   for (int k = 0; k < v.sp.pre; k++) {
     if (k == 0 && zero_start) {
-      if (!ready) kl_jacobi_zero(P.stream, L, p, L.lf, t, om);
+      if (!ready) kl_jacobi_zero<T>(P.stream, L, p, f, t, om);
     } else {
-      kl_jacobi(P.stream, L, p, x, L.lf, t, om);
+      kl_jacobi<T>(P.stream, L, p, x, f, t, om);
     }
     std::swap(x, t);
   }
   const size_t nn3 = (size_t)L.nn * L.nn * L.nn;
-  if (v.sp.pre == 0 && zero_start) HIPCHK(hipMemsetAsync(x, 0, sizeof(float) * nn3, P.stream));
-  kl_defect(P.stream, L, p, x, L.lf, L.la);
+  if (v.sp.pre == 0 && zero_start) HIPCHK(hipMemsetAsync(x, 0, sizeof(T) * nn3, P.stream));
+  kl_defect<T>(P.stream, L, p, x, f, l.a);
   // the coarse level's zero-start sweep rides on the restriction when that
   // level runs the launch-per-sweep cycle (not the direct solve of level 0 or
   // the one-launch bottom) with uniform stencils
   const bool fuse = v.fuse_zero && v.sp.pre > 0 && i - 1 > 0 && i - 1 != v.small && i - 1 < 32 &&
                     kl_zero_sweep_fusable(C);
-  kl_restrict(P.stream, L, C, p, L.la, C.lf, fuse ? C.lt : nullptr, om);
+  kl_restrict<T>(P.stream, L, C, p, l.a, c.f, fuse ? c.t : nullptr, om);
   if (fuse) v.zero_ready |= 1u << (i - 1);
-  for (int r = 0; r < v.rec[i]; r++) cycleL(v, i - 1, r == 0);
+  for (int r = 0; r < v.rec[i]; r++) cycleL<T>(v, i - 1, r == 0);
   if (v.sp.cycle < 1) v.rec[i] = 1;  // F-cycle
-  kl_prolong_update(P.stream, L, C, p, C.lx, x, (float)v.sp.gmg_damp);
+  kl_prolong_update<T>(P.stream, L, C, p, c.x, x, (T)v.sp.gmg_damp);
   for (int k = 0; k < v.sp.post; k++) {
-    kl_jacobi(P.stream, L, p, x, L.lf, t, om);
-    std::swap(x, t);
+    T *o = ztop && k + 1 == v.sp.post ? ztop : t;
+    kl_jacobi<T>(P.stream, L, p, x, f, o, om);
+    if (o == t) std::swap(x, t);
+    else x = o;
   }
-  if (x != L.lx) HIPCHK(hipMemcpyAsync(L.lx, x, sizeof(float) * nn3, hipMemcpyDeviceToDevice, P.stream));
+  T *dst = ztop ? ztop : l.x;
+  if (x != dst) HIPCHK(hipMemcpyAsync(dst, x, sizeof(T) * nn3, hipMemcpyDeviceToDevice, P.stream));
+}
+
+// CD3D_FP64_LATTICE=0: the plain form keeps CSR products on every level
+bool fp64_lattice_on() {
+  const char *e = getenv("CD3D_FP64_LATTICE");
+  return !(e && e[0] == '0');
+}
+
+// The plain form runs on the lattice where the class stencils are exactly
+// the CSR values on every level above the coarsest (constant coefficients or
+// the rotating field, assembled through class stencils): the same matrices
+// and smoother in FP64, 16-24 bytes per unknown and product instead of 12
+// per nonzero (Q2 64^3 cells, fine level: CSR Jacobi sweep 350 us, 1.6 GB).
+// Assemble + solve Q2 64^3 79.5 -> 13.7 ms, three TCD3D steps Q1 128^3 34.8
+// -> 13.8 ms.  Other levels (per-point coefficients, general hexahedra,
+// entries set by the caller) and smoothers keep the CSR form.
+bool lattice64_ok(const cd3d_problem &P, const cd3d_solver_params &sp) {
+  if (sp.precision != CD3D_FP64 || P.dl.size() < 2 || sp.smoother != 1 || !fp64_lattice_on()) return false;
+  for (size_t l = 1; l < P.dl.size(); l++)
+    if (P.dl[l].nclass <= 0 || !(P.dl[l].lat_exact64 || P.dl[l].lat_aff64)) return false;
+  return true;
+}
+
+// the FP64 lattice vectors of every level start with zero boundary entries
+void clear_lattice64(cd3d_problem &P) {
+  for (DevLevel &D : P.dl) kl_clear_boundary4(P.stream, D, D.sol, D.rhs, D.aux, D.tmp);
 }
 
 // TMultiGridScaIte::Iterate (MultiGridScaIte.C:63-104): z = V(r), zero start.
@@ -826,9 +886,16 @@ void precondition(VC &v, const double *r, double *z, bool rhs_dirichlet_zero) {
   const int top = (int)P.dl.size() - 1;
   DevLevel &F = P.dl[top];
   if (v.sp.precision == CD3D_MIXED && top > 0 && rhs_dirichlet_zero && v.sp.smoother == 1) {
-    kl_from_dof(P.stream, F, r, F.lf);
-    cycleL(v, top, true);
-    kl_to_dof(P.stream, F, F.lx, z);
+    kl_from_dof<float>(P.stream, F, r, F.lf);
+    cycleL<float>(v, top, true);
+    kl_to_dof<float>(P.stream, F, F.lx, z);
+    return;
+  }
+  if (rhs_dirichlet_zero && lattice64_ok(P, v.sp)) {
+    clear_lattice64(P);
+    kl_from_dof<double>(P.stream, F, r, F.rhs);
+    cycleL<double>(v, top, true);
+    kl_to_dof<double>(P.stream, F, F.sol, z);
     return;
   }
   k_copy(P.stream, F.ndof, r, F.rhs);
@@ -887,6 +954,8 @@ struct Space {
   // orthogonalise by the low-synchronisation form of MGS (k_ls_step)
   // instead of MGS step by step (the FP64 form keeps the reference's MGS)
   bool lowsync = false;
+  // before the iteration, once the Krylov space (R columns) is there
+  std::function<void(int)> prepare;
 };
 
 Space dof_space(cd3d_problem &P) {
@@ -924,8 +993,33 @@ Space lattice_space(cd3d_problem &P) {
     v.reset();
     if (r32_state == 0) kl_cast_d2f(P.stream, F.ndof, r, F.lf);
     if (r32_state == 2 && top < 32) v.zero_ready |= 1u << top;
-    cycleL(v, top, true);
+    cycleL<float>(v, top, true);
     if (z) kl_cast_f2d(P.stream, F.ndof, F.lx, z);
+  };
+  return S;
+}
+
+// the plain form in lattice order (lattice64_ok): the V-cycle reads each
+// Krylov vector in place and its last sweep writes the column of Z
+Space lattice64_space(cd3d_problem &P) {
+  DevLevel &F = P.dl.back();
+  const int p = P.mesh.order, top = (int)P.dl.size() - 1;
+  Space S;
+  S.n = F.ndof;
+  S.x = P.xl;
+  S.b = P.bl;
+  S.defect = [&P, &F, p](const double *x, const double *f, double *d) { kl_defect64(P.stream, F, p, x, f, d); };
+  S.matvec = [&P, &F, p](const double *x, double *y) { kl_spmv64(P.stream, F, p, x, y); };
+  S.lat_top = &F;
+  S.lat_order = p;
+  S.prepare = [&P, &F](int R) {
+    clear_lattice64(P);
+    kl_clear_boundary(P.stream, F, P.Z, P.krylov_ld, R);  // the sweeps write interior nodes only
+  };
+  S.precond = [top](VC &v, const double *r, double *z, int state) {
+    v.reset();
+    if (state == 2 && top < 32) v.zero_ready |= 1u << top;
+    cycleL<double>(v, top, true, r, z);
   };
   return S;
 }
@@ -974,13 +1068,15 @@ int fgmres_iterate(cd3d_problem &P, const cd3d_solver_params &sp, const Space &S
   // vector's FP32 copy (TopZeroSweep); CD3D_FUSE_ZERO_SWEEP=0: launched
   TopZeroSweep zt{};
   bool topz = false;
-  if (S.lat_top && S.r32 && sp.pre > 0) {
+  if (S.lat_top && sp.pre > 0) {
     const char *ez = getenv("CD3D_FUSE_ZERO_SWEEP");
     if (!(ez && ez[0] == '0'))
-      topz = kl_top_zero_sweep(*S.lat_top, S.lat_order, (float)sp.omega, S.lat_top->lt, zt);
+      topz = S.r32 ? kl_top_zero_sweep(*S.lat_top, S.lat_order, (float)sp.omega, S.lat_top->lt, zt)
+                   : kl_top_zero_sweep(*S.lat_top, S.lat_order, sp.omega, S.lat_top->tmp, zt);
   }
   const TopZeroSweep *ztp = topz ? &zt : nullptr;
-  const int r32_state = S.r32 ? (topz ? 2 : 1) : 0;
+  const int r32_state = topz ? 2 : S.r32 ? 1 : 0;
+  if (S.prepare) S.prepare(R);
   S.defect(S.x, S.b, Vk(0));
   double beta = dev_norm(P, N, Vk(0));
   r0 = beta;
@@ -1836,14 +1932,16 @@ cd3d_status cd3d_solve(cd3d_problem *p, const cd3d_solver_params *sp, const doub
     double r0 = 0;
     int its;
     const int top = (int)p->dl.size() - 1;
-    if (sp->precision == CD3D_MIXED && top > 0 && sp->smoother == 1 && (F.lat_exact64 || F.lat_aff64)) {
+    const bool lat64 = lattice64_ok(*p, *sp);
+    if (lat64 ||
+        (sp->precision == CD3D_MIXED && top > 0 && sp->smoother == 1 && (F.lat_exact64 || F.lat_aff64))) {
       if (!p->xl) {
         p->xl = dalloc<double>(*p, N);
         p->bl = dalloc<double>(*p, N);
       }
       kl_dof_to_lat64(p->stream, F, p->bs, p->bl);
       kl_dof_to_lat64(p->stream, F, p->xs, p->xl);
-      its = fgmres(*p, *sp, lattice_space(*p), r0, solve_status);
+      its = fgmres(*p, *sp, lat64 ? lattice64_space(*p) : lattice_space(*p), r0, solve_status);
       kl_lat64_to_dof(p->stream, F, p->xl, p->xs);
     } else {
       its = fgmres(*p, *sp, dof_space(*p), r0, solve_status);
@@ -2020,15 +2118,15 @@ static int tcd_step_impl(cd3d_problem &P, const cd3d_coeffs &co0, const cd3d_sol
   k_copy(P.stream, N, P.xs, P.tcd_oldsol);
   cd3d_coeffs co = co0;
   co.t = P.tcd_t + tau;
-  // The mixed form works on the lattice wherever the assembled matrices are
+  // Both forms work on the lattice wherever the assembled matrices are
   // affine class stencils with a uniform mass matrix (rotating field): there
   // the system matrix fma(tau th1, A, M) and the rhs matrix
   // fma(-tau th2, A, M) are evaluated entry by entry from the stencils by the
-  // FP32 sweeps and the FP64 lattice operator, with the arithmetic of the CSR
+  // sweeps and the FP64 lattice operator, with the arithmetic of the CSR
   // path, so levels above the coarsest get no CSR values.  The coarsest level
   // keeps its CSR system matrix for the exact coarse solve.
   const bool affine_asm = co.conv_kind == 1 && co.f_kind == 0 && !co.supg && !uniform_assembly_off(P);
-  bool lattice = sp.precision == CD3D_MIXED && Lf > 0 && affine_asm && sp.smoother == 1;
+  bool lattice = (sp.precision == CD3D_MIXED || fp64_lattice_on()) && Lf > 0 && affine_asm && sp.smoother == 1;
   for (int l = 1; l <= Lf; l++) lattice = lattice && P.dl[l].tcd_mass_uniform && P.dl[l].nclass > 0;
   // AssembleARhs at t_new (SystemTCD3D.C:204-226); with SUPG the A and rhs of
   // MatricesAKRhsAssemble_SUPG (TCD3D.C:102) and its time-derivative matrix
@@ -2110,19 +2208,20 @@ static int tcd_step_impl(cd3d_problem &P, const cd3d_coeffs &co0, const cd3d_sol
     D.lat_alpha_m = 1.0;
     D.lat_alpha = tau * th1;
   }
-  refresh_f32(P);
-  // Solve (SystemTCD3D.C:317-376); the mixed form runs FGMRES in lattice
-  // order when the FP64 lattice operator is exactly the system matrix
+  refresh_f32(P, sp.precision == CD3D_MIXED);
+  // Solve (SystemTCD3D.C:317-376); FGMRES runs in lattice order when the FP64
+  // lattice operator is exactly the system matrix
   double r0;
   int its;
-  if (sp.precision == CD3D_MIXED && Lf > 0 && sp.smoother == 1 && (F.lat_exact64 || F.lat_aff64)) {
+  const bool lat64 = lattice64_ok(P, sp);
+  if (lat64 || (sp.precision == CD3D_MIXED && Lf > 0 && sp.smoother == 1 && (F.lat_exact64 || F.lat_aff64))) {
     if (!P.xl) {
       P.xl = dalloc<double>(P, N);
       P.bl = dalloc<double>(P, N);
     }
     kl_dof_to_lat64(P.stream, F, P.bs, P.bl);
     kl_dof_to_lat64(P.stream, F, P.xs, P.xl);
-    its = fgmres(P, sp, lattice_space(P), r0, solve_status, rf_out);
+    its = fgmres(P, sp, lat64 ? lattice64_space(P) : lattice_space(P), r0, solve_status, rf_out);
     kl_lat64_to_dof(P.stream, F, P.xl, P.xs);
   } else {
     its = fgmres(P, sp, dof_space(P), r0, solve_status, rf_out);
@@ -2447,7 +2546,7 @@ cd3d_status cd3d_kernel_bench(cd3d_problem *p, int which, int level, int reps, d
         DevLevel &C = p->dl[level - 1];
         const double nc = (double)C.nn * C.nn * C.nn;
         if (which == 3) {
-          launch = [&] { kl_restrict(p->stream, L, C, o, L.la, C.lf); };
+          launch = [&] { kl_restrict<float>(p->stream, L, C, o, L.la, C.lf, nullptr, 0.f); };
           b = 4 * N + 4 * nc;
         } else {
           launch = [&] { kl_prolong_update(p->stream, L, C, o, C.lx, L.lt, 1.0f); };

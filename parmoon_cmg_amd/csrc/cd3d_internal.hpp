@@ -312,13 +312,17 @@ void k_axpy_dot(hipStream_t s, int n, const double *alpha_partials, double sign,
 // beside the FP32 copy of a Krylov vector (which is that V-cycle's rhs f):
 // x[e] = omega f[e] d[c dstride] at the interior lattice nodes e (1 <= X,
 // Y, Z <= nn - 2), c the node's parity class (X & 1) + 2 (Y & 1) + 4 (Z & 1)
-// for Q2, 0 for Q1; other entries untouched.  x == nullptr: none.
+// for Q2, 0 for Q1; other entries untouched.  x == nullptr (and x64): none.
 struct TopZeroSweep {
   float *x = nullptr;
   const float *d = nullptr;
   int dstride = 0;
   float omega = 0.f;
   int nn = 0, order = 0;
+  // the FP64 V-cycle's sweep, from the FP64 Krylov vector itself
+  double *x64 = nullptr;
+  const double *d64 = nullptr;
+  double omega64 = 0.0;
 };
 // zt: the finest level's zero-start sweep beside y32 (y32 in lattice order)
 void k_scale_copy(hipStream_t s, int n, const double *partials, double *norm_out, const double *x, double *y,
@@ -467,26 +471,36 @@ int k_errors_blocks(int ncell);
 void k_errors(hipStream_t s, const DevLevel &L, int order, const double *tab, const double *u, const FnParams &f,
               double *partials, double *out);
 // ---------------------------------------------------------------- lattice form (lattice.hip)
-void kl_jacobi(hipStream_t s, const DevLevel &L, int order, const float *x, const float *f, float *out,
-               float omega);
-void kl_jacobi_zero(hipStream_t s, const DevLevel &L, int order, const float *f, float *out, float omega);
-void kl_defect(hipStream_t s, const DevLevel &L, int order, const float *x, const float *f, float *d);
+// The V-cycle's kernels, on FP32 (mixed form) or FP64 vectors (plain form on
+// levels whose matrix is its class stencils: lat_exact64 or lat_aff64)
+template <typename T>
+void kl_jacobi(hipStream_t s, const DevLevel &L, int order, const T *x, const T *f, T *out, T omega);
+template <typename T>
+void kl_jacobi_zero(hipStream_t s, const DevLevel &L, int order, const T *f, T *out, T omega);
+template <typename T>
+void kl_defect(hipStream_t s, const DevLevel &L, int order, const T *x, const T *f, T *d);
 // zero_sweep: also write the coarse level's first pre-smoothing sweep from a
 // zero start, omega D^-1 coarse (needs kl_zero_sweep_fusable(C))
-void kl_restrict(hipStream_t s, const DevLevel &F, const DevLevel &C, int order, const float *fine, float *coarse,
-                 float *zero_sweep = nullptr, float omega = 0.f);
+template <typename T>
+void kl_restrict(hipStream_t s, const DevLevel &F, const DevLevel &C, int order, const T *fine, T *coarse,
+                 T *zero_sweep, T omega);
 // every class of C has a uniform stencil (and no affine field)
 bool kl_zero_sweep_fusable(const DevLevel &C);
 // zt for the finest level F (x: its lt) when its classes allow it
 bool kl_top_zero_sweep(const DevLevel &F, int order, float omega, float *x, TopZeroSweep &zt);
+// the same for the FP64 V-cycle (needs lat_exact64)
+bool kl_top_zero_sweep(const DevLevel &F, int order, double omega, double *x, TopZeroSweep &zt);
+// zeros at the boundary nodes of count lattice vectors (v, v + ld, ...), and of four vectors
+void kl_clear_boundary(hipStream_t s, const DevLevel &L, double *v, int64_t ld, int count);
+void kl_clear_boundary4(hipStream_t s, const DevLevel &L, double *a, double *b, double *c, double *d);
 // y = A x on the lattice with FP32 x (converted exactly: the products of
 // kl_spmv64 on the FP64 copy of x); xcopy (optional) receives x at every
 // lattice node.  Only where kl_spmv64 takes its quad form
 // (kl_spmv64_f32_ok)
 bool kl_spmv64_f32_ok(const DevLevel &L, int order);
 void kl_spmv64_f32(hipStream_t s, const DevLevel &L, int order, const float *x, double *y, float *xcopy);
-void kl_prolong_update(hipStream_t s, const DevLevel &F, const DevLevel &C, int order, const float *coarse, float *x,
-                       float damp);
+template <typename T>
+void kl_prolong_update(hipStream_t s, const DevLevel &F, const DevLevel &C, int order, const T *coarse, T *x, T damp);
 // classes whose stencil is the same at every node (within 1e-12 of the
 // largest entry) get the compact form; synchronises the stream (flag_host:
 // pinned, 8 ints).  all_uniform false: kl_convert must fill lval / linv.
@@ -524,19 +538,22 @@ void kl_dof_to_lat64(hipStream_t s, const DevLevel &L, const double *v, double *
 void kl_lat64_to_dof(hipStream_t s, const DevLevel &L, const double *l, double *v);
 void kl_cast_d2f(hipStream_t s, int64_t n, const double *a, float *b);
 void kl_cast_f2d(hipStream_t s, int64_t n, const float *a, double *b);
-// DOF-ordered f64 <-> lattice f32 (Dirichlet DOFs map to zero)
-void kl_from_dof(hipStream_t s, const DevLevel &L, const double *v, float *l);
+// DOF-ordered f64 <-> lattice vectors (Dirichlet DOFs map to zero)
+template <typename T>
+void kl_from_dof(hipStream_t s, const DevLevel &L, const double *v, T *l);
 // zero-start mixed V-cycle of levels top..1 and the exact coarse solve in
 // one launch (levels[0..top]; 1 <= top <= 3)
 void kl_small_vcycle(hipStream_t s, const DevLevel *levels, int top, int order, int pre, int post, float omega,
                      float damp, const double *Ainv);
-void kl_to_dof(hipStream_t s, const DevLevel &L, const float *l, double *v);
+template <typename T>
+void kl_to_dof(hipStream_t s, const DevLevel &L, const T *l, double *v);
 // scratch: gj_scratch_doubles(na) doubles; inv: na^2 doubles
 void k_invert_active(hipStream_t s, const DevLevel &L, double *scratch, double *inv);
 int64_t gj_scratch_doubles(int na);
-// x_A = A_AA^-1 f_A on the FP32 lattice vectors of the coarsest level (zero
+// x_A = A_AA^-1 f_A on the lattice vectors of the coarsest level (zero
 // iterate, zero Dirichlet data)
-void k_coarse_from_lattice(hipStream_t s, const DevLevel &C, const double *Ainv, const float *lf, float *lx);
+template <typename T>
+void k_coarse_from_lattice(hipStream_t s, const DevLevel &C, const double *Ainv, const T *lf, T *lx);
 // the inversion takes more than one launch (larger than the one-workgroup LDS form)
 bool k_invert_multi_launch(int na);
 void k_multi_axpy(hipStream_t s, int n, int m, const double *coef, const double *Z, int64_t ldz, double *x);

@@ -502,31 +502,40 @@ __global__ __launch_bounds__(kBlock) void scale_copy_k(int n, const double *__re
 // the finest lattice level's zero-start sweep at lattice node e from the
 // FP32 value f just stored there (TopZeroSweep); d: the 8 class values of
 // t.d staged in LDS by top_zero_stage
-__device__ inline void top_zero_stage(const TopZeroSweep &t, float *d) {
-  if (t.x && threadIdx.x < 8) d[threadIdx.x] = threadIdx.x < (t.order == 2 ? 8u : 1u) ? t.d[threadIdx.x * t.dstride] : 0.f;
+__device__ inline void top_zero_stage(const TopZeroSweep &t, float *d, double *d64) {
+  if (threadIdx.x >= 8) return;
+  const bool used = threadIdx.x < (t.order == 2 ? 8u : 1u);
+  if (t.x) d[threadIdx.x] = used ? t.d[threadIdx.x * t.dstride] : 0.f;
+  if (t.x64) d64[threadIdx.x] = used ? t.d64[threadIdx.x * t.dstride] : 0.0;
 }
-__device__ inline void top_zero_sweep(const TopZeroSweep &t, const float *d, int64_t e, float f) {
+template <typename T>
+__device__ inline void top_zero_sweep(const TopZeroSweep &t, T *x, T omega, const T *d, int64_t e, T f) {
   // 32-bit unsigned division: a level has fewer than 2^31 lattice nodes
   const unsigned u = (unsigned)e, nn = (unsigned)t.nn, q = u / nn, Z = q / nn;
   const unsigned X = u - q * nn, Y = q - Z * nn;
   if (X - 1u < nn - 2u && Y - 1u < nn - 2u && Z - 1u < nn - 2u) {
     const int c = t.order == 2 ? (int)((X & 1u) + 2u * (Y & 1u) + 4u * (Z & 1u)) : 0;
-    t.x[e] = t.omega * f * d[c];
+    x[e] = omega * f * d[c];
   }
+}
+// the sweeps that t asks for at node e, from the Krylov vector's entry v
+__device__ inline void top_zero_sweeps(const TopZeroSweep &t, const float *d, const double *d64, int64_t e, double v) {
+  if (t.x) top_zero_sweep<float>(t, t.x, t.omega, d, e, (float)v);
+  if (t.x64) top_zero_sweep<double>(t, t.x64, t.omega64, d64, e, v);
 }
 
 __global__ __launch_bounds__(kBlock) void scale_copy2_k(int n, const double *__restrict__ partials,
                                                         double *__restrict__ norm_out, const double *__restrict__ x,
                                                         double *__restrict__ y, float *__restrict__ y32,
                                                         TopZeroSweep zt) {
-  __shared__ double sh[17];
+  __shared__ double sh[17], zd64[8];
   __shared__ float zd[8];
   const int n2 = n >> 1, gs = gridDim.x * kBlock;
   const double2 *x2 = (const double2 *)x;
   double2 *y2 = (double2 *)y;
   int i = blockIdx.x * kBlock + threadIdx.x;
   const double2 v0 = i < n2 ? x2[i] : double2{0, 0};  // issued before the reduction
-  top_zero_stage(zt, zd);                              // visible after its barriers
+  top_zero_stage(zt, zd, zd64);                        // visible after its barriers
   const double nrm = sqrt(sum_partials(partials, sh));
   if (blockIdx.x == 0 && threadIdx.x == 0) *norm_out = nrm;
   const double s = nrm != 0.0 ? 1.0 / nrm : 1.0;
@@ -534,35 +543,23 @@ __global__ __launch_bounds__(kBlock) void scale_copy2_k(int n, const double *__r
   if (i < n2) {
     const double2 r = {v0.x * s, v0.y * s};
     y2[i] = r;
-    if (y32) {
-      const f2 r32 = f2{(float)r.x, (float)r.y};
-      ((f2 *)y32)[i] = r32;
-      if (zt.x) {
-        top_zero_sweep(zt, zd, 2 * (int64_t)i, r32.x);
-        top_zero_sweep(zt, zd, 2 * (int64_t)i + 1, r32.y);
-      }
-    }
+    if (y32) ((f2 *)y32)[i] = f2{(float)r.x, (float)r.y};
+    top_zero_sweeps(zt, zd, zd64, 2 * (int64_t)i, r.x);
+    top_zero_sweeps(zt, zd, zd64, 2 * (int64_t)i + 1, r.y);
   }
   for (i += gs; i < n2; i += gs) {
     const double2 v = x2[i];
     const double2 r = {v.x * s, v.y * s};
     y2[i] = r;
-    if (y32) {
-      const f2 r32 = f2{(float)r.x, (float)r.y};
-      ((f2 *)y32)[i] = r32;
-      if (zt.x) {
-        top_zero_sweep(zt, zd, 2 * (int64_t)i, r32.x);
-        top_zero_sweep(zt, zd, 2 * (int64_t)i + 1, r32.y);
-      }
-    }
+    if (y32) ((f2 *)y32)[i] = f2{(float)r.x, (float)r.y};
+    top_zero_sweeps(zt, zd, zd64, 2 * (int64_t)i, r.x);
+    top_zero_sweeps(zt, zd, zd64, 2 * (int64_t)i + 1, r.y);
   }
   if ((n & 1) && blockIdx.x == 0 && threadIdx.x == 0) {
-    y[n - 1] = x[n - 1] * s;
-    if (y32) {
-      const float v32 = (float)(x[n - 1] * s);
-      y32[n - 1] = v32;
-      if (zt.x) top_zero_sweep(zt, zd, n - 1, v32);
-    }
+    const double v = x[n - 1] * s;
+    y[n - 1] = v;
+    if (y32) y32[n - 1] = (float)v;
+    top_zero_sweeps(zt, zd, zd64, n - 1, v);
   }
 }
 
@@ -730,16 +727,14 @@ __global__ __launch_bounds__(kBlock) void ls_update2_k(int n, int i, const doubl
 // x *= alpha and, when y32 is given, y32 = (float) x (scalar loop)
 __global__ void scale_cast_k(int n, double alpha, double *__restrict__ x, float *__restrict__ y32, TopZeroSweep zt) {
   __shared__ float zd[8];
-  top_zero_stage(zt, zd);
+  __shared__ double zd64[8];
+  top_zero_stage(zt, zd, zd64);
   __syncthreads();
   for (int i = blockIdx.x * kBlock + threadIdx.x; i < n; i += gridDim.x * kBlock) {
     const double v = x[i] * alpha;
     x[i] = v;
-    if (y32) {
-      const float v32 = (float)v;
-      y32[i] = v32;
-      if (zt.x) top_zero_sweep(zt, zd, i, v32);
-    }
+    if (y32) y32[i] = (float)v;
+    top_zero_sweeps(zt, zd, zd64, i, v);
   }
 }
 
@@ -819,21 +814,22 @@ __global__ __launch_bounds__(kBlock) void coarse_update_k(int na, const double *
   if (lane == 0) x[row] += s;
 }
 
-// Mixed-form exact coarse solve from a zero iterate with zero Dirichlet data
-// (the V-cycle's visit of the coarsest level): x_A = A_AA^-1 f_A, read from
-// and written to the FP32 lattice vectors.  The defect f - A x of a zero
+// Exact coarse solve of the lattice V-cycles from a zero iterate with zero
+// Dirichlet data (the V-cycle's visit of the coarsest level): x_A = A_AA^-1
+// f_A, read from and written to the lattice vectors.  The defect f - A x of a zero
 // iterate is f itself, so these are the products and the summation order of
 // lat_to_dof_k, csr_stream<kDefect> and coarse_update_k into a zeroed x and
 // dof_to_lat_k, in one launch instead of six.
+template <typename T>
 __global__ __launch_bounds__(kBlock) void coarse_lat_k(int na, const double *__restrict__ Ainv,
-                                                       const int *__restrict__ dof2node, const float *__restrict__ lf,
-                                                       float *__restrict__ lx) {
+                                                       const int *__restrict__ dof2node, const T *__restrict__ lf,
+                                                       T *__restrict__ lx) {
   const int row = (blockIdx.x * kBlock + threadIdx.x) >> 6, lane = threadIdx.x & 63;
   if (row >= na) return;
   double s = 0;
   for (int j = lane; j < na; j += 64) s += Ainv[(int64_t)row * na + j] * (double)lf[dof2node[j]];
   s = group_sum<64>(s);
-  if (lane == 0) lx[dof2node[row]] = (float)(0.0 + s);
+  if (lane == 0) lx[dof2node[row]] = (T)(0.0 + s);
 }
 
 // Coarse-level smoothing loop of TMultiGrid3D::Smooth(CoarseSmooth)
@@ -1822,12 +1818,12 @@ void k_axpy_dot(hipStream_t s, int n, const double *alpha_partials, double sign,
 }
 void k_scale_copy(hipStream_t s, int n, const double *partials, double *norm_out, const double *x, double *y,
                   float *y32, const TopZeroSweep *zt) {
-  const TopZeroSweep z = zt && y32 ? *zt : TopZeroSweep{};
+  const TopZeroSweep z = zt ? *zt : TopZeroSweep{};
   if (al16(x) && al16(y) && ((uintptr_t)y32 & 7) == 0) {
     scale_copy2_k<<<kRedBlocks, kBlock, 0, s>>>(n, partials, norm_out, x, y, y32, z);
   } else {
     scale_copy_k<<<kRedBlocks, kBlock, 0, s>>>(n, partials, norm_out, x, y);
-    if (y32) scale_cast_k<<<grid_for(n), kBlock, 0, s>>>(n, 1.0, y, y32, z);
+    if (y32 || z.x64) scale_cast_k<<<grid_for(n), kBlock, 0, s>>>(n, 1.0, y, y32, z);
   }
 }
 int k_ls_blocks(int n) { return (n + kLsChunk - 1) / kLsChunk; }
@@ -1840,7 +1836,7 @@ void k_ls_step(hipStream_t s, int n, int i, const double *V, int64_t ld, double 
   ls_update2_k<<<kRedBlocks, kBlock, 0, s>>>(n, i, h, V, ld, w, partials);
 }
 void k_scale_cast(hipStream_t s, int n, double alpha, double *x, float *y32, const TopZeroSweep *zt) {
-  scale_cast_k<<<grid_for(n), kBlock, 0, s>>>(n, alpha, x, y32, zt && y32 ? *zt : TopZeroSweep{});
+  scale_cast_k<<<grid_for(n), kBlock, 0, s>>>(n, alpha, x, y32, zt ? *zt : TopZeroSweep{});
 }
 void k_scale(hipStream_t s, int n, double alpha, double *x) { scale_k<<<grid_for(n), kBlock, 0, s>>>(n, alpha, x); }
 void k_axpy(hipStream_t s, int n, double alpha, const double *x, double *y) {
@@ -1854,10 +1850,13 @@ void k_fill(hipStream_t s, int64_t n, double v, double *y) { fill_k<<<grid_for(n
 void k_matadd(hipStream_t s, int64_t n, double *C, const double *D, double alpha) {
   matadd_k<<<grid_for(n), kBlock, 0, s>>>(n, C, D, alpha);
 }
-void k_coarse_from_lattice(hipStream_t s, const DevLevel &C, const double *Ainv, const float *lf, float *lx) {
+template <typename T>
+void k_coarse_from_lattice(hipStream_t s, const DevLevel &C, const double *Ainv, const T *lf, T *lx) {
   if (C.nact > 0)
-    coarse_lat_k<<<(C.nact * 64 + kBlock - 1) / kBlock, kBlock, 0, s>>>(C.nact, Ainv, C.ldof2node, lf, lx);
+    coarse_lat_k<T><<<(C.nact * 64 + kBlock - 1) / kBlock, kBlock, 0, s>>>(C.nact, Ainv, C.ldof2node, lf, lx);
 }
+template void k_coarse_from_lattice<float>(hipStream_t, const DevLevel &, const double *, const float *, float *);
+template void k_coarse_from_lattice<double>(hipStream_t, const DevLevel &, const double *, const double *, double *);
 void k_gemv_dense(hipStream_t s, int n, const double *A, const double *x, double *y) {
   if (n > 0) coarse_update_k<<<(n * 64 + kBlock - 1) / kBlock, kBlock, 0, s>>>(n, A, x, y);
 }

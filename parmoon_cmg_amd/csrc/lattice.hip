@@ -1,5 +1,6 @@
-// Lattice-stencil kernels of the mixed-precision V-cycle (FP32 values, FP32
-// accumulation).
+// Lattice-stencil kernels of the V-cycle: FP32 values and accumulation in the
+// mixed-precision form, FP64 in the plain form on levels whose matrix is
+// exactly its class stencils.
 //
 // A level's unknowns are stored in node-lattice order (X fastest), boundary
 // nodes included and kept at zero: inside the preconditioner the Dirichlet
@@ -68,24 +69,25 @@ __host__ __device__ inline constexpr int lo_off() { return (P == 1 || PXS == 0) 
 template <int P, int PXS>
 __host__ __device__ inline constexpr int hi_off() { return (P == 1 || PXS == 0) ? P : 1; }
 
-// Compact class stencil: kCst floats per class, entry kCst - 1 is 1 / a_ii.
+// Compact class stencil: kCst values per class, entry kCst - 1 is 1 / a_ii.
 constexpr int kCst = 128;
 
-// The FP64 value of the lattice system matrix alpha (S0 + X SX + Y SY) +
-// alpha_m M at entry s of a node of coordinates (X, Y), with the rounding
-// spelled out (explicit fma), so that the per-node fill and the sweeps that
-// evaluate it on the fly produce the same bits.  s0, sx, sy, sm: the class's
-// S0, SX, SY and mass stencils.
-__host__ __device__ inline double affine_value(const double *s0, const double *sx, const double *sy,
-                                               const double *sm, double alpha, double alpha_m, int s, int X,
-                                               int Y) {
-  const double e = fma((double)Y, sy[s], fma((double)X, sx[s], s0[s]));
-  return alpha_m != 0.0 ? fma(alpha_m, sm[s], alpha * e) : alpha * e;
-}
+// The node functions below take the value type T of a V-cycle (FP32 in the
+// mixed form, FP64 in the plain form) as their last template parameter; their
+// arguments do not deduce it
+template <typename T>
+struct ScalarOf {
+  typedef T type;
+};
+template <typename T>
+using Sc = typename ScalarOf<T>::type;
 
-// The same entry for the FP32 preconditioner: the stencils rounded to FP32
-// and the expression evaluated with FP32 fma (the FP64 operator keeps
-// affine_value and matches the CSR values)
+// Entry s of the lattice system matrix alpha (S0 + X SX + Y SY) + alpha_m M at
+// a node of coordinates (X, Y), with the rounding spelled out (explicit fma),
+// so that the per-node fill and the sweeps that evaluate it on the fly produce
+// the same bits; s0, sx, sy, sm: the class's S0, SX, SY and mass stencils.
+// FP32 preconditioner: the stencils rounded to FP32 and the expression
+// evaluated with FP32 fma
 __host__ __device__ inline float affine_value32(const float *s0, const float *sx, const float *sy, const float *sm,
                                                 float alpha, float alpha_m, int s, int X, int Y) {
   const float e = fmaf((float)Y, sy[s], fmaf((float)X, sx[s], s0[s]));
@@ -94,22 +96,22 @@ __host__ __device__ inline float affine_value32(const float *s0, const float *sx
 
 // UNI: the class's stencil (and diagonal) are the same at every node and are
 // read from cst (uniform across the block); otherwise per-node values.
-template <int P, int PX, int PY, int PZ, int MODE, bool UNI>
-__host__ __device__ inline void lat_node(const LatArgs &a, const LatDev &C, long long k, const float *__restrict__ val,
-                                         const float *__restrict__ inv, const float *__restrict__ cst,
-                                         const float *__restrict__ x, const float *__restrict__ f,
-                                         float *__restrict__ out, float omega) {
+template <int P, int PX, int PY, int PZ, int MODE, bool UNI, typename T = float>
+__host__ __device__ inline void lat_node(const LatArgs &a, const LatDev &C, long long k,
+                                         const Sc<T> *__restrict__ val, const Sc<T> *__restrict__ inv,
+                                         const Sc<T> *__restrict__ cst, const Sc<T> *__restrict__ x,
+                                         const Sc<T> *__restrict__ f, Sc<T> *__restrict__ out, Sc<T> omega) {
   int kx, ky, kz;
   class_coords(C, k, kx, ky, kz);
   const int X = C.lo[0] + C.step * kx, Y = C.lo[1] + C.step * ky, Z = C.lo[2] + C.step * kz;
   const long long nn = a.nn, node = X + nn * (Y + nn * Z);
-  const float di = UNI ? cst[kCst - 1] : (MODE == kLDefect ? 0.f : inv[C.first + k]);
+  const T di = UNI ? cst[kCst - 1] : (MODE == kLDefect ? T(0) : inv[C.first + k]);
   if (MODE == kLJacobiZero) {
     out[node] = omega * f[node] * di;
     return;
   }
-  const float *__restrict__ v = val + C.off + k;
-  float s = 0.f;
+  const T *__restrict__ v = val + C.off + k;
+  T s = 0;
   int si = 0;
 #pragma unroll
   for (int dz = lo_off<P, PZ>(); dz <= hi_off<P, PZ>(); dz++)
@@ -123,33 +125,33 @@ __host__ __device__ inline void lat_node(const LatArgs &a, const LatDev &C, long
 }
 
 // node k of class c (the class fixes the parities, hence the stencil shape)
-template <int P, int PX, int PY, int PZ, int MODE>
-__host__ __device__ inline void lat_node_any(const LatArgs &a, int c, long long k, const float *__restrict__ val,
-                                             const float *__restrict__ inv, const float *__restrict__ cst,
-                                             const float *__restrict__ x, const float *__restrict__ f,
-                                             float *__restrict__ out, float omega) {
-  if (a.uni[c]) lat_node<P, PX, PY, PZ, MODE, true>(a, a.c[c], k, val, inv, cst + c * kCst, x, f, out, omega);
-  else lat_node<P, PX, PY, PZ, MODE, false>(a, a.c[c], k, val, inv, cst, x, f, out, omega);
+template <int P, int PX, int PY, int PZ, int MODE, typename T = float>
+__host__ __device__ inline void lat_node_any(const LatArgs &a, int c, long long k, const Sc<T> *__restrict__ val,
+                                             const Sc<T> *__restrict__ inv, const Sc<T> *__restrict__ cst,
+                                             const Sc<T> *__restrict__ x, const Sc<T> *__restrict__ f,
+                                             Sc<T> *__restrict__ out, Sc<T> omega) {
+  if (a.uni[c]) lat_node<P, PX, PY, PZ, MODE, true, T>(a, a.c[c], k, val, inv, cst + c * kCst, x, f, out, omega);
+  else lat_node<P, PX, PY, PZ, MODE, false, T>(a, a.c[c], k, val, inv, cst, x, f, out, omega);
 }
 
 // node k of class c (the class fixes the parities, hence the stencil shape)
-template <int P, int MODE>
-__host__ __device__ inline void lat_class_node(const LatArgs &a, int c, long long k, const float *__restrict__ val,
-                                               const float *__restrict__ inv, const float *__restrict__ cst,
-                                               const float *__restrict__ x, const float *__restrict__ f,
-                                               float *__restrict__ out, float omega) {
+template <int P, int MODE, typename T = float>
+__host__ __device__ inline void lat_class_node(const LatArgs &a, int c, long long k, const Sc<T> *__restrict__ val,
+                                               const Sc<T> *__restrict__ inv, const Sc<T> *__restrict__ cst,
+                                               const Sc<T> *__restrict__ x, const Sc<T> *__restrict__ f,
+                                               Sc<T> *__restrict__ out, Sc<T> omega) {
   if (P == 1) {
-    lat_node_any<1, 0, 0, 0, MODE>(a, c, k, val, inv, cst, x, f, out, omega);
+    lat_node_any<1, 0, 0, 0, MODE, T>(a, c, k, val, inv, cst, x, f, out, omega);
   } else {
     switch (c) {
-      case 0: lat_node_any<2, 0, 0, 0, MODE>(a, c, k, val, inv, cst, x, f, out, omega); break;
-      case 1: lat_node_any<2, 1, 0, 0, MODE>(a, c, k, val, inv, cst, x, f, out, omega); break;
-      case 2: lat_node_any<2, 0, 1, 0, MODE>(a, c, k, val, inv, cst, x, f, out, omega); break;
-      case 3: lat_node_any<2, 1, 1, 0, MODE>(a, c, k, val, inv, cst, x, f, out, omega); break;
-      case 4: lat_node_any<2, 0, 0, 1, MODE>(a, c, k, val, inv, cst, x, f, out, omega); break;
-      case 5: lat_node_any<2, 1, 0, 1, MODE>(a, c, k, val, inv, cst, x, f, out, omega); break;
-      case 6: lat_node_any<2, 0, 1, 1, MODE>(a, c, k, val, inv, cst, x, f, out, omega); break;
-      default: lat_node_any<2, 1, 1, 1, MODE>(a, c, k, val, inv, cst, x, f, out, omega); break;
+      case 0: lat_node_any<2, 0, 0, 0, MODE, T>(a, c, k, val, inv, cst, x, f, out, omega); break;
+      case 1: lat_node_any<2, 1, 0, 0, MODE, T>(a, c, k, val, inv, cst, x, f, out, omega); break;
+      case 2: lat_node_any<2, 0, 1, 0, MODE, T>(a, c, k, val, inv, cst, x, f, out, omega); break;
+      case 3: lat_node_any<2, 1, 1, 0, MODE, T>(a, c, k, val, inv, cst, x, f, out, omega); break;
+      case 4: lat_node_any<2, 0, 0, 1, MODE, T>(a, c, k, val, inv, cst, x, f, out, omega); break;
+      case 5: lat_node_any<2, 1, 0, 1, MODE, T>(a, c, k, val, inv, cst, x, f, out, omega); break;
+      case 6: lat_node_any<2, 0, 1, 1, MODE, T>(a, c, k, val, inv, cst, x, f, out, omega); break;
+      default: lat_node_any<2, 1, 1, 1, MODE, T>(a, c, k, val, inv, cst, x, f, out, omega); break;
     }
   }
 }
@@ -166,21 +168,33 @@ struct LatAff {
   int centre[8];      // stencil index of the offset (0, 0, 0) per class
 };
 
-template <int P, int PX, int PY, int PZ, int MODE>
-__host__ __device__ inline void lat_node_aff(const LatArgs &a, const LatDev &C, long long k, const float *s0,
-                                             const float *sx, const float *sy, const float *sm, float alpha,
-                                             float alpha_m, int centre, const float *__restrict__ x,
-                                             const float *__restrict__ f, float *__restrict__ out, float omega) {
+// FP64: the arithmetic of the CSR values (affine_entry, matadd_into_k; the
+// FP64 lattice forms are used for alpha_m 0 or 1 only)
+__host__ __device__ inline float affine_at(const float *s0, const float *sx, const float *sy, const float *sm,
+                                           float alpha, float alpha_m, int s, int X, int Y) {
+  return affine_value32(s0, sx, sy, sm, alpha, alpha_m, s, X, Y);
+}
+__host__ __device__ inline double affine_at(const double *s0, const double *sx, const double *sy, const double *sm,
+                                            double alpha, double alpha_m, int s, int X, int Y) {
+  const double e = fma((double)Y, sy[s], fma((double)X, sx[s], s0[s]));
+  return alpha_m != 0.0 ? fma(alpha, e, sm[s]) : alpha * e;
+}
+
+template <int P, int PX, int PY, int PZ, int MODE, typename T = float>
+__host__ __device__ inline void lat_node_aff(const LatArgs &a, const LatDev &C, long long k, const Sc<T> *s0,
+                                             const Sc<T> *sx, const Sc<T> *sy, const Sc<T> *sm, Sc<T> alpha,
+                                             Sc<T> alpha_m, int centre, const Sc<T> *__restrict__ x,
+                                             const Sc<T> *__restrict__ f, Sc<T> *__restrict__ out, Sc<T> omega) {
   int kx, ky, kz;
   class_coords(C, k, kx, ky, kz);
   const int X = C.lo[0] + C.step * kx, Y = C.lo[1] + C.step * ky, Z = C.lo[2] + C.step * kz;
   const long long nn = a.nn, node = X + nn * (Y + nn * Z);
-  const float di = MODE == kLDefect ? 0.f : 1.0f / affine_value32(s0, sx, sy, sm, alpha, alpha_m, centre, X, Y);
+  const T di = MODE == kLDefect ? T(0) : T(1) / affine_at(s0, sx, sy, sm, alpha, alpha_m, centre, X, Y);
   if (MODE == kLJacobiZero) {
     out[node] = omega * f[node] * di;
     return;
   }
-  float s = 0.f;
+  T s = 0;
   int si = 0;
 #pragma unroll
   for (int dz = lo_off<P, PZ>(); dz <= hi_off<P, PZ>(); dz++)
@@ -188,18 +202,18 @@ __host__ __device__ inline void lat_node_aff(const LatArgs &a, const LatDev &C, 
     for (int dy = lo_off<P, PY>(); dy <= hi_off<P, PY>(); dy++)
 #pragma unroll
       for (int dx = lo_off<P, PX>(); dx <= hi_off<P, PX>(); dx++, si++)
-        s += affine_value32(s0, sx, sy, sm, alpha, alpha_m, si, X, Y) * x[node + dx + nn * (dy + nn * dz)];
+        s += affine_at(s0, sx, sy, sm, alpha, alpha_m, si, X, Y) * x[node + dx + nn * (dy + nn * dz)];
   if (MODE == kLDefect) out[node] = f[node] - s;
   else out[node] = x[node] + omega * (f[node] - s) * di;
 }
 
-template <int P, int MODE>
-__host__ __device__ inline void lat_class_node_aff(const LatArgs &a, int c, long long k, const float *s0,
-                                                   const float *sx, const float *sy, const float *sm,
-                                                   float alpha, float alpha_m, int centre, const float *x,
-                                                   const float *f, float *out, float omega) {
+template <int P, int MODE, typename T = float>
+__host__ __device__ inline void lat_class_node_aff(const LatArgs &a, int c, long long k, const Sc<T> *s0,
+                                                   const Sc<T> *sx, const Sc<T> *sy, const Sc<T> *sm, Sc<T> alpha,
+                                                   Sc<T> alpha_m, int centre, const Sc<T> *x, const Sc<T> *f,
+                                                   Sc<T> *out, Sc<T> omega) {
 #define CD3D_AFF(PX, PY, PZ) \
-  lat_node_aff<P, PX, PY, PZ, MODE>(a, a.c[c], k, s0, sx, sy, sm, alpha, alpha_m, centre, x, f, out, omega)
+  lat_node_aff<P, PX, PY, PZ, MODE, T>(a, a.c[c], k, s0, sx, sy, sm, alpha, alpha_m, centre, x, f, out, omega)
   if (P == 1) {
     CD3D_AFF(0, 0, 0);
   } else {
@@ -217,23 +231,22 @@ __host__ __device__ inline void lat_class_node_aff(const LatArgs &a, int c, long
 #undef CD3D_AFF
 }
 
-template <int P, int MODE>
-__global__ __launch_bounds__(kB) void lat_aff_sweep_k(LatArgs a, LatAff af, const float *__restrict__ x,
-                                                      const float *__restrict__ f, float *__restrict__ out,
-                                                      float omega) {
-  __shared__ float st[4][kCst];  // S0, SX, SY, mass of the block's class, rounded to FP32
+template <int P, int MODE, typename T>
+__global__ __launch_bounds__(kB) void lat_aff_sweep_k(LatArgs a, LatAff af, const T *__restrict__ x,
+                                                      const T *__restrict__ f, T *__restrict__ out, T omega) {
+  __shared__ T st[4][kCst];  // S0, SX, SY, mass of the block's class (FP32 sweeps: rounded)
   const int c = block_class(a.bstart, a.nclass, (int)blockIdx.x);
   for (int i = threadIdx.x; i < kCst; i += kB) {
-    st[0][i] = (float)af.st[c * kCst + i];
-    st[1][i] = (float)af.st[8 * kCst + 8 + c * kCst + i];
-    st[2][i] = (float)af.st[2 * 8 * kCst + 8 + c * kCst + i];
-    st[3][i] = af.stm ? (float)af.stm[c * kCst + i] : 0.f;
+    st[0][i] = (T)af.st[c * kCst + i];
+    st[1][i] = (T)af.st[8 * kCst + 8 + c * kCst + i];
+    st[2][i] = (T)af.st[2 * 8 * kCst + 8 + c * kCst + i];
+    st[3][i] = af.stm ? (T)af.stm[c * kCst + i] : T(0);
   }
   __syncthreads();
   const long long k = (long long)(blockIdx.x - a.bstart[c]) * kB + threadIdx.x;
   if (k < a.c[c].nodes)
-    lat_class_node_aff<P, MODE>(a, c, k, st[0], st[1], st[2], st[3], (float)af.alpha, (float)af.alpha_m,
-                                af.centre[c], x, f, out, omega);
+    lat_class_node_aff<P, MODE, T>(a, c, k, st[0], st[1], st[2], st[3], (T)af.alpha, (T)af.alpha_m, af.centre[c], x,
+                                   f, out, omega);
 }
 
 // Q2 sweeps by vertex/midpoint pairs along X.  A thread takes the nodes
@@ -281,17 +294,17 @@ __host__ __device__ inline PairPos pair_pos(const LatArgs &a, long long k) {
 
 // the stencil sums s0 (vertex) and s1 (midpoint) of a pair and the pair's
 // own x values; UNI: compact stencils cs0, cs1, else per-node values val
-// ([class][entry][node], FP32)
+// ([class][entry][node])
 template <typename T, int PY, int PZ, bool UNI>
 __host__ __device__ inline void pair_sums(const LatArgs &a, const PairPos &q, long long k,
-                                          const float *__restrict__ val, const T *cs0, const T *cs1,
+                                          const T *__restrict__ val, const T *cs0, const T *cs1,
                                           const T *__restrict__ x, T &s0, T &s1, T &xv, T &xm) {
   typedef typename Vec2<T>::type V2;
   constexpr int c0 = 2 * PY + 4 * PZ, c1 = c0 + 1;
   const LatDev &V = a.c[c0], &M = a.c[c1];
   const long long nn = a.nn;
-  const float *__restrict__ v0 = UNI ? nullptr : val + V.off + (q.hv ? q.kv : 0);
-  const float *__restrict__ v1 = UNI ? nullptr : val + M.off + k;
+  const T *__restrict__ v0 = UNI ? nullptr : val + V.off + (q.hv ? q.kv : 0);
+  const T *__restrict__ v1 = UNI ? nullptr : val + M.off + k;
   // a boundary vertex (ix = 0) has no sum: its left segment is read from the
   // centre instead (in bounds, unused), so the loads need no branch
   const int lft_off = q.hv ? -2 : 0;
@@ -316,40 +329,41 @@ __host__ __device__ inline void pair_sums(const LatArgs &a, const PairPos &q, lo
       const T w[5] = {lft.x, lft.y, ctr.x, ctr.y, rgt};
 #pragma unroll
       for (int j = 0; j < 5; j++)
-        s0 += (UNI ? cs0[li * 5 + j] : T(v0[(long long)(li * 5 + j) * V.nodes])) * w[j];
+        s0 += (UNI ? cs0[li * 5 + j] : v0[(long long)(li * 5 + j) * V.nodes]) * w[j];
 #pragma unroll
       for (int j = 0; j < 3; j++)
-        s1 += (UNI ? cs1[li * 3 + j] : T(v1[(long long)(li * 3 + j) * M.nodes])) * w[j + 2];
+        s1 += (UNI ? cs1[li * 3 + j] : v1[(long long)(li * 3 + j) * M.nodes]) * w[j + 2];
     }
   }
 }
 
-// FP32 sweep of pair k (modes of lat_node); cs0, cs1: the compact stencils of
+// sweep of pair k (modes of lat_node); cs0, cs1: the compact stencils of
 // the two classes (UNI)
-template <int PY, int PZ, int MODE, bool UNI>
-__host__ __device__ inline void lat_pair(const LatArgs &a, long long k, const float *__restrict__ val,
-                                         const float *__restrict__ inv, const float *cs0, const float *cs1,
-                                         const float *__restrict__ x, const float *__restrict__ f,
-                                         float *__restrict__ out, float omega) {
+template <int PY, int PZ, int MODE, bool UNI, typename T>
+__host__ __device__ inline void lat_pair(const LatArgs &a, long long k, const T *__restrict__ val,
+                                         const T *__restrict__ inv, const T *cs0, const T *cs1,
+                                         const T *__restrict__ x, const T *__restrict__ f, T *__restrict__ out,
+                                         T omega) {
+  typedef typename Vec2<T>::type V2;
   const PairPos q = pair_pos<PY, PZ>(a, k);
   const long long nv = q.nv;
   const bool hv = q.hv;
-  const f2u fp = *(const f2u *)(f + nv);
-  float d0 = 0.f, d1 = 0.f;
+  const V2 fp = *(const V2 *)(f + nv);
+  T d0 = 0, d1 = 0;
   if (UNI) {
     d0 = cs0[kCst - 1];
     d1 = cs1[kCst - 1];
   } else if (MODE != kLDefect) {
-    d0 = hv ? inv[a.c[2 * PY + 4 * PZ].first + q.kv] : 0.f;
+    d0 = hv ? inv[a.c[2 * PY + 4 * PZ].first + q.kv] : T(0);
     d1 = inv[a.c[2 * PY + 4 * PZ + 1].first + k];
   }
-  float r0, r1;
+  T r0, r1;
   if (MODE == kLJacobiZero) {
     r0 = omega * fp.x * d0;
     r1 = omega * fp.y * d1;
   } else {
-    float s0, s1, xv, xm;
-    pair_sums<float, PY, PZ, UNI>(a, q, k, val, cs0, cs1, x, s0, s1, xv, xm);
+    T s0, s1, xv, xm;
+    pair_sums<T, PY, PZ, UNI>(a, q, k, val, cs0, cs1, x, s0, s1, xv, xm);
     if (MODE == kLDefect) {
       r0 = fp.x - s0;
       r1 = fp.y - s1;
@@ -358,35 +372,34 @@ __host__ __device__ inline void lat_pair(const LatArgs &a, long long k, const fl
       r1 = xm + omega * (fp.y - s1) * d1;
     }
   }
-  // vertex and midpoint are adjacent: one 8-byte store unless the vertex is
+  // vertex and midpoint are adjacent: one paired store unless the vertex is
   // a boundary node (not written)
-  if (hv) *(f2u *)(out + nv) = f2u{r0, r1};
+  if (hv) *(V2 *)(out + nv) = V2{r0, r1};
   else out[nv + 1] = r1;
 }
 
 // pair k of pair class pc = py + 2 pz; UNI: every class has compact values
 // (cs0, cs1 those of the pair class), else every class has per-node values
-template <int MODE, bool UNI>
-__host__ __device__ inline void lat_pair_node(const LatArgs &a, int pc, long long k, const float *__restrict__ val,
-                                              const float *__restrict__ inv, const float *cs0, const float *cs1,
-                                              const float *__restrict__ x, const float *__restrict__ f,
-                                              float *__restrict__ out, float omega) {
+template <int MODE, bool UNI, typename T = float>
+__host__ __device__ inline void lat_pair_node(const LatArgs &a, int pc, long long k, const Sc<T> *__restrict__ val,
+                                              const Sc<T> *__restrict__ inv, const Sc<T> *cs0, const Sc<T> *cs1,
+                                              const Sc<T> *__restrict__ x, const Sc<T> *__restrict__ f,
+                                              Sc<T> *__restrict__ out, Sc<T> omega) {
   switch (pc) {
-    case 0: lat_pair<0, 0, MODE, UNI>(a, k, val, inv, cs0, cs1, x, f, out, omega); break;
-    case 1: lat_pair<1, 0, MODE, UNI>(a, k, val, inv, cs0, cs1, x, f, out, omega); break;
-    case 2: lat_pair<0, 1, MODE, UNI>(a, k, val, inv, cs0, cs1, x, f, out, omega); break;
-    default: lat_pair<1, 1, MODE, UNI>(a, k, val, inv, cs0, cs1, x, f, out, omega); break;
+    case 0: lat_pair<0, 0, MODE, UNI, T>(a, k, val, inv, cs0, cs1, x, f, out, omega); break;
+    case 1: lat_pair<1, 0, MODE, UNI, T>(a, k, val, inv, cs0, cs1, x, f, out, omega); break;
+    case 2: lat_pair<0, 1, MODE, UNI, T>(a, k, val, inv, cs0, cs1, x, f, out, omega); break;
+    default: lat_pair<1, 1, MODE, UNI, T>(a, k, val, inv, cs0, cs1, x, f, out, omega); break;
   }
 }
 
 // UNI: the pair class's two compact stencils are staged in LDS (200 values
 // do not fit the scalar registers)
-template <int MODE, bool UNI>
-__global__ __launch_bounds__(kB) void lat_pair_k(LatArgs a, const float *__restrict__ val,
-                                                 const float *__restrict__ inv, const float *__restrict__ cst,
-                                                 const float *__restrict__ x, const float *__restrict__ f,
-                                                 float *__restrict__ out, float omega) {
-  __shared__ float cs[2 * kCst];
+template <int MODE, bool UNI, typename T>
+__global__ __launch_bounds__(kB) void lat_pair_k(LatArgs a, const T *__restrict__ val, const T *__restrict__ inv,
+                                                 const T *__restrict__ cst, const T *__restrict__ x,
+                                                 const T *__restrict__ f, T *__restrict__ out, T omega) {
+  __shared__ T cs[2 * kCst];
   // blocks in pair-class order: a CU sweeps one class's code path at a time
   // (measured: interleaving the four classes per tile, also per XCD, saves
   // HBM traffic but is slower)
@@ -399,7 +412,7 @@ __global__ __launch_bounds__(kB) void lat_pair_k(LatArgs a, const float *__restr
     __syncthreads();
   }
   const long long k = (long long)tile * kB + threadIdx.x;
-  if (k < a.c[2 * pc + 1].nodes) lat_pair_node<MODE, UNI>(a, pc, k, val, inv, cs, cs + kCst, x, f, out, omega);
+  if (k < a.c[2 * pc + 1].nodes) lat_pair_node<MODE, UNI, T>(a, pc, k, val, inv, cs, cs + kCst, x, f, out, omega);
 }
 
 // 16-byte vector at a 4-byte aligned address
@@ -648,38 +661,41 @@ __host__ __device__ inline void quad_sums(const LatArgs &a, const QuadPos &p, co
   }
 }
 
-// quad k of the FP32 sweep: G vertex/midpoint pairs on each of the 4 lines
+// quad k of the sweep: G vertex/midpoint pairs on each of the 4 lines
 // (Y0 + oy, Z0 + oz) (cs: the 8 classes' compact stencils)
-template <int G, int MODE>
+template <int G, int MODE, typename T = float>
 __host__ __device__ __attribute__((always_inline)) inline void lat_quad_node(const LatArgs &a, long long k,
-                                                                             const float *cs,
-                                              const float *__restrict__ x, const float *__restrict__ f,
-                                              float *__restrict__ out, float omega) {
+                                                                             const Sc<T> *cs,
+                                              const Sc<T> *__restrict__ x, const Sc<T> *__restrict__ f,
+                                              Sc<T> *__restrict__ out, Sc<T> omega) {
+  typedef typename Vec2<T>::type V2;
+  typedef typename Vec16<T>::type V16;
+  constexpr int vn = Vec16<T>::n;
   QuadPos p;
   if (!quad_pos<G>(a, k, p)) return;
   const long long nn = a.nn;
-  float s0[4][G], s1[4][G], xs[4][2 * G];
-  if (MODE != kLJacobiZero) quad_sums<float, G>(a, p, cs, x, s0, s1, xs);
+  T s0[4][G], s1[4][G], xs[4][2 * G];
+  if (MODE != kLJacobiZero) quad_sums<T, G>(a, p, cs, x, s0, s1, xs);
 #pragma unroll
   for (int pc = 0; pc < 4; pc++) {
     const int oy = pc & 1, oz = pc >> 1;
     if ((oy == 0 && p.by == 0) || (oz == 0 && p.bz == 0)) continue;  // a boundary line
     const long long nv = p.base + nn * (oy + nn * oz);
-    const float d0 = cs[2 * pc * kCst + kCst - 1], d1 = cs[(2 * pc + 1) * kCst + kCst - 1];
-    float fv[2 * G];
+    const T d0 = cs[2 * pc * kCst + kCst - 1], d1 = cs[(2 * pc + 1) * kCst + kCst - 1];
+    T fv[2 * G];
     if constexpr (G == 1) {
-      const f2u t = *(const f2u *)(f + nv);
+      const V2 t = *(const V2 *)(f + nv);
       fv[0] = t.x;
       fv[1] = t.y;
     } else {
 #pragma unroll
-      for (int h = 0; h < G / 2; h++) {
-        const f4u t = *(const f4u *)(f + nv + 4 * h);
+      for (int h = 0; h < 2 * G / vn; h++) {
+        const V16 t = *(const V16 *)(f + nv + vn * h);
 #pragma unroll
-        for (int e = 0; e < 4; e++) fv[4 * h + e] = t[e];
+        for (int e = 0; e < vn; e++) fv[vn * h + e] = t[e];
       }
     }
-    float r[2 * G];
+    T r[2 * G];
 #pragma unroll
     for (int q = 0; q < G; q++) {
       if (MODE == kLJacobiZero) {
@@ -693,14 +709,19 @@ __host__ __device__ __attribute__((always_inline)) inline void lat_quad_node(con
         r[2 * q + 1] = xs[pc][2 * q + 1] + omega * (fv[2 * q + 1] - s1[pc][q]) * d1;
       }
     }
-    // the segment's 2G nodes are adjacent: vector stores (4-byte alignment
-    // suffices) unless its first vertex is a boundary node (not written)
+    // the segment's 2G nodes are adjacent: vector stores (the alignment of
+    // T suffices) unless its first vertex is a boundary node (not written)
     if (p.hv) {
       if constexpr (G == 1) {
-        *(f2u *)(out + nv) = f2u{r[0], r[1]};
+        *(V2 *)(out + nv) = V2{r[0], r[1]};
       } else {
 #pragma unroll
-        for (int h = 0; h < G / 2; h++) *(f4u *)(out + nv + 4 * h) = f4u{r[4 * h], r[4 * h + 1], r[4 * h + 2], r[4 * h + 3]};
+        for (int h = 0; h < 2 * G / vn; h++) {
+          V16 t;
+#pragma unroll
+          for (int e = 0; e < vn; e++) t[e] = r[vn * h + e];
+          *(V16 *)(out + nv + vn * h) = t;
+        }
       }
     } else {
 #pragma unroll
@@ -709,25 +730,23 @@ __host__ __device__ __attribute__((always_inline)) inline void lat_quad_node(con
   }
 }
 
-template <int G, int MODE, int TB>
-__global__ __launch_bounds__(TB) void lat_quad_gk(LatArgs a, const float *__restrict__ cst,
-                                                  const float *__restrict__ x, const float *__restrict__ f,
-                                                  float *__restrict__ out, float omega, int xcd) {
-  __shared__ float cs[8 * kCst];
+template <int G, int MODE, int TB, typename T>
+__global__ __launch_bounds__(TB) void lat_quad_gk(LatArgs a, const T *__restrict__ cst, const T *__restrict__ x,
+                                                  const T *__restrict__ f, T *__restrict__ out, T omega, int xcd) {
+  __shared__ T cs[8 * kCst];
   for (int i = threadIdx.x; i < 8 * kCst; i += TB) cs[i] = cst[i];
   __syncthreads();
   const int bid = xcd ? xcd_block(blockIdx.x, gridDim.x) : (int)blockIdx.x;
-  lat_quad_node<G, MODE>(a, (long long)bid * TB + threadIdx.x, cs, x, f, out, omega);
+  lat_quad_node<G, MODE, T>(a, (long long)bid * TB + threadIdx.x, cs, x, f, out, omega);
 }
 
-template <int P, int MODE>
-__global__ __launch_bounds__(kB) void lat_sweep_k(LatArgs a, const float *__restrict__ val,
-                                                  const float *__restrict__ inv, const float *__restrict__ cst,
-                                                  const float *__restrict__ x, const float *__restrict__ f,
-                                                  float *__restrict__ out, float omega) {
+template <int P, int MODE, typename T>
+__global__ __launch_bounds__(kB) void lat_sweep_k(LatArgs a, const T *__restrict__ val, const T *__restrict__ inv,
+                                                  const T *__restrict__ cst, const T *__restrict__ x,
+                                                  const T *__restrict__ f, T *__restrict__ out, T omega) {
   const int c = block_class(a.bstart, a.nclass, (int)blockIdx.x);
   const long long k = (long long)(blockIdx.x - a.bstart[c]) * kB + threadIdx.x;
-  if (k < a.c[c].nodes) lat_class_node<P, MODE>(a, c, k, val, inv, cst, x, f, out, omega);
+  if (k < a.c[c].nodes) lat_class_node<P, MODE, T>(a, c, k, val, inv, cst, x, f, out, omega);
 }
 
 // 1D transfer weights (nodal interpolation of the coarse basis at the fine
@@ -768,18 +787,20 @@ struct Restr1D<2, 1> {
 // omega * f * d_c at the nodes it writes (d_c = cst[c kCst + kCst - 1], the
 // value and expression the sweep uses, so the bits are the same), and the
 // sweep's launch is saved.  x == nullptr: f only.
-struct ZeroSweep {
-  float *x;
-  const float *cst;
-  float omega;
+template <typename T>
+struct ZeroSweepT {
+  T *x;
+  const T *cst;
+  T omega;
 };
+using ZeroSweep = ZeroSweepT<float>;
 
-template <int P, int PX, int PY, int PZ>
+template <int P, int PX, int PY, int PZ, typename T>
 __host__ __device__ inline void restrict_node(const LatArgs &ca, const LatDev &C, long long k, int nnf,
-                                              const float *__restrict__ fine, float *__restrict__ coarse,
-                                              int cls, const ZeroSweep &zs) {
+                                              const T *__restrict__ fine, T *__restrict__ coarse, int cls,
+                                              const ZeroSweepT<T> &zs) {
   // the class value first: its load overlaps the gathers
-  const float dz = zs.x ? zs.cst[cls * kCst + kCst - 1] : 0.f;
+  const T dz = zs.x ? zs.cst[cls * kCst + kCst - 1] : T(0);
   using RX = Restr1D<P, PX>;
   using RY = Restr1D<P, PY>;
   using RZ = Restr1D<P, PZ>;
@@ -787,13 +808,13 @@ __host__ __device__ inline void restrict_node(const LatArgs &ca, const LatDev &C
   class_coords(C, k, kx, ky, kz);
   const int Xc = C.lo[0] + C.step * kx, Yc = C.lo[1] + C.step * ky, Zc = C.lo[2] + C.step * kz;
   const long long F = nnf, centre = 2 * Xc + F * (2 * Yc + F * 2 * Zc);
-  float s = 0.f;
+  T s = 0;
 #pragma unroll
   for (int c = 0; c < RZ::n; c++) {
-    float sy = 0.f;
+    T sy = 0;
 #pragma unroll
     for (int b = 0; b < RY::n; b++) {
-      float sx = 0.f;
+      T sx = 0;
 #pragma unroll
       for (int a = 0; a < RX::n; a++) sx += RX::w(a) * fine[centre + RX::off(a) + F * (RY::off(b) + F * RZ::off(c))];
       sy += RY::w(b) * sx;
@@ -805,10 +826,10 @@ __host__ __device__ inline void restrict_node(const LatArgs &ca, const LatDev &C
   if (zs.x) zs.x[node] = zs.omega * s * dz;
 }
 
-template <int P>
+template <int P, typename T>
 __host__ __device__ inline void restrict_class_node(const LatArgs &ca, int c, long long k, int nnf,
-                                                    const float *__restrict__ fine, float *__restrict__ coarse,
-                                                    const ZeroSweep &zs) {
+                                                    const T *__restrict__ fine, T *__restrict__ coarse,
+                                                    const ZeroSweepT<T> &zs) {
   const LatDev &C = ca.c[c];
   if (P == 1) {
     restrict_node<1, 0, 0, 0>(ca, C, k, nnf, fine, coarse, c, zs);
@@ -828,9 +849,9 @@ __host__ __device__ inline void restrict_class_node(const LatArgs &ca, int c, lo
 
 // coarse interior <- R fine (DefectRestriction + CorrectDefect: the coarse
 // boundary stays zero); ca: the coarse level's classes
-template <int P>
-__global__ __launch_bounds__(kB) void lat_restrict_k(LatArgs ca, int nnf, const float *__restrict__ fine,
-                                                     float *__restrict__ coarse, ZeroSweep zs) {
+template <int P, typename T>
+__global__ __launch_bounds__(kB) void lat_restrict_k(LatArgs ca, int nnf, const T *__restrict__ fine,
+                                                     T *__restrict__ coarse, ZeroSweepT<T> zs) {
   const int c = block_class(ca.bstart, ca.nclass, (int)blockIdx.x);
   const long long k = (long long)(blockIdx.x - ca.bstart[c]) * kB + threadIdx.x;
   if (k < ca.c[c].nodes) restrict_class_node<P>(ca, c, k, nnf, fine, coarse, zs);
@@ -844,13 +865,16 @@ __global__ __launch_bounds__(kB) void lat_restrict_k(LatArgs ca, int nnf, const 
 // consecutive pairs) instead of 5 + 3 loads at a stride of 4 floats.  Each
 // node's sum keeps restrict_node's order.  A boundary vertex (ix = 0) is not
 // written; its left values are read from the centre.
-template <int PY, int PZ>
-__host__ __device__ inline void restrict_pair(const LatArgs &ca, long long k, int nnf, const float *__restrict__ fine,
-                                              float *__restrict__ coarse, const ZeroSweep &zs) {
+template <int PY, int PZ, typename T>
+__host__ __device__ inline void restrict_pair(const LatArgs &ca, long long k, int nnf, const T *__restrict__ fine,
+                                              T *__restrict__ coarse, const ZeroSweepT<T> &zs) {
+  typedef typename Vec2<T>::type V2;
+  typedef typename Vec16<T>::type V16;
+  constexpr int vn = Vec16<T>::n;
   // vertex class 2 PY + 4 PZ, midpoint class one above; loaded first so the
   // loads overlap the gathers
   constexpr int cv = 2 * PY + 4 * PZ;
-  const float dz0 = zs.x ? zs.cst[cv * kCst + kCst - 1] : 0.f, dz1 = zs.x ? zs.cst[(cv + 1) * kCst + kCst - 1] : 0.f;
+  const T dz0 = zs.x ? zs.cst[cv * kCst + kCst - 1] : T(0), dz1 = zs.x ? zs.cst[(cv + 1) * kCst + kCst - 1] : T(0);
   using RX0 = Restr1D<2, 0>;
   using RX1 = Restr1D<2, 1>;
   using RY = Restr1D<2, PY>;
@@ -861,24 +885,25 @@ __host__ __device__ inline void restrict_pair(const LatArgs &ca, long long k, in
   const long long Xc = u - t * nnc, Yc = t - tz * nnc, Zc = tz;
   const long long centre = 2 * Xc + F * (2 * Yc + F * 2 * Zc);
   const int lo = q.hv ? 0 : 3;
-  float s0 = 0.f, s1 = 0.f;
+  T s0 = 0, s1 = 0;
 #pragma unroll
   for (int c = 0; c < RZ::n; c++) {
-    float sy0 = 0.f, sy1 = 0.f;
+    T sy0 = 0, sy1 = 0;
 #pragma unroll
     for (int b = 0; b < RY::n; b++) {
-      const float *fl = fine + centre + F * (RY::off(b) + F * RZ::off(c));
-      float w[7];
+      const T *fl = fine + centre + F * (RY::off(b) + F * RZ::off(c));
+      T w[7];
       w[0] = fl[lo - 3];
-      const f2u l2 = *(const f2u *)(fl + lo - 2);
+      const V2 l2 = *(const V2 *)(fl + lo - 2);
       w[1] = l2.x;
       w[2] = l2.y;
-      const f4u m = *(const f4u *)fl;
-      w[3] = m.x;
-      w[4] = m.y;
-      w[5] = m.z;
-      w[6] = m.w;
-      float sx0 = 0.f, sx1 = 0.f;
+#pragma unroll
+      for (int h = 0; h < 4 / vn; h++) {
+        const V16 m = *(const V16 *)(fl + vn * h);
+#pragma unroll
+        for (int e = 0; e < vn; e++) w[3 + vn * h + e] = m[e];
+      }
+      T sx0 = 0, sx1 = 0;
 #pragma unroll
       for (int a = 0; a < RX0::n; a++) sx0 += RX0::w(a) * w[3 + RX0::off(a)];
 #pragma unroll
@@ -889,20 +914,21 @@ __host__ __device__ inline void restrict_pair(const LatArgs &ca, long long k, in
     s0 += RZ::w(c) * sy0;
     s1 += RZ::w(c) * sy1;
   }
-  // vertex and midpoint are adjacent: one 8-byte store (4-byte alignment
+  // vertex and midpoint are adjacent: one paired store (the alignment of T
   // suffices) unless the vertex is a boundary node
   if (q.hv) {
-    *(f2u *)(coarse + q.nv) = f2u{s0, s1};
-    if (zs.x) *(f2u *)(zs.x + q.nv) = f2u{zs.omega * s0 * dz0, zs.omega * s1 * dz1};
+    *(V2 *)(coarse + q.nv) = V2{s0, s1};
+    if (zs.x) *(V2 *)(zs.x + q.nv) = V2{zs.omega * s0 * dz0, zs.omega * s1 * dz1};
   } else {
     coarse[q.nv + 1] = s1;
     if (zs.x) zs.x[q.nv + 1] = zs.omega * s1 * dz1;
   }
 }
 
+template <typename T>
 __host__ __device__ inline void restrict_pair_node(const LatArgs &ca, int pc, long long k, int nnf,
-                                                   const float *__restrict__ fine, float *__restrict__ coarse,
-                                                   const ZeroSweep &zs) {
+                                                   const T *__restrict__ fine, T *__restrict__ coarse,
+                                                   const ZeroSweepT<T> &zs) {
   switch (pc) {
     case 0: restrict_pair<0, 0>(ca, k, nnf, fine, coarse, zs); break;
     case 1: restrict_pair<1, 0>(ca, k, nnf, fine, coarse, zs); break;
@@ -920,8 +946,9 @@ __host__ __device__ inline void restrict_pair_node(const LatArgs &ca, int pc, lo
 // 6.0 us (the class-order re-reads come from the Infinity Cache), and the
 // mixed solve is unchanged; class order is the default
 // (CD3D_RESTRICT_INTER=1 selects the other, bitwise the same)
-__global__ __launch_bounds__(kB) void lat_restrict_pair_k(LatArgs ca, int nnf, const float *__restrict__ fine,
-                                                          float *__restrict__ coarse, int inter, ZeroSweep zs) {
+template <typename T>
+__global__ __launch_bounds__(kB) void lat_restrict_pair_k(LatArgs ca, int nnf, const T *__restrict__ fine,
+                                                          T *__restrict__ coarse, int inter, ZeroSweepT<T> zs) {
   int pc = 0, j;
   if (inter) {
     const int lb = xcd_block(blockIdx.x, gridDim.x);
@@ -1012,55 +1039,55 @@ __host__ __device__ inline void prolong_cell(long long t, int ncc, int nnf, int 
 // device the weights of prolong_cell are compile-time constants and its
 // products may be folded differently, so every device path (the
 // launch-per-step V-cycle and the one-workgroup program) uses this form.
-template <int P>
-__host__ __device__ inline void prolong_row(long long t, int ncc, int nnf, int nnc, const float *__restrict__ coarse,
-                                            float *__restrict__ x, float damp) {
-  constexpr int P1 = P + 1, T = 2 * P;
+template <int P, typename T>
+__host__ __device__ inline void prolong_row(long long t, int ncc, int nnf, int nnc, const T *__restrict__ coarse,
+                                            T *__restrict__ x, Sc<T> damp) {
+  constexpr int P1 = P + 1, NF = 2 * P;
   // 32-bit unsigned division: t counts fine-level rows, below 2^31
   const unsigned n = (unsigned)ncc;
   unsigned r = (unsigned)t / n;
   const int cx = (int)((unsigned)t - r * n);
-  const int ty = (int)(r % T);
-  r /= T;
-  const int tz = (int)(r % T);
-  r /= T;
+  const int ty = (int)(r % NF);
+  r /= NF;
+  const int tz = (int)(r % NF);
+  r /= NF;
   const int cy = (int)(r % n), cz = (int)(r / n);
-  const int Y = T * cy + ty, Z = T * cz + tz;
+  const int Y = NF * cy + ty, Z = NF * cz + tz;
   if (Y == 0 || Z == 0) return;
   const long long C = nnc, F = nnf;
-  float pz[P1][P1];
+  T pz[P1][P1];
 #pragma unroll
   for (int b = 0; b < P1; b++)
 #pragma unroll
     for (int a = 0; a < P1; a++) {
-      float v = 0.f;
+      T v = 0;
 #pragma unroll
       for (int c = 0; c < P1; c++)
         v += prol_w<P>(tz, c) * coarse[(P * cx + a) + C * ((P * cy + b) + C * (P * cz + c))];
       pz[b][a] = v;
     }
-  float py[P1];
+  T py[P1];
 #pragma unroll
   for (int a = 0; a < P1; a++) {
-    float v = 0.f;
+    T v = 0;
 #pragma unroll
     for (int b = 0; b < P1; b++) v += prol_w<P>(ty, b) * pz[b][a];
     py[a] = v;
   }
 #pragma unroll
-  for (int tx = 0; tx < T; tx++) {
-    const int X = T * cx + tx;
+  for (int tx = 0; tx < NF; tx++) {
+    const int X = NF * cx + tx;
     if (X == 0) continue;
-    float v = 0.f;
+    T v = 0;
 #pragma unroll
     for (int a = 0; a < P1; a++) v += prol_w<P>(tx, a) * py[a];
     x[X + F * (Y + F * (long long)Z)] += damp * v;
   }
 }
 
-template <int P>
-__global__ __launch_bounds__(kB) void lat_prolong_k(int ncc, int nnf, int nnc, const float *__restrict__ coarse,
-                                                    float *__restrict__ x, float damp) {
+template <int P, typename T>
+__global__ __launch_bounds__(kB) void lat_prolong_k(int ncc, int nnf, int nnc, const T *__restrict__ coarse,
+                                                    T *__restrict__ x, T damp) {
   const long long t = (long long)blockIdx.x * kB + threadIdx.x;
   if (t < (long long)ncc * ncc * ncc * 4 * P * P) prolong_row<P>(t, ncc, nnf, nnc, coarse, x, damp);
 }
@@ -1335,7 +1362,9 @@ __global__ __launch_bounds__(kCst) void class_stencil_k(LatArgs a, const double 
   }
   if (s == kCst - 1) {
     const int d0[3] = {0, 0, 0};
-    cst[c * kCst + kCst - 1] = (float)(1.0 / stencil_entry<P>(E, nl, l, d0));
+    const double di = 1.0 / stencil_entry<P>(E, nl, l, d0);
+    st[c * kCst + kCst - 1] = di;  // no stencil has kCst entries: the FP64 sweeps find 1/a_ii here
+    cst[c * kCst + kCst - 1] = (float)di;
     double r = 0.0;
     for (int az = 0; az < nl[2]; az++)
       for (int ay = 0; ay < nl[1]; ay++)
@@ -1865,15 +1894,36 @@ __global__ void cast_f2d_k(long long n, const float *__restrict__ a, double *__r
     b[i] = (double)a[i];
 }
 
-// DOF-ordered f64 <-> lattice-ordered f32 (the boundary of the lattice vector
-// is left untouched: it stays zero)
+// DOF-ordered f64 <-> lattice-ordered vectors (the boundary of the lattice
+// vector is left untouched: it stays zero)
+template <typename T>
 __global__ void dof_to_lat_k(int n, int nact, const int *__restrict__ dof2node, const double *__restrict__ v,
-                             float *__restrict__ l) {
+                             T *__restrict__ l) {
   const int d = blockIdx.x * kB + threadIdx.x;
-  if (d < nact) l[dof2node[d]] = (float)v[d];
+  if (d < nact) l[dof2node[d]] = (T)v[d];
 }
 
-__global__ void lat_to_dof_k(int n, int nact, const int *__restrict__ dof2node, const float *__restrict__ l,
+// zeros at the boundary nodes of count lattice vectors, ld apart
+__global__ void clear_boundary_k(int nact, int ndof, const int *__restrict__ dof2node, double *__restrict__ v,
+                                 int64_t ld, int count) {
+  const int d = nact + blockIdx.x * kB + threadIdx.x;
+  if (d >= ndof) return;
+  const int node = dof2node[d];
+  for (int k = blockIdx.y; k < count; k += gridDim.y) v[(int64_t)k * ld + node] = 0.0;
+}
+__global__ void clear_boundary4_k(int nact, int ndof, const int *__restrict__ dof2node, double *__restrict__ a,
+                                  double *__restrict__ b, double *__restrict__ c, double *__restrict__ e) {
+  const int d = nact + blockIdx.x * kB + threadIdx.x;
+  if (d >= ndof) return;
+  const int node = dof2node[d];
+  a[node] = 0.0;
+  b[node] = 0.0;
+  c[node] = 0.0;
+  e[node] = 0.0;
+}
+
+template <typename T>
+__global__ void lat_to_dof_k(int n, int nact, const int *__restrict__ dof2node, const T *__restrict__ l,
                              double *__restrict__ v) {
   const int d = blockIdx.x * kB + threadIdx.x;
   if (d < n) v[d] = d < nact ? (double)l[dof2node[d]] : 0.0;
@@ -1978,20 +2028,41 @@ static bool all_uni(const LatArgs &a) {
   return true;
 }
 
-template <int MODE>
-void lat_sweep(hipStream_t s, const DevLevel &L, int order, const float *x, const float *f, float *out,
-               float omega) {
+// the per-class and per-node values of a level for sweeps of value type T
+template <typename T>
+struct LatVals;
+template <>
+struct LatVals<float> {
+  const float *val, *inv, *cst;
+  bool affine;
+  explicit LatVals(const DevLevel &L) : val(L.lval), inv(L.linv), cst(L.lcst), affine(L.lat_affine) {}
+};
+// FP64: the class stencils of the assembly (levels with lat_exact64 or
+// lat_aff64 only)
+template <>
+struct LatVals<double> {
+  const double *val = nullptr, *inv = nullptr, *cst;
+  bool affine;
+  explicit LatVals(const DevLevel &L) : cst(L.lst64), affine(L.lat_aff64) {}
+};
+
+template <int MODE, typename T>
+void lat_sweep(hipStream_t s, const DevLevel &L, int order, const T *x, const T *f, T *out, T omega) {
   const LatArgs a = lat_args(L);
+  const LatVals<T> v(L);
   const int grid = a.bstart[L.nclass];
   if (grid <= 0) return;
-  if (L.lat_affine) {
+  if (v.affine) {
     const LatAff af = lat_aff(L);
-    if (order == 1) lat_aff_sweep_k<1, MODE><<<grid, kB, 0, s>>>(a, af, x, f, out, omega);
-    else lat_aff_sweep_k<2, MODE><<<grid, kB, 0, s>>>(a, af, x, f, out, omega);
+    if (order == 1) lat_aff_sweep_k<1, MODE, T><<<grid, kB, 0, s>>>(a, af, x, f, out, omega);
+    else lat_aff_sweep_k<2, MODE, T><<<grid, kB, 0, s>>>(a, af, x, f, out, omega);
     return;
   }
-  const int G = order == 2 && lat_pairs() && L.nn > kPairMinNN && all_uni(a) ? pair_group(a, 4) : 1;
-  if (order == 1) lat_sweep_k<1, MODE><<<grid, kB, 0, s>>>(a, L.lval, L.linv, L.lcst, x, f, out, omega);
+  const bool uni = all_uni(a);
+  if (sizeof(T) == 8 && !uni) throw std::logic_error("FP64 lattice sweep without class stencils");
+  const bool pairs = order == 2 && lat_pairs() && L.nn > kPairMinNN;
+  const int G = pairs && uni ? pair_group(a, sizeof(T) == 4 ? 4 : 2) : 1;
+  if (order == 1) lat_sweep_k<1, MODE, T><<<grid, kB, 0, s>>>(a, v.val, v.inv, v.cst, x, f, out, omega);
   else if (G > 1 && lat_quads()) {
     // measured on the 129^3-node level of a 64^3-cell Q2 mesh (FP32 Jacobi
     // sweep): 2 pairs per thread, 256 threads, XCD-contiguous blocks 12.4 us;
@@ -2001,49 +2072,65 @@ void lat_sweep(hipStream_t s, const DevLevel &L, int order, const float *x, cons
     // (CD3D_QUAD_G, CD3D_QUAD_TB, CD3D_QUAD_XCD select the variants)
     const char *eg = getenv("CD3D_QUAD_G"), *et = getenv("CD3D_QUAD_TB"), *ex = getenv("CD3D_QUAD_XCD");
     const int gq_g = eg ? atoi(eg) : 2, tb = et ? atoi(et) : 256, xcd = ex ? atoi(ex) : 1;
-    // G == 4 implies 2 divides the pairs per line too
-    const int Gq = gq_g == 1 ? 1 : (gq_g == 4 && G == 4) ? 4 : 2;
-    const long long n = a.c[1].cnt[0], threads = n / Gq * n * n;
-    const int gq = (int)((threads + tb - 1) / tb);
-    if (tb == 128) {
-      if (Gq == 1) lat_quad_gk<1, MODE, 128><<<gq, 128, 0, s>>>(a, L.lcst, x, f, out, omega, xcd);
-      else if (Gq == 2) lat_quad_gk<2, MODE, 128><<<gq, 128, 0, s>>>(a, L.lcst, x, f, out, omega, xcd);
-      else lat_quad_gk<4, MODE, 128><<<gq, 128, 0, s>>>(a, L.lcst, x, f, out, omega, xcd);
+    const long long n = a.c[1].cnt[0];
+    if constexpr (sizeof(T) == 8) {
+      // FP64: one pair per line (two pairs take 256 VGPRs, one wave per SIMD)
+      lat_quad_gk<1, MODE, 256, T><<<(int)((n * n * n + 255) / 256), 256, 0, s>>>(a, v.cst, x, f, out, omega, xcd);
     } else {
-      if (Gq == 1) lat_quad_gk<1, MODE, 256><<<gq, 256, 0, s>>>(a, L.lcst, x, f, out, omega, xcd);
-      else if (Gq == 2) lat_quad_gk<2, MODE, 256><<<gq, 256, 0, s>>>(a, L.lcst, x, f, out, omega, xcd);
-      else lat_quad_gk<4, MODE, 256><<<gq, 256, 0, s>>>(a, L.lcst, x, f, out, omega, xcd);
+      // G == 4 implies 2 divides the pairs per line too
+      const int Gq = gq_g == 1 ? 1 : (gq_g == 4 && G == 4) ? 4 : 2;
+      const long long threads = n / Gq * n * n;
+      const int gq = (int)((threads + tb - 1) / tb);
+      if (tb == 128) {
+        if (Gq == 1) lat_quad_gk<1, MODE, 128, T><<<gq, 128, 0, s>>>(a, v.cst, x, f, out, omega, xcd);
+        else if (Gq == 2) lat_quad_gk<2, MODE, 128, T><<<gq, 128, 0, s>>>(a, v.cst, x, f, out, omega, xcd);
+        else lat_quad_gk<4, MODE, 128, T><<<gq, 128, 0, s>>>(a, v.cst, x, f, out, omega, xcd);
+      } else {
+        if (Gq == 1) lat_quad_gk<1, MODE, 256, T><<<gq, 256, 0, s>>>(a, v.cst, x, f, out, omega, xcd);
+        else if (Gq == 2) lat_quad_gk<2, MODE, 256, T><<<gq, 256, 0, s>>>(a, v.cst, x, f, out, omega, xcd);
+        else lat_quad_gk<4, MODE, 256, T><<<gq, 256, 0, s>>>(a, v.cst, x, f, out, omega, xcd);
+      }
     }
-  } else if (G > 1) {
-    const LatArgs ag = group_args(a, G);
-    if (G == 2) lat_pair_gk<MODE, 2><<<ag.pstart[4], kB, 0, s>>>(ag, L.lcst, x, f, out, omega);
-    else lat_pair_gk<MODE, 4><<<ag.pstart[4], kB, 0, s>>>(ag, L.lcst, x, f, out, omega);
-  } else if (lat_pairs() && L.nn > kPairMinNN && all_uni(a))
-    lat_pair_k<MODE, true><<<a.pstart[4], kB, 0, s>>>(a, L.lval, L.linv, L.lcst, x, f, out, omega);
-  else if (lat_pairs() && L.nn > kPairMinNN)
-    lat_pair_k<MODE, false><<<a.pstart[4], kB, 0, s>>>(a, L.lval, L.linv, L.lcst, x, f, out, omega);
-  else lat_sweep_k<2, MODE><<<grid, kB, 0, s>>>(a, L.lval, L.linv, L.lcst, x, f, out, omega);
+  } else if (G > 1 && sizeof(T) == 4) {
+    if constexpr (sizeof(T) == 4) {
+      const LatArgs ag = group_args(a, G);
+      if (G == 2) lat_pair_gk<MODE, 2><<<ag.pstart[4], kB, 0, s>>>(ag, v.cst, x, f, out, omega);
+      else lat_pair_gk<MODE, 4><<<ag.pstart[4], kB, 0, s>>>(ag, v.cst, x, f, out, omega);
+    }
+  } else if (pairs && uni)
+    lat_pair_k<MODE, true, T><<<a.pstart[4], kB, 0, s>>>(a, v.val, v.inv, v.cst, x, f, out, omega);
+  else if (pairs)
+    lat_pair_k<MODE, false, T><<<a.pstart[4], kB, 0, s>>>(a, v.val, v.inv, v.cst, x, f, out, omega);
+  else lat_sweep_k<2, MODE, T><<<grid, kB, 0, s>>>(a, v.val, v.inv, v.cst, x, f, out, omega);
 }
 
 }  // namespace
 
-void kl_jacobi(hipStream_t s, const DevLevel &L, int order, const float *x, const float *f, float *out,
-               float omega) {
-  lat_sweep<kLJacobi>(s, L, order, x, f, out, omega);
+template <typename T>
+void kl_jacobi(hipStream_t s, const DevLevel &L, int order, const T *x, const T *f, T *out, T omega) {
+  lat_sweep<kLJacobi, T>(s, L, order, x, f, out, omega);
 }
-void kl_jacobi_zero(hipStream_t s, const DevLevel &L, int order, const float *f, float *out, float omega) {
-  lat_sweep<kLJacobiZero>(s, L, order, nullptr, f, out, omega);
+template <typename T>
+void kl_jacobi_zero(hipStream_t s, const DevLevel &L, int order, const T *f, T *out, T omega) {
+  lat_sweep<kLJacobiZero, T>(s, L, order, nullptr, f, out, omega);
 }
-void kl_defect(hipStream_t s, const DevLevel &L, int order, const float *x, const float *f, float *d) {
-  lat_sweep<kLDefect>(s, L, order, x, f, d, 0.f);
+template <typename T>
+void kl_defect(hipStream_t s, const DevLevel &L, int order, const T *x, const T *f, T *d) {
+  lat_sweep<kLDefect, T>(s, L, order, x, f, d, T(0));
 }
+template void kl_jacobi<float>(hipStream_t, const DevLevel &, int, const float *, const float *, float *, float);
+template void kl_jacobi<double>(hipStream_t, const DevLevel &, int, const double *, const double *, double *, double);
+template void kl_jacobi_zero<float>(hipStream_t, const DevLevel &, int, const float *, float *, float);
+template void kl_jacobi_zero<double>(hipStream_t, const DevLevel &, int, const double *, double *, double);
+template void kl_defect<float>(hipStream_t, const DevLevel &, int, const float *, const float *, float *);
+template void kl_defect<double>(hipStream_t, const DevLevel &, int, const double *, const double *, double *);
 bool kl_zero_sweep_fusable(const DevLevel &C) {
-  if (C.lat_affine || C.nclass <= 0) return false;
+  if (C.lat_affine || C.lat_aff64 || C.nclass <= 0) return false;
   for (int c = 0; c < C.nclass; c++)
     if (!C.uni[c]) return false;
   return true;
 }
-bool kl_top_zero_sweep(const DevLevel &F, int order, float omega, float *x, TopZeroSweep &zt) {
+static bool top_zero_classes(const DevLevel &F, int order) {
   // uniform stencils, and classes that are exactly the parity sub-lattices of
   // the interior (class c holds the nodes of parity c, all of them)
   if (!kl_zero_sweep_fusable(F) || F.nclass != (order == 2 ? 8 : 1)) return false;
@@ -2058,40 +2145,63 @@ bool kl_top_zero_sweep(const DevLevel &F, int order, float omega, float *x, TopZ
     }
     tot += L.nodes;
   }
-  if (tot != (long long)(nn - 2) * (nn - 2) * (nn - 2)) return false;
+  return tot == (long long)(nn - 2) * (nn - 2) * (nn - 2);
+}
+bool kl_top_zero_sweep(const DevLevel &F, int order, float omega, float *x, TopZeroSweep &zt) {
+  if (!top_zero_classes(F, order)) return false;
   zt.x = x;
   zt.d = F.lcst + kCst - 1;
   zt.dstride = kCst;
   zt.omega = omega;
-  zt.nn = nn;
+  zt.nn = F.nn;
   zt.order = order;
   return true;
 }
-void kl_restrict(hipStream_t s, const DevLevel &F, const DevLevel &C, int order, const float *fine, float *coarse,
-                 float *zero_sweep, float omega) {
+bool kl_top_zero_sweep(const DevLevel &F, int order, double omega, double *x, TopZeroSweep &zt) {
+  if (!F.lat_exact64 || !top_zero_classes(F, order)) return false;
+  zt.x64 = x;
+  zt.d64 = F.lst64 + kCst - 1;
+  zt.dstride = kCst;
+  zt.omega64 = omega;
+  zt.nn = F.nn;
+  zt.order = order;
+  return true;
+}
+template <typename T>
+void kl_restrict(hipStream_t s, const DevLevel &F, const DevLevel &C, int order, const T *fine, T *coarse,
+                 T *zero_sweep, T omega) {
   const LatArgs ca = lat_args(C);
   const int grid = ca.bstart[C.nclass];
   if (grid <= 0) return;
   if (zero_sweep && !kl_zero_sweep_fusable(C))
     throw std::logic_error("the restriction writes the zero-start sweep only for uniform class stencils");
-  const ZeroSweep zs{zero_sweep, C.lcst, omega};
-  if (order == 1) lat_restrict_k<1><<<grid, kB, 0, s>>>(ca, F.nn, fine, coarse, zs);
+  const ZeroSweepT<T> zs{zero_sweep, LatVals<T>(C).cst, omega};
+  if (order == 1) lat_restrict_k<1, T><<<grid, kB, 0, s>>>(ca, F.nn, fine, coarse, zs);
   else if (lat_pairs() && C.nn > kPairMinNN) {
     const char *e = getenv("CD3D_RESTRICT_INTER");
     const int inter = e ? atoi(e) : 0;
     int nbmax = 0;
     for (int pc = 0; pc < 4; pc++) nbmax = std::max(nbmax, ca.pstart[pc + 1] - ca.pstart[pc]);
-    lat_restrict_pair_k<<<inter ? 4 * nbmax : ca.pstart[4], kB, 0, s>>>(ca, F.nn, fine, coarse, inter, zs);
+    lat_restrict_pair_k<T><<<inter ? 4 * nbmax : ca.pstart[4], kB, 0, s>>>(ca, F.nn, fine, coarse, inter, zs);
   }
-  else lat_restrict_k<2><<<grid, kB, 0, s>>>(ca, F.nn, fine, coarse, zs);
+  else lat_restrict_k<2, T><<<grid, kB, 0, s>>>(ca, F.nn, fine, coarse, zs);
 }
-void kl_prolong_update(hipStream_t s, const DevLevel &F, const DevLevel &C, int order, const float *coarse, float *x,
-                       float damp) {
+template <typename T>
+void kl_prolong_update(hipStream_t s, const DevLevel &F, const DevLevel &C, int order, const T *coarse, T *x, T damp) {
   const long long ncc = (C.nn - 1) / order, n = ncc * ncc * ncc * 4 * order * order;  // (cell, fine Z, fine Y)
   if (n <= 0) return;
-  if (order == 1) lat_prolong_k<1><<<(int)((n + kB - 1) / kB), kB, 0, s>>>((int)ncc, F.nn, C.nn, coarse, x, damp);
-  else lat_prolong_k<2><<<(int)((n + kB - 1) / kB), kB, 0, s>>>((int)ncc, F.nn, C.nn, coarse, x, damp);
+  const int grid = (int)((n + kB - 1) / kB);
+  if (order == 1) lat_prolong_k<1, T><<<grid, kB, 0, s>>>((int)ncc, F.nn, C.nn, coarse, x, damp);
+  else lat_prolong_k<2, T><<<grid, kB, 0, s>>>((int)ncc, F.nn, C.nn, coarse, x, damp);
 }
+template void kl_restrict<float>(hipStream_t, const DevLevel &, const DevLevel &, int, const float *, float *, float *,
+                                 float);
+template void kl_restrict<double>(hipStream_t, const DevLevel &, const DevLevel &, int, const double *, double *,
+                                  double *, double);
+template void kl_prolong_update<float>(hipStream_t, const DevLevel &, const DevLevel &, int, const float *, float *,
+                                       float);
+template void kl_prolong_update<double>(hipStream_t, const DevLevel &, const DevLevel &, int, const double *, double *,
+                                        double);
 hipError_t kl_detect_uniform(hipStream_t s, DevLevel &L, int *flag_host, bool *all_uniform) {
   *all_uniform = true;
   if (L.nclass <= 0) return hipSuccess;
@@ -2344,11 +2454,28 @@ void kl_small_vcycle(hipStream_t st, const DevLevel *levels, int top, int order,
   else lat_small_k<2, false><<<1, small_threads<2>(), 0, st>>>(s);
 }
 
-void kl_from_dof(hipStream_t s, const DevLevel &L, const double *v, float *l) {
+void kl_clear_boundary(hipStream_t s, const DevLevel &L, double *v, int64_t ld, int count) {
+  const int nd = L.ndof - L.nact;
+  if (nd <= 0 || count <= 0) return;
+  clear_boundary_k<<<dim3((nd + kB - 1) / kB, std::min(count, 64)), kB, 0, s>>>(L.nact, L.ndof, L.ldof2node, v, ld,
+                                                                              count);
+}
+void kl_clear_boundary4(hipStream_t s, const DevLevel &L, double *a, double *b, double *c, double *d) {
+  const int nd = L.ndof - L.nact;
+  if (nd <= 0) return;
+  clear_boundary4_k<<<(nd + kB - 1) / kB, kB, 0, s>>>(L.nact, L.ndof, L.ldof2node, a, b, c, d);
+}
+template <typename T>
+void kl_from_dof(hipStream_t s, const DevLevel &L, const double *v, T *l) {
   dof_to_lat_k<<<(L.ndof + kB - 1) / kB, kB, 0, s>>>(L.ndof, L.nact, L.ldof2node, v, l);
 }
-void kl_to_dof(hipStream_t s, const DevLevel &L, const float *l, double *v) {
+template <typename T>
+void kl_to_dof(hipStream_t s, const DevLevel &L, const T *l, double *v) {
   lat_to_dof_k<<<(L.ndof + kB - 1) / kB, kB, 0, s>>>(L.ndof, L.nact, L.ldof2node, l, v);
 }
+template void kl_from_dof<float>(hipStream_t, const DevLevel &, const double *, float *);
+template void kl_from_dof<double>(hipStream_t, const DevLevel &, const double *, double *);
+template void kl_to_dof<float>(hipStream_t, const DevLevel &, const float *, double *);
+template void kl_to_dof<double>(hipStream_t, const DevLevel &, const double *, double *);
 
 }  // namespace cd3d

@@ -1,0 +1,85 @@
+"""The plain FP64 form on the lattice (class stencils, lattice order) against
+the same form on the CSR matrices (CD3D_FP64_LATTICE=0): the same matrices,
+smoother and Krylov iteration in FP64, so only the order of the sums differs.
+A product sums at most 125 terms (relative rounding <= 125 eps = 2.8e-14) and a
+V-cycle chains fewer than 50 of them with O(1) factors: 2e-12 for the cycle;
+a solve stops at 1e-10 of its residual after the same number of iterations,
+and its solutions agree to that."""
+import numpy as np
+import pytest
+
+import parmoon_cmg_amd as pm
+
+pytestmark = pytest.mark.gpu
+
+CYCLE_TOL, SOL_TOL = 2e-12, 1e-10
+
+
+def both(monkeypatch, work):
+    out = []
+    for on in ("1", "0"):
+        monkeypatch.setenv("CD3D_FP64_LATTICE", on)
+        out.append(work())
+    return out
+
+
+def rel(a, b):
+    return np.linalg.norm(a - b) / np.linalg.norm(b)
+
+
+# levels by class, by pairs (more than 40 nodes per side) and by quads (more
+# than 2^17 pair groups); odd cells per side; V, W and F cycles; no pre- or
+# post-smoothing; an odd number of sweeps; a coarse smoother other than the
+# exact solve (the DOF-ordered coarse path)
+@pytest.mark.parametrize("order,m,k0,levels,kw", [
+    (1, 1, 1, 2, {}), (1, 3, 0, 4, {}), (1, 5, 0, 3, dict(cycle=2)), (1, 1, 2, 5, dict(pre=2, post=1)),
+    (2, 1, 1, 2, {}), (2, 3, 0, 3, dict(cycle=0)), (2, 11, 0, 2, dict(pre=0, post=2)), (2, 1, 1, 5, dict(pre=2, post=0)),
+    (2, 1, 2, 5, {}), (2, 3, 1, 5, dict(pre=1, post=2)), (2, 2, 0, 3, dict(coarse_smoother=3)),
+    (1, 2, 0, 4, dict(coarse_smoother=1, cycle=2))])
+def test_fp64_lattice_matches_csr(order, m, k0, levels, kw, monkeypatch):
+    P = pm.Problem(order, m, k0, levels, box=(1.0, 0.7, 0.5))
+    P.assemble(pm.coeffs(eps=0.05, b=(1.0, 0.5, 0.25), c=0.3, supg=1, f_val=1.0))
+    i = P.info(levels - 1)
+    r = np.random.default_rng(5).standard_normal(i["ndof"])
+    r[i["nact"]:] = 0.0
+    rhs = np.random.default_rng(6).standard_normal(i["ndof"])  # Dirichlet values among it
+    sp = pm.solver_params(**dict(dict(omega=0.5, pre=3, post=3, rel_tol=1e-10, restart=7), **kw))
+    (z1, x1, s1), (z0, x0, s0) = both(monkeypatch, lambda: (P.vcycle(sp, r), *P.solve(sp, rhs=rhs, check=False)))
+    print(f"[gpu] fp64 lattice order={order} m={m} levels={levels} {kw}: cycle {rel(z1, z0):.1e}, its {s1.iterations} / "
+          f"{s0.iterations}, solution {rel(x1, x0):.1e}", flush=True)
+    assert rel(z1, z0) < CYCLE_TOL
+    assert (s1.iterations, s1.status) == (s0.iterations, s0.status)
+    assert rel(x1, x0) < SOL_TOL and np.array_equal(x1[i["nact"]:], rhs[i["nact"]:])
+    # a solve after it that keeps the CSR form (entries set by the caller) finds nothing of the lattice vectors
+    P.set_entries(levels - 1, P.csr(levels - 1)[2])
+    monkeypatch.setenv("CD3D_FP64_LATTICE", "1")
+    x2, s2 = P.solve(sp, rhs=rhs, check=False)
+    assert np.array_equal(x2, x0) and s2.iterations == s0.iterations
+    P.close()
+
+
+@pytest.mark.parametrize("order,m,k0,levels,theta", [(1, 2, 1, 2, 0.5), (1, 3, 0, 4, 1.0), (2, 2, 0, 3, 0.5), (2, 3, 1, 3, 0.7)])
+def test_fp64_lattice_time_steps_match_csr(order, m, k0, levels, theta, monkeypatch):
+    P = pm.Problem(order, m, k0, levels, box=(1.0, 1.0, 1.0))
+    co = pm.coeffs(eps=1e-3, conv_kind=1, rot_c=(0.45, 0.55), pulse_c=(0.3, 0.5, 0.5), f_val=0.7)
+    sp = pm.solver_params(omega=0.5, pre=3, post=3, rel_tol=1e-10)
+    u0 = P.interp_pulse(levels - 1, co)
+
+    def steps():
+        P.tcd_init(co, 0.1, u0)
+        out = [P.tcd_step(co, sp, 2e-3, theta=theta) for _ in range(3)]
+        return out[-1][0], [st.iterations for _, st in out]
+
+    (u1, i1), (u0_, i0) = both(monkeypatch, steps)
+    print(f"[gpu] fp64 lattice steps order={order}: its {i1} / {i0}, state {rel(u1, u0_):.1e}", flush=True)
+    assert i1 == i0 and rel(u1, u0_) < SOL_TOL
+    P.close()
+
+
+def test_fp64_lattice_rotating_field_solve(monkeypatch):
+    P = pm.Problem(1, 3, 0, 4, box=(1.0, 1.0, 1.0))
+    P.assemble(pm.coeffs(eps=0.05, conv_kind=1, rot_c=(0.45, 0.55), f_val=1.0))
+    sp = pm.solver_params(omega=0.5, pre=3, post=3, rel_tol=1e-10)
+    (x1, s1), (x0, s0) = both(monkeypatch, lambda: P.solve(sp))
+    assert s1.iterations == s0.iterations and rel(x1, x0) < SOL_TOL
+    P.close()
