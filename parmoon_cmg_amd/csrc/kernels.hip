@@ -1358,229 +1358,355 @@ __global__ __launch_bounds__(kBlock) void gj_step_k(int na, int k, double *__res
   }
 }
 
-// dval: the pivot values (blocked form), else M[perm[k]][k]
 __global__ __launch_bounds__(kBlock) void gj_final_k(int na, const double *__restrict__ M,
-                                                     const int *__restrict__ perm, const double *__restrict__ dval,
-                                                     double *__restrict__ inv) {
+                                                     const int *__restrict__ perm, double *__restrict__ inv) {
   const int w2 = 2 * na, wave = blockIdx.x * kGjWaves + (threadIdx.x >> 6), lane = threadIdx.x & 63;
   for (int k = wave; k < na; k += gridDim.x * kGjWaves) {
     const double *row = M + (int64_t)perm[k] * w2;
-    const double d = 1.0 / (dval ? dval[k] : row[k]);
+    const double d = 1.0 / row[k];
     for (int j = lane; j < na; j += 64) inv[(int64_t)k * na + j] = row[na + j] * d;
   }
 }
 
-// Small coarse blocks (na <= kGjLdsMax): the whole in-place Gauss-Jordan
-// inversion in one workgroup with the matrix in LDS.  Partial pivoting with
-// row interchanges (the largest |a_ik| for i >= k, ties to the lower row);
-// the interchanges are undone as column interchanges in reverse order at the
-// end.  One launch instead of na + 2.
-constexpr int kGjLdsMax = 128;
-
-__global__ __launch_bounds__(1024) void gj_lds_k(int na, const int *__restrict__ rp, const int *__restrict__ col,
-                                                 const double *__restrict__ val, double *__restrict__ inv) {
-  extern __shared__ double A[];  // na x na, row-major
-  __shared__ double fcol[kGjLdsMax];
-  __shared__ int ipiv[kGjLdsMax];
-  __shared__ int pivrow;
-  const int t = threadIdx.x, nt = blockDim.x, nn = na * na;
-  for (int i = t; i < nn; i += nt) A[i] = 0.0;
-  __syncthreads();
-  for (int r = t; r < na; r += nt)
-    for (int q = rp[r]; q < rp[r + 1]; q++)
-      if (col[q] < na) A[r * na + col[q]] = val[q];
-  __syncthreads();
-  for (int k = 0; k < na; k++) {
-    if (t < 64) {  // pivot search by the first wavefront
-      double best = -1.0;
-      int bi = k;
-      for (int i = k + t; i < na; i += 64) {
-        const double v = gj_score(A[i * na + k]);
-        if (v > best || (v == best && i < bi)) { best = v; bi = i; }
-      }
-#pragma unroll
-      for (int o = 32; o > 0; o >>= 1) {
-        const double v = __shfl_xor(best, o);
-        const int r = __shfl_xor(bi, o);
-        if (v > best || (v == best && r < bi)) { best = v; bi = r; }
-      }
-      if (t == 0) {
-        pivrow = bi;
-        ipiv[k] = bi;
-      }
-    }
-    __syncthreads();
-    const int p = pivrow;
-    if (p != k)
-      for (int j = t; j < na; j += nt) {
-        const double a = A[k * na + j];
-        A[k * na + j] = A[p * na + j];
-        A[p * na + j] = a;
-      }
-    __syncthreads();
-    const double dinv = 1.0 / A[k * na + k];
-    for (int j = t; j < na; j += nt) {
-      if (j != k) A[k * na + j] *= dinv;
-      fcol[j] = A[j * na + k];  // column k before the elimination
-    }
-    __syncthreads();
-    if (t == 0) A[k * na + k] = dinv;
-    for (int e = t; e < nn; e += nt) {
-      const int i = e / na, j = e % na;
-      if (i == k) continue;
-      if (j == k) A[e] = -fcol[i] * dinv;
-      else A[e] -= fcol[i] * A[k * na + j];
-    }
-    __syncthreads();
-  }
-  for (int k = na - 1; k >= 0; k--) {
-    const int p = ipiv[k];
-    if (p != k)
-      for (int i = t; i < na; i += nt) {
-        const double a = A[i * na + k];
-        A[i * na + k] = A[i * na + p];
-        A[i * na + p] = a;
-      }
-    __syncthreads();
-  }
-  for (int i = t; i < nn; i += nt) inv[i] = A[i];
+// |x| as an integer pivot key: the high word of the double (exponent and 20
+// mantissa bits) plus one, so that the pivot is within 2^-20 of the largest
+// candidate, and the maximum over lanes is integer DPP instead of FP64
+// compares; 0: not a candidate.  A NaN keys like zero: some unused row is
+// always chosen and the pivot index stays in range.
+__device__ inline unsigned gj_key(double x) {
+  const unsigned h = (unsigned)__double2hiint(x) & 0x7fffffffu;
+  return h > 0x7ff00000u ? 1u : h + 1u;
+}
+// maximum over each row of 16 lanes (row_ror:8, 4, 2, 1), and over the wave
+// (uniform); every lane takes part
+template <int CTRL>
+__device__ inline unsigned dpp_max(unsigned v) {
+  const unsigned o = (unsigned)__builtin_amdgcn_update_dpp((int)v, (int)v, CTRL, 0xf, 0xf, false);
+  return v > o ? v : o;
+}
+__device__ inline unsigned row16_max(unsigned v) {
+  return dpp_max<0x121>(dpp_max<0x122>(dpp_max<0x124>(dpp_max<0x128>(v))));
+}
+__device__ inline unsigned wave_max(unsigned v) {
+  v = row16_max(v);
+  const unsigned a = (unsigned)__builtin_amdgcn_readlane((int)v, 0), b = (unsigned)__builtin_amdgcn_readlane((int)v, 16),
+                 c = (unsigned)__builtin_amdgcn_readlane((int)v, 32), d = (unsigned)__builtin_amdgcn_readlane((int)v, 48);
+  const unsigned ab = a > b ? a : b, cd = c > d ? c : d;
+  return ab > cd ? ab : cd;
+}
+__device__ inline double lane_f64(double v, int lane) {
+  return __hiloint2double(__builtin_amdgcn_readlane(__double2hiint(v), lane),
+                          __builtin_amdgcn_readlane(__double2loint(v), lane));
 }
 
-// Blocked form of the same elimination for kGjLdsMax < na <= kGjBlockedMax:
-// the same pivots (largest unused |m_rk|, ties to the lower row), the same
-// multipliers and the same extraction, reorganised by panels of NB pivot
-// columns.  The panel kernel (one workgroup; each thread holds RPT rows of the
-// panel in registers) finds the NB pivots of the panel and every row's
-// multipliers W[r][j] (0 for the pivot row of step j).  The update kernel then
-// applies their combined effect to the columns right of the panel as one
-// rank-NB update,
-//   U_j  = M[p_j] - sum_{i<j} W[p_j][i] U_i   (pivot row p_j as it was at step j)
-//   M'[r] = M[r] - sum_j W[r][j] U_j           (every row r),
-// reading M and writing M' (two buffers, so that the U rows are formed from
-// the old values while M' is written).  The pivot values go to dval[k].  Two
-// launches per panel instead of NB.
-constexpr int kGjPanel = 16;        // stride of the multiplier rows W
-constexpr int kGjBlockedMax = 4096;  // 4 rows per thread of the panel kernel
-constexpr int kGjUpdRows = 16;      // rows per workgroup of the update kernel
-
-template <int NB, int RPT>
-__global__ __launch_bounds__(1024) void gj_panel_k(int na, int k0, int b, const double *__restrict__ M,
-                                                   int *__restrict__ used, int *__restrict__ perm,
-                                                   double *__restrict__ dval, double *__restrict__ W) {
-  __shared__ double sv[2][16];
-  __shared__ int si[2][16];
-  __shared__ double srow[2][16][NB];  // each wave's candidate row, double-buffered by step
-  const int w2 = 2 * na, t = threadIdx.x, lane = t & 63, wv = t >> 6;
-  double v[RPT][NB];
-  bool un[RPT];
-  int pj[RPT];
+// Explicit inverse by Gauss-Jordan exchange steps in place: y = A x is solved
+// step by step for x_k through the row p with the largest unused |t_pk| (ties
+// to the lower row in its wave),
+//   t_pk' = 1/t_pk, t_pj' = -t_pj / t_pk, t_ik' = t_ik / t_pk,
+//   t_ij' = t_ij - (t_ik / t_pk) t_pj,
+// so that after na steps row p_k holds x_k and column k belongs to y_{p_k}:
+// inv[k][p_c] = t[p_k][c].  No rows are interchanged and no second na x na
+// block is carried.
+//
+// Small blocks (na <= TS TL): one workgroup of TS x TS threads, each holding
+// the entries (ty + TS a, tx + TS b), a, b < TL, in registers.  Two barriers
+// per pivot: the column goes to LDS, every wave finds the pivot for itself,
+// the pivot row goes to LDS.  Bound by that chain and by the instructions a
+// wave issues per pivot (1.3 us), so few waves with large tiles: 125 unknowns
+// 168 us with 4 waves of 8 x 8 tiles (16 waves of 4 x 4: 288 us; the matrix in
+// LDS with five barriers per pivot: 607 us); 27 unknowns 50 -> 31 us.
+constexpr int kGjSmallMax = 128;
+template <int TS, int TL>
+__global__ __launch_bounds__(TS *TS) void gj_small_k(int na, const int *__restrict__ rp, const int *__restrict__ col,
+                                                     const double *__restrict__ val, double *__restrict__ inv) {
+  constexpr int N = TS * TL, NT = TS * TS;
+  __shared__ double cs[2][N], rs[2][N];
+  __shared__ int perm[N], iperm[N];
+  const int t = threadIdx.x, tx = t % TS, ty = t / TS, lane = t & 63;
+  const int wv = __builtin_amdgcn_readfirstlane(t >> 6);
+  // the dense matrix is spread out in inv first
+  for (int i = t; i < na * na; i += NT) inv[i] = 0.0;
+  __syncthreads();
+  for (int r = wv; r < na; r += NT / 64)
+    for (int q = rp[r] + lane; q < rp[r + 1]; q += 64)
+      if (col[q] < na) inv[r * na + col[q]] = val[q];
+  __syncthreads();
+  // v[b][a]: row ty + TS a, column tx + TS b (vectors over a: the pivot row's
+  // place is read and written by a dynamic register index)
+  typedef double Col __attribute__((ext_vector_type(TL)));
+  Col v[TL];
 #pragma unroll
-  for (int q = 0; q < RPT; q++) {
-    const int r = t + q * 1024;
-    pj[q] = -1;
-    un[q] = r < na && !used[r];
+  for (int b = 0; b < TL; b++)
 #pragma unroll
-    for (int j = 0; j < NB; j++) v[q][j] = (r < na && j < b) ? M[(int64_t)r * w2 + k0 + j] : 0.0;
-  }
-  // the wave's best unused row for column j; its owner lane stages the row
-  auto propose = [&](const int j, const int buf) {
-    double bv = -1.0;
-    int bi = 1 << 30;
-#pragma unroll
-    for (int q = 0; q < RPT; q++)
-      if (un[q]) gj_better(bv, bi, gj_score(v[q][j]), t + q * 1024);
-#pragma unroll
-    for (int o = 32; o > 0; o >>= 1) {
-      const double ov = __shfl_xor(bv, o);
-      const int oi = __shfl_xor(bi, o);
-      gj_better(bv, bi, ov, oi);
+    for (int a = 0; a < TL; a++) {
+      const int r = ty + TS * a, c = tx + TS * b;
+      v[b][a] = r < na && c < na ? inv[min(r, na - 1) * na + min(c, na - 1)] : 0.0;
     }
+  // rows lane and lane + 64, kept by every wave
+  bool u0 = lane < na, u1 = N > 64 && lane + 64 < na;
+  const int l0 = lane < N ? lane : 0, l1 = N > 64 ? lane + 64 : 0;
+  // the tile column of the pivot is a constant of the unrolled outer loop
+  // (branches per register cost more than the arithmetic of a step)
 #pragma unroll
-    for (int q = 0; q < RPT; q++)
-      if (un[q] && t + q * 1024 == bi) {
+  for (int kb = 0; kb < TL; kb++)
+#pragma unroll 1
+    for (int kc = 0; kc < TS; kc++) {
+      const int k = kb * TS + kc, buf = k & 1;
+      if (k >= na) break;
+      if (tx == kc)
 #pragma unroll
-        for (int jj = j; jj < NB; jj++) srow[buf][wv][jj] = v[q][jj];
-      }
-    if (lane == 0) {
-      sv[buf][wv] = bv;
-      si[buf][wv] = bi;
-    }
-  };
-  const int nw = blockDim.x >> 6;
-  propose(0, 0);
-#pragma unroll
-  for (int j = 0; j < NB; j++) {
-    if (j < b) {
-      const int buf = j & 1;
+        for (int a = 0; a < TL; a++) cs[buf][ty + TS * a] = v[kb][a];
       __syncthreads();
-      double gv = lane < nw ? sv[buf][lane] : -2.0;
-      int gi = lane < nw ? si[buf][lane] : (1 << 30), gs = lane;
+      const double x0 = cs[buf][l0], x1 = cs[buf][l1];
+      double cf[TL];
 #pragma unroll
-      for (int o = 8; o > 0; o >>= 1) {
-        const double ov = __shfl_xor(gv, o);
-        const int oi = __shfl_xor(gi, o), os = __shfl_xor(gs, o);
-        if (ov > gv || (ov == gv && oi < gi)) { gv = ov; gi = oi; gs = os; }
+      for (int a = 0; a < TL; a++) cf[a] = cs[buf][ty + TS * a];
+      const unsigned s0 = u0 ? gj_key(x0) : 0u, s1 = u1 ? gj_key(x1) : 0u;
+      const unsigned best = wave_max(s0 > s1 ? s0 : s1);
+      const unsigned long long m0 = __ballot(s0 == best), m1 = __ballot(s1 == best);
+      const int p0 = __ffsll(m0) - 1, p1 = __ffsll(m1) + 63;
+      const unsigned p = (unsigned)__builtin_amdgcn_readfirstlane(m0 ? p0 : p1);
+      u0 = u0 && lane != (int)p;
+      u1 = u1 && lane + 64 != (int)p;
+      const unsigned pa = p / TS, pr = p % TS;
+      const bool mine = pr / (64 / TS) == (unsigned)wv;  // the wave holds row p (64 / TS rows per wave)
+      if (mine) {
+        double row[TL];
+#pragma unroll
+        for (int b = 0; b < TL; b++) row[b] = v[b][pa];
+        if (ty == (int)pr)
+#pragma unroll
+          for (int b = 0; b < TL; b++) rs[buf][tx + TS * b] = row[b];
       }
-      const int p = __shfl(gi, 0), ps = __shfl(gs, 0);
-      const double d = srow[buf][ps][j];
+      const double dinv = 1.0 / lane_f64(p < 64 ? x0 : x1, p & 63);
       if (t == 0) {
-        perm[k0 + j] = p;
-        used[p] = 1;
-        dval[k0 + j] = d;
+        perm[k] = p;
+        iperm[p] = k;
       }
 #pragma unroll
-      for (int q = 0; q < RPT; q++) {
-        const int r = t + q * 1024;
-        if (r == p) {
-          un[q] = false;
-          pj[q] = j;
-        } else if (r < na) {
-          const double f = v[q][j] / d;
-          if (f != 0.0)
+      for (int a = 0; a < TL; a++) cf[a] *= dinv;
+      __syncthreads();
 #pragma unroll
-            for (int jj = j + 1; jj < NB; jj++) v[q][jj] -= f * srow[buf][ps][jj];
-          v[q][j] = f;
+      for (int b = 0; b < TL; b++) {
+        const double g = rs[buf][tx + TS * b];
+#pragma unroll
+        for (int a = 0; a < TL; a++) v[b][a] = fma(-cf[a], g, v[b][a]);
+        if (b == kb)
+#pragma unroll
+          for (int a = 0; a < TL; a++) v[b][a] = tx == kc ? cf[a] : v[b][a];
+        // row p: -g / d, and 1 / d at the pivot
+        if (mine) {
+          const double old = v[b][pa], w = b == kb && tx == kc ? dinv : -g * dinv;
+          v[b][pa] = ty == (int)pr ? w : old;
         }
       }
-      if (j + 1 < b) propose(j + 1, buf ^ 1);
     }
-  }
+  __syncthreads();
 #pragma unroll
-  for (int q = 0; q < RPT; q++) {
-    const int r = t + q * 1024;
-    if (r < na)
+  for (int a = 0; a < TL; a++)
 #pragma unroll
-      for (int j = 0; j < NB; j++) W[(int64_t)r * kGjPanel + j] = (j < b && j != pj[q]) ? v[q][j] : 0.0;
+    for (int b = 0; b < TL; b++) {
+      const int r = ty + TS * a, c = tx + TS * b;
+      if (r < na && c < na) inv[iperm[r] * na + perm[c]] = v[b][a];
+    }
+}
+
+// Larger blocks (up to kGjBlockedMax): panels of NB columns, one launch per
+// panel.  Workgroup 0 brings panel s up to date with panel s - 1 (rank-NB, as
+// below) and runs its NB exchange steps on the panel's columns alone, RPT rows
+// per thread in registers: the result W (column-major, NB x na) is at once the
+// panel's new columns and the multipliers of every other column c,
+//   t_rc' = (r a pivot row of the panel ? 0 : t_rc) - sum_j W_rj t_{p_j c}.
+// The other workgroups of the launch apply panel s - 1 to all other columns,
+// from one buffer into the other (a wave takes 64 columns of kGjUpdRows rows:
+// its pivot-row entries stay in registers, W is read as scalars), so the
+// factorisation of a panel, a serial chain of NB pivots in one workgroup, runs
+// beside the update by the one before.  They write panel s + 1's columns to
+// the compact column-major buffer C, which workgroup 0 of the next launch
+// reads with consecutive lanes on consecutive rows (read from the row-major
+// matrix, each lane on its own cache line, a 2197-row panel took 12 us to load
+// and 12 us to bring up to date).  The last launch writes the inverse itself.
+// Bound by the chain of pivots and the launches; per pivot: column keys (DPP
+// maximum), the wave's candidate row to LDS, one barrier, the best candidate.
+// Whole inversion, with separate panel and update launches over na x 2 na
+// before: 343 unknowns 900 -> 509 us, 1331 7.7 -> 4.0 ms, 2197 19.2 -> 10.2 ms
+// (256-thread workgroups with more rows per thread: 17.7 ms).
+constexpr int kGjPanel = 16;        // widest panel
+constexpr int kGjBlockedMax = 4096;  // 4 rows per thread of the panel
+constexpr int kGjUpdRows = 8;        // rows per wave of the update
+
+__global__ __launch_bounds__(kBlock) void gj_dense_k(int na, const int *__restrict__ rp, const int *__restrict__ col,
+                                                     const double *__restrict__ val, double *__restrict__ M,
+                                                     int *__restrict__ iperm) {
+  const int wave = blockIdx.x * kGjWaves + (threadIdx.x >> 6), lane = threadIdx.x & 63;
+  for (int r = wave; r < na; r += gridDim.x * kGjWaves) {
+    for (int j = lane; j < na; j += 64) M[(int64_t)r * na + j] = 0.0;
+    __threadfence_block();  // the zeros land before the entries below
+    for (int t = rp[r] + lane; t < rp[r + 1]; t += 64)
+      if (col[t] < na) M[(int64_t)r * na + col[t]] = val[t];
+    if (lane == 0) iperm[r] = -1;
   }
 }
 
-// rank-NB update of the columns right of the panel; a workgroup forms U for
-// its 64 columns (each wave its own copy, in registers) and updates
-// kGjUpdRows rows of them
-template <int NB>
-__global__ __launch_bounds__(256) void gj_update_k(int na, int k0, int b, const double *__restrict__ Min,
-                                                   double *__restrict__ Mout, const int *__restrict__ perm,
-                                                   const double *__restrict__ W) {
-  const int w2 = 2 * na, c = k0 + b + blockIdx.x * 64 + (threadIdx.x & 63), wv = threadIdx.x >> 6;
-  if (c >= w2) return;
-  double u[NB];
+// kp, bp: the panel to apply (bp 0: none); k0, b: the panel to factor (b 0:
+// none, the result goes to inv).  perm[k]: pivot row of column k; iperm[r]:
+// column of pivot row r or -1.  (The update looks at iperm for panel kp while
+// workgroup 0 sets entries of panel k0: those rows are -1 or >= k0, not of
+// panel kp either way.)  C: the columns of panel k0 or null (then read from
+// M); Cn: receives those of the panel after it.  Wp, iperm are read up to
+// kGjUpdRows entries past their end (scratch).
+template <int NB, int RPT>
+__global__ __launch_bounds__(1024) void gj_block_k(int na, int kp, int bp, int k0, int b, const double *__restrict__ M,
+                                                   double *__restrict__ Mo, const double *__restrict__ Wp,
+                                                   double *__restrict__ W, const double *__restrict__ C,
+                                                   double *__restrict__ Cn, int *perm, int *iperm,
+                                                   double *__restrict__ inv, int ncb) {
+  const int t = threadIdx.x, lane = t & 63, wv = __builtin_amdgcn_readfirstlane(t >> 6), nw = blockDim.x >> 6;
+  if (blockIdx.x > 0 || b == 0) {
+    const int blk = (int)blockIdx.x - (b ? 1 : 0), cb = blk % ncb, rb = blk / ncb;
+    const int c = cb * 64 + lane, r0 = (rb * nw + wv) * kGjUpdRows;
+    if (c >= na || r0 >= na || (c >= k0 && c < k0 + b)) return;
+    const bool own = c >= kp && c < kp + bp;  // a column of the applied panel: its new values are W
+    const int cn = c - (k0 + NB);             // a column of the next panel: 0 <= cn < NB
+    const int oc = b ? c : perm[c];
+    double u[NB], m[kGjUpdRows];
+    int ir[kGjUpdRows];
 #pragma unroll
-  for (int j = 0; j < NB; j++) {
-    u[j] = 0.0;
-    if (j < b) {
-      const int p = perm[k0 + j];
-      double s = Min[(int64_t)p * w2 + c];
+    for (int j = 0; j < NB; j++) u[j] = j < bp ? M[(int64_t)perm[kp + j] * na + c] : 0.0;
 #pragma unroll
-      for (int i = 0; i < j; i++) s -= W[(int64_t)p * kGjPanel + i] * u[i];
-      u[j] = s;
+    for (int i = 0; i < kGjUpdRows; i++) {
+      m[i] = M[(int64_t)min(r0 + i, na - 1) * na + c];
+      ir[i] = iperm[r0 + i];
+    }
+#pragma unroll
+    for (int i = 0; i < kGjUpdRows; i++) m[i] = ir[i] >= kp && ir[i] < kp + bp ? 0.0 : m[i];
+#pragma unroll
+    for (int j = 0; j < NB; j++) {
+      const double *w = Wp + (int64_t)j * na + r0;  // uniform: scalar loads
+#pragma unroll
+      for (int i = 0; i < kGjUpdRows; i++) m[i] = fma(-w[i], u[j], m[i]);
+    }
+#pragma unroll
+    for (int i = 0; i < kGjUpdRows; i++) {
+      const int r = r0 + i;
+      if (r >= na) break;
+      const double s = own ? Wp[(int64_t)(c - kp) * na + r] : m[i];
+      if (b == 0) inv[(int64_t)ir[i] * na + oc] = s;
+      else if (cn >= 0 && cn < NB) Cn[(int64_t)cn * na + r] = s;
+      else Mo[(int64_t)r * na + c] = s;
+    }
+    return;
+  }
+  __shared__ double srow[2][16][NB + 1], us[NB][NB];
+  __shared__ unsigned sk[2][16];
+  __shared__ int si[2][16], sp[NB];
+  double v[RPT][NB];
+  bool un[RPT];
+#pragma unroll
+  for (int q = 0; q < RPT; q++) {
+    const int r = t + q * (int)blockDim.x, ir = r < na ? iperm[r] : 0;
+    un[q] = r < na && ir < 0;
+    const bool pr = r >= na || (ir >= kp && ir < kp + bp);
+#pragma unroll
+    for (int j = 0; j < NB; j++)
+      v[q][j] = pr || j >= b ? 0.0 : C ? C[(int64_t)j * na + r] : M[(int64_t)r * na + k0 + j];
+  }
+  if (bp) {
+    // the applied panel's pivot rows at the new panel's columns
+    for (int e = t; e < NB * NB; e += blockDim.x) {
+      const int i = e / NB, j = e % NB, p = i < bp ? perm[kp + i] : 0;
+      us[i][j] = i >= bp || j >= b ? 0.0 : C ? C[(int64_t)j * na + p] : M[(int64_t)p * na + k0 + j];
+    }
+    __syncthreads();
+#pragma unroll 2
+    for (int i = 0; i < NB; i++) {
+      double w[RPT];
+#pragma unroll
+      for (int q = 0; q < RPT; q++) {
+        const int r = t + q * (int)blockDim.x;
+        w[q] = r < na ? Wp[(int64_t)i * na + r] : 0.0;
+      }
+#pragma unroll
+      for (int j = 0; j < NB; j++) {
+        const double uj = us[i][j];
+#pragma unroll
+        for (int q = 0; q < RPT; q++) v[q][j] = fma(-w[q], uj, v[q][j]);
+      }
     }
   }
-  const int r1 = min(na, (int)(blockIdx.y + 1) * kGjUpdRows);
-  for (int r = blockIdx.y * kGjUpdRows + wv; r < r1; r += 4) {
-    double s = 0.0;
+  // The pivot column is always column 0: every step moves the columns one
+  // place down and the finished one to the end, so the loop stays rolled with
+  // its columns in registers.
+#pragma unroll 1
+  for (int j = 0; j < b; j++) {
+    const int buf = j & 1;
+    // the wave's best unused row of the column; its lane stages the row
+    unsigned key = 0;
+    int bq = 0;
+    double bx = 1.0;
 #pragma unroll
-    for (int j = 0; j < NB; j++) s += W[(int64_t)r * kGjPanel + j] * u[j];
-    Mout[(int64_t)r * w2 + c] = Min[(int64_t)r * w2 + c] - s;
+    for (int q = 0; q < RPT; q++) {
+      const unsigned kq = un[q] ? gj_key(v[q][0]) : 0u;
+      if (q == 0 || kq > key) {
+        key = kq;
+        bq = q;
+        bx = v[q][0];
+      }
+    }
+    const double bi = 1.0 / bx;  // beside the search
+    const unsigned wb = wave_max(key);
+    const int wl = __ffsll(__ballot(key == wb)) - 1;
+    if (lane == wl) {
+      sk[buf][wv] = wb;
+      si[buf][wv] = t + bq * (int)blockDim.x;
+      srow[buf][wv][NB] = bi;
+#pragma unroll
+      for (int q = 0; q < RPT; q++)
+        if (q == bq)
+#pragma unroll
+          for (int jj = 0; jj < NB; jj++) srow[buf][wv][jj] = v[q][jj];
+    }
+    __syncthreads();
+    const unsigned gk = lane < nw ? sk[buf][lane] : 0u;
+    const unsigned gb = (unsigned)__builtin_amdgcn_readlane((int)row16_max(gk), 0);  // nw <= 16: the first row of lanes
+    const int ps = __ffsll(__ballot(gk == gb)) - 1;
+    const double *g = srow[buf][ps];
+    const int p = si[buf][ps];
+    const double dinv = g[NB];
+    if (t == 0) sp[j] = p;  // (a global store here would be waited for at the next barrier)
+    double f[RPT];
+#pragma unroll
+    for (int q = 0; q < RPT; q++) {
+      // row p: t_pj' = -g_j / d, the others t_ij - f g_j
+      const bool pr = t + q * (int)blockDim.x == p;
+      f[q] = pr ? dinv : v[q][0] * dinv;
+      if (pr) {
+        un[q] = false;
+#pragma unroll
+        for (int jj = 1; jj < NB; jj++) v[q][jj] = 0.0;
+      }
+    }
+#pragma unroll
+    for (int jj = 1; jj < NB; jj++) {
+      const double gj = g[jj];
+#pragma unroll
+      for (int q = 0; q < RPT; q++) v[q][jj - 1] = fma(-f[q], gj, v[q][jj]);
+    }
+#pragma unroll
+    for (int q = 0; q < RPT; q++) v[q][NB - 1] = f[q];
+  }
+  __syncthreads();
+  if (t < b) {
+    perm[k0 + t] = sp[t];
+    iperm[sp[t]] = k0 + t;
+  }
+  // column j of the panel now sits at (j - b) mod NB
+#pragma unroll
+  for (int q = 0; q < RPT; q++) {
+    const int r = t + q * (int)blockDim.x;
+    if (r < na)
+#pragma unroll
+      for (int j = 0; j < NB; j++) W[(int64_t)((j + b) & (NB - 1)) * na + r] = v[q][j];
   }
 }
 
@@ -1956,19 +2082,32 @@ void k_hconv_geo(hipStream_t s, const DevLevel &L, const double *tab, const AsmP
   else hconv_geo_k<2><<<grid, kBlock, 0, s>>>(L.ncell, L.cells, tab, ap, hconv);
 }
 
-// blocked elimination (panels of NB pivots); returns the buffer holding the result
+// blocked elimination in panels of NB pivots (gj_block_k); M, M1: na x na
+// each; W, W1, C, C1: kGjPanel x na each
 template <int NB, int RPT>
-const double *gj_blocked(hipStream_t s, int na, double *M, double *M1, int *used, int *perm, double *dval,
-                         double *W) {
-  double *Mi = M, *Mo = M1;
-  for (int k0 = 0; k0 < na; k0 += NB) {
-    const int b = std::min(NB, na - k0), ncol = 2 * na - k0 - b;  // ncol >= na > 0
-    gj_panel_k<NB, RPT><<<1, RPT == 1 ? (na + 63) / 64 * 64 : 1024, 0, s>>>(na, k0, b, Mi, used, perm, dval, W);
-    const dim3 grid((ncol + 63) / 64, (na + kGjUpdRows - 1) / kGjUpdRows);
-    gj_update_k<NB><<<grid, 256, 0, s>>>(na, k0, b, Mi, Mo, perm, W);
-    std::swap(Mi, Mo);
+void gj_blocked(hipStream_t s, int na, double *M, double *M1, double *W, double *W1, double *C, double *C1, int *perm,
+                int *iperm, double *inv) {
+  const int bd = RPT == 1 ? (na + 63) / 64 * 64 : 1024, ncb = (na + 63) / 64;
+  const int nrb = (na + bd / 64 * kGjUpdRows - 1) / (bd / 64 * kGjUpdRows), upd = ncb * nrb;
+  const double *Mi = M;
+  double *Mo = M1, *Wi = W1, *Wo = W, *Ci = C1, *Co = C;
+  int kp = 0, bp = 0, step = 0;
+  for (int k0 = 0; k0 < na; k0 += NB, step++) {
+    const int b = std::min(NB, na - k0);
+    // the first two panels are still unchanged in M
+    gj_block_k<NB, RPT><<<bp ? 1 + upd : 1, bd, 0, s>>>(na, kp, bp, k0, b, Mi, Mo, Wi, Wo, step > 1 ? Ci : nullptr, Co,
+                                                        perm, iperm, inv, ncb);
+    if (bp) {
+      double *o = Mo;
+      Mo = o == M1 ? M : M1;
+      Mi = o;
+    }
+    std::swap(Wi, Wo);
+    std::swap(Ci, Co);
+    kp = k0;
+    bp = b;
   }
-  return Mi;
+  gj_block_k<NB, RPT><<<upd, bd, 0, s>>>(na, kp, bp, na, 0, Mi, Mo, Wi, Wo, nullptr, nullptr, perm, iperm, inv, ncb);
 }
 
 // CD3D_GJ_UNBLOCKED=1: one launch per pivot also for large blocks (comparison runs)
@@ -1981,64 +2120,46 @@ static bool gj_unblocked() {
 }
 
 void k_invert_active(hipStream_t s, const DevLevel &L, double *scratch, double *inv) {
-  // scratch layout: M, M' (2 na^2 doubles each), W (kGjPanel na), dval[na],
-  // two partial (value, index) buffers, used[na], perm[na]
   const int na = L.nact;
   if (na <= 0) return;
-  if (na <= kGjLdsMax) {
-    // the larger-than-64 KiB LDS opt-in, once per device; the serving loop's
-    // worker threads reach this concurrently
-    static std::mutex lds_mu;
-    static int lds_ok[64];
-    static bool lds_init = false;
-    int dev = 0;
-    (void)hipGetDevice(&dev);
-    bool ok;
-    {
-      std::lock_guard<std::mutex> g(lds_mu);
-      if (!lds_init) {
-        for (int &v : lds_ok) v = -1;
-        lds_init = true;
-      }
-      int &st = lds_ok[dev & 63];
-      if (st < 0)
-        st = hipFuncSetAttribute((const void *)gj_lds_k, hipFuncAttributeMaxDynamicSharedMemorySize,
-                                 (int)(sizeof(double) * kGjLdsMax * kGjLdsMax)) == hipSuccess;
-      ok = st != 0;
-    }
-    const size_t bytes = sizeof(double) * na * na;
-    if (ok || bytes <= 65536) {
-      gj_lds_k<<<1, 1024, bytes, s>>>(na, L.rowptr, L.col, L.val, inv);
-      return;
-    }
-    (void)hipGetLastError();
-  }
-  const int nblk = std::min((na + kGjWaves - 1) / kGjWaves, 256);
-  double *M = scratch, *M1 = M + (int64_t)2 * na * na, *W = M1 + (int64_t)2 * na * na, *dval = W + (int64_t)kGjPanel * na;
-  double *pv0 = dval + na, *pv1 = pv0 + 256;
-  int *pi0 = (int *)(pv1 + 256), *pi1 = pi0 + 256, *used = pi1 + 256, *perm = used + na;
-  gj_init_k<<<nblk, kBlock, 0, s>>>(na, L.rowptr, L.col, L.val, M, used, pv0, pi0);
-  if (na <= kGjBlockedMax && !gj_unblocked()) {
-    const int rpt = (na + 1023) / 1024;
-    const double *Mf = rpt == 1   ? gj_blocked<16, 1>(s, na, M, M1, used, perm, dval, W)
-                       : rpt == 2 ? gj_blocked<8, 2>(s, na, M, M1, used, perm, dval, W)
-                       : rpt == 3 ? gj_blocked<8, 3>(s, na, M, M1, used, perm, dval, W)
-                                  : gj_blocked<8, 4>(s, na, M, M1, used, perm, dval, W);
-    gj_final_k<<<nblk, kBlock, 0, s>>>(na, Mf, perm, dval, inv);
+  if (na <= kGjSmallMax) {
+    if (na <= 32) gj_small_k<8, 4><<<1, 64, 0, s>>>(na, L.rowptr, L.col, L.val, inv);
+    else if (na <= 64) gj_small_k<8, 8><<<1, 64, 0, s>>>(na, L.rowptr, L.col, L.val, inv);
+    else gj_small_k<16, 8><<<1, 256, 0, s>>>(na, L.rowptr, L.col, L.val, inv);
     return;
   }
+  const int nblk = std::min((na + kGjWaves - 1) / kGjWaves, 256);
+  const int64_t na2 = (int64_t)na * na;
+  if (na <= kGjBlockedMax && !gj_unblocked()) {
+    // scratch: M, M' (na^2 doubles each), W, W', C, C' (kGjPanel na each), perm[na], iperm[na], slack
+    const int64_t pn = (int64_t)kGjPanel * na;
+    double *M = scratch, *M1 = M + na2, *W = M1 + na2, *W1 = W + pn, *C = W1 + pn, *C1 = C + pn;
+    int *perm = (int *)(C1 + pn), *iperm = perm + na;
+    gj_dense_k<<<nblk, kBlock, 0, s>>>(na, L.rowptr, L.col, L.val, M, iperm);
+    const int rpt = (na + 1023) / 1024;
+    if (rpt == 1) gj_blocked<16, 1>(s, na, M, M1, W, W1, C, C1, perm, iperm, inv);
+    else if (rpt == 2) gj_blocked<16, 2>(s, na, M, M1, W, W1, C, C1, perm, iperm, inv);
+    else if (rpt == 3) gj_blocked<8, 3>(s, na, M, M1, W, W1, C, C1, perm, iperm, inv);
+    else gj_blocked<8, 4>(s, na, M, M1, W, W1, C, C1, perm, iperm, inv);
+    return;
+  }
+  // scratch: M (2 na^2 doubles), two partial (value, index) buffers, used[na], perm[na]
+  double *M = scratch, *pv0 = M + 2 * na2, *pv1 = pv0 + 256;
+  int *pi0 = (int *)(pv1 + 256), *pi1 = pi0 + 256, *used = pi1 + 256, *perm = used + na;
+  gj_init_k<<<nblk, kBlock, 0, s>>>(na, L.rowptr, L.col, L.val, M, used, pv0, pi0);
   for (int k = 0; k < na; k++) {
     const bool even = (k % 2) == 0;
     gj_step_k<<<nblk, kBlock, 0, s>>>(na, k, M, used, perm, even ? pv0 : pv1, even ? pi0 : pi1, even ? pv1 : pv0,
                                       even ? pi1 : pi0);
   }
-  gj_final_k<<<nblk, kBlock, 0, s>>>(na, M, perm, nullptr, inv);
+  gj_final_k<<<nblk, kBlock, 0, s>>>(na, M, perm, inv);
 }
-bool k_invert_multi_launch(int na) { return na > kGjLdsMax; }
+bool k_invert_multi_launch(int na) { return na > kGjSmallMax; }
 
 int64_t gj_scratch_doubles(int na) {
-  // M and M' (na x 2na each), W (na x kGjPanel), dval, partials, used + perm (ints)
-  return (int64_t)4 * na * na + (int64_t)(kGjPanel + 1) * na + 512 + (512 + 2 * (int64_t)na + 2) / 2 + 1;
+  // both layouts of k_invert_active: 2 na^2, four panels (or the pivot
+  // partials), two int arrays of na and slack
+  return (int64_t)2 * na * na + (int64_t)4 * kGjPanel * na + 512 + (512 + 2 * (int64_t)na + 2) / 2 + 1;
 }
 void k_multi_axpy32(hipStream_t s, int n, int m, const double *coef, const float *Z, int64_t ldz, double *x) {
   multi_axpy32_k<<<grid_for(n), kBlock, 0, s>>>(n, m, coef, Z, ldz, x);
