@@ -604,24 +604,17 @@ static void refresh_f32(cd3d_problem &P, bool values = true) {
 
 namespace {
 
-// Mixed V-cycles: the bottom levels, up to the highest level with at most
-// this many lattice nodes (and at most kSmallMaxLevels of them above an exact
-// coarse solve of at most kSmallCoarseMax unknowns), run as one launch
-// (kl_small_vcycle).  One workgroup pays off only while a level's nodes take
-// about one round of the CU (measured: 4913-node Q2 levels and a 343-unknown
-// coarse solve are several times slower than the launch-per-step form).
-// The node bound is small_nodes_bound().
-constexpr int kSmallMaxLevels = 3, kSmallCoarseMax = 128;
+// Lattice V-cycles: the bottom levels, up to the highest level that the
+// one-workgroup program takes (kl_small_ok: its vectors in LDS, at most
+// small_nodes_bound() nodes) above an exact coarse solve of at most
+// kSmallCoarseMax unknowns, run as one launch (kl_small_vcycle).
+constexpr int kSmallCoarseMax = 128;
 
+template <typename T>
 static int small_top(const cd3d_problem &P, const cd3d_solver_params &sp) {
   if (sp.cycle != 1 || sp.coarse_smoother != 17 || P.dl.empty() || P.dl[0].nact > kSmallCoarseMax) return 0;
   int top = 0;
-  for (int i = 1; i < (int)P.dl.size() && i <= kSmallMaxLevels; i++) {
-    const long long nn = P.dl[i].nn;
-    // the program reads compact or per-node FP32 values (not the node-by-node affine form)
-    if (nn * nn * nn > small_nodes_bound() || P.dl[i].nclass <= 0 || P.dl[i].lat_affine) break;
-    top = i;
-  }
+  while (top + 1 < (int)P.dl.size() && kl_small_ok<T>(P.dl.data(), top + 1, small_nodes_bound())) top++;
   return top;
 }
 
@@ -629,7 +622,7 @@ struct VC {
   cd3d_problem &P;
   const cd3d_solver_params &sp;
   int rec[32];     // mg_recursions (TMultiGrid3D::SetRecursion, MultiGrid3D.C:690-703)
-  int small = -1;  // the level whose zero-start visit runs as one launch (mixed V-cycle; 0: none)
+  int small = -1;  // the level whose zero-start visit runs as one launch (lattice V-cycles; 0: none)
   // mixed V-cycle: bit i set when the restriction into level i also wrote
   // its first pre-smoothing sweep from zero (into lt); CD3D_FUSE_ZERO_SWEEP=0
   // launches that sweep instead
@@ -803,19 +796,17 @@ void cycleL(VC &v, int i, bool zero_start, const T *ftop = nullptr, T *ztop = nu
     coarseL<T>(v, zero_start);
     return;
   }
-  if constexpr (sizeof(T) == 4) {
-    if (v.small < 0) v.small = small_top(P, v.sp);
-    if (zero_start && i == v.small) {
-      coarse_join(P);
-      kl_small_vcycle(P.stream, P.dl.data(), i, P.mesh.order, v.sp.pre, v.sp.post, (float)v.sp.omega,
-                      (float)v.sp.gmg_damp, P.cinv);
-      return;
-    }
-  }
   DevLevel &L = P.dl[i], &C = P.dl[i - 1];
   const int p = P.mesh.order;
   const LatVecs<T> l = lat_vecs<T>(L, i), c = lat_vecs<T>(C, i - 1);
   const T *f = ftop ? ftop : l.f;
+  if (v.small < 0) v.small = small_top<T>(P, v.sp);
+  if (zero_start && i == v.small) {
+    coarse_join(P);
+    kl_small_vcycle<T>(P.stream, P.dl.data(), i, p, v.sp.pre, v.sp.post, (T)v.sp.omega, (T)v.sp.gmg_damp, P.cinv, f,
+                       ztop ? ztop : l.x);
+    return;
+  }
   T *x = l.x, *t = l.t;
   const T om = (T)v.sp.omega;
   const bool ready = zero_start && (v.zero_ready >> i & 1u);

@@ -541,10 +541,15 @@ void kl_cast_f2d(hipStream_t s, int64_t n, const float *a, double *b);
 // DOF-ordered f64 <-> lattice vectors (Dirichlet DOFs map to zero)
 template <typename T>
 void kl_from_dof(hipStream_t s, const DevLevel &L, const double *v, T *l);
-// zero-start mixed V-cycle of levels top..1 and the exact coarse solve in
-// one launch (levels[0..top]; 1 <= top <= 3)
-void kl_small_vcycle(hipStream_t s, const DevLevel *levels, int top, int order, int pre, int post, float omega,
-                     float damp, const double *Ainv);
+// zero-start V-cycle of levels top..1 and the exact coarse solve in one
+// launch (levels[0..top]): level top's rhs fin, its result xout.  kl_small_ok:
+// level top (and the vectors of all levels below it) fits the program, within
+// max_nodes lattice nodes
+template <typename T>
+bool kl_small_ok(const DevLevel *levels, int top, long long max_nodes);
+template <typename T>
+void kl_small_vcycle(hipStream_t s, const DevLevel *levels, int top, int order, int pre, int post, T omega, T damp,
+                     const double *Ainv, const T *fin, T *xout);
 template <typename T>
 void kl_to_dof(hipStream_t s, const DevLevel &L, const T *l, double *v);
 // scratch: gj_scratch_doubles(na) doubles; inv: na^2 doubles

@@ -1093,17 +1093,33 @@ __global__ __launch_bounds__(kB) void lat_prolong_k(int ncc, int nnf, int nnc, c
 }
 
 // ---------------------------------------------------------------- small levels
-// The bottom of a mixed V-cycle in one launch: one workgroup runs the
-// pre-smoothing, defect and restriction of the small FP32 levels top..1, the
-// exact coarse solve x_A = A_AA^-1 f_A (zero iterate, zero Dirichlet data, as
+// The bottom of a lattice V-cycle in one launch: one workgroup runs the
+// pre-smoothing, defect and restriction of the small levels top..1, the exact
+// coarse solve x_A = A_AA^-1 f_A (zero iterate, zero Dirichlet data, as
 // coarse_lat_k), and the prolongation and post-smoothing back up, with a
-// workgroup barrier between steps.  Each step is the per-node code of the
-// multi-workgroup kernels (lat_class_node, restrict_class_node,
-// prolong_cell) over the same nodes, and the iterates ping-pong between lx
-// and lt exactly as the host loop does, so the results are bitwise those of
-// the launch-per-step V-cycle.  On small levels every launch is mostly fixed
-// cost; one launch replaces 9 per level plus the coarse solve.
-constexpr int kSmallMax = 3;  // FP32 levels in one program
+// workgroup barrier between steps.  Every level's iterate, sweep buffer and
+// rhs stay in LDS (the defect takes the sweep buffer): global memory is read
+// for the top level's rhs, the stencils and the coarse inverse only.  Each
+// step is the per-node code of the multi-workgroup kernels (lat_node,
+// restrict_class_node, prolong_row) over the same nodes, so the results are
+// bitwise those of the launch-per-step V-cycle.  On small levels every launch
+// is mostly fixed cost; one launch replaces 9 per level plus the coarse solve.
+// A wave takes 64 nodes of one class at a time, the classes with the longest
+// stencils first.
+// Bound by the gathers and scalar coefficient loads of one CU.  One FGMRES
+// iteration of a solve whose whole V-cycle is the program, against launches
+// (and the program with its vectors in global memory before): Q1 9^3 nodes
+// 62 / 102 (66) us, Q1 13^3 71 / 102 (79), Q2 9^3 79 / 80 (111), per-node
+// stencils Q2 9^3 89 / 97 (229); FP64 Q1 9^3 82 / 116, Q1 13^3 92 / 118, Q2 9^3
+// 110 / 101.  Q2 13^3 loses, 105 / 82 (144) us: kl_small_ok's bound on a
+// level's stencil values lies between (Q1 13^3 35937, Q2 9^3 19683, Q2 13^3
+// 79507 values), for FP64 Q2 below 9^3.
+constexpr int kSmallMax = 3;  // levels above the coarsest in one program
+constexpr long long kSmallLds = 65536;     // bytes of LDS it may take
+// stencil values (entries times nodes) of a level that one CU sweeps faster
+// than a launch over many; FP64 Q2 (waves of 64 nodes of one class leave more
+// of the CU idle)
+constexpr long long kSmallValues = 40000, kSmallValues64Q2 = 10000;
 // workgroup size: Q2's 125-point stencils need more than 128 registers per
 // lane (1024 threads) without spilling
 template <int P>
@@ -1111,108 +1127,121 @@ constexpr int small_threads() {
   return P == 1 ? 1024 : 512;
 }
 
+template <typename T>
 struct SmallLevel {
   LatArgs a;
-  const float *val, *inv, *cst;
-  float *lx, *lt, *la, *lf;
+  const T *val, *inv, *cst;
+  int x, t, f;  // LDS offsets of the level's vectors
 };
 
+template <typename T>
 struct SmallArgs {
-  SmallLevel L[kSmallMax + 1];  // L[0]: the coarsest level (a, lx, lf), L[1..top]: FP32 levels
-  int top, pre, post, na;
-  float omega, damp;
+  SmallLevel<T> L[kSmallMax + 1];  // L[0]: the coarsest level (a, x, f)
+  int top, pre, post, na, words;
+  T omega, damp;
   const double *Ainv;
   const int *dof2node0;
+  const T *fin;  // the top level's rhs
+  T *xout;       // its result
 };
-static_assert(sizeof(SmallArgs) <= 4096, "kernel arguments are limited to 4 KiB");
+static_assert(sizeof(SmallArgs<double>) <= 4096, "kernel arguments are limited to 4 KiB");
 
 // UNI: every class of the level has compact stencils (else per-node values)
-template <int P, int MODE, bool UNI>
-__device__ inline void small_sweep(const SmallLevel &L, const float *x, const float *f, float *out, float omega) {
+template <int P, int MODE, bool UNI, typename T>
+__device__ inline void small_sweep(const SmallLevel<T> &L, const T *x, const T *f, T *out, T omega) {
+  const int lane = threadIdx.x & 63;
+  int item = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), base = 0;
   for (int c = 0; c < L.a.nclass; c++) {
-    const float *cst = L.cst + c * kCst;
-    for (long long k = threadIdx.x; k < L.a.c[c].nodes; k += small_threads<P>()) {
+    const int nodes = (int)L.a.c[c].nodes, chunks = (nodes + 63) / 64;
+    const T *cst = L.cst + c * kCst;
+    for (; item < base + chunks; item += small_threads<P>() / 64) {
+      const int k = (item - base) * 64 + lane;
+      if (k >= nodes) continue;
       if (P == 1) {
-        lat_node<1, 0, 0, 0, MODE, UNI>(L.a, L.a.c[c], k, L.val, L.inv, cst, x, f, out, omega);
+        lat_node<1, 0, 0, 0, MODE, UNI, T>(L.a, L.a.c[c], k, L.val, L.inv, cst, x, f, out, omega);
       } else {
         switch (c) {
-          case 0: lat_node<2, 0, 0, 0, MODE, UNI>(L.a, L.a.c[c], k, L.val, L.inv, cst, x, f, out, omega); break;
-          case 1: lat_node<2, 1, 0, 0, MODE, UNI>(L.a, L.a.c[c], k, L.val, L.inv, cst, x, f, out, omega); break;
-          case 2: lat_node<2, 0, 1, 0, MODE, UNI>(L.a, L.a.c[c], k, L.val, L.inv, cst, x, f, out, omega); break;
-          case 3: lat_node<2, 1, 1, 0, MODE, UNI>(L.a, L.a.c[c], k, L.val, L.inv, cst, x, f, out, omega); break;
-          case 4: lat_node<2, 0, 0, 1, MODE, UNI>(L.a, L.a.c[c], k, L.val, L.inv, cst, x, f, out, omega); break;
-          case 5: lat_node<2, 1, 0, 1, MODE, UNI>(L.a, L.a.c[c], k, L.val, L.inv, cst, x, f, out, omega); break;
-          case 6: lat_node<2, 0, 1, 1, MODE, UNI>(L.a, L.a.c[c], k, L.val, L.inv, cst, x, f, out, omega); break;
-          default: lat_node<2, 1, 1, 1, MODE, UNI>(L.a, L.a.c[c], k, L.val, L.inv, cst, x, f, out, omega); break;
+          case 0: lat_node<2, 0, 0, 0, MODE, UNI, T>(L.a, L.a.c[c], k, L.val, L.inv, cst, x, f, out, omega); break;
+          case 1: lat_node<2, 1, 0, 0, MODE, UNI, T>(L.a, L.a.c[c], k, L.val, L.inv, cst, x, f, out, omega); break;
+          case 2: lat_node<2, 0, 1, 0, MODE, UNI, T>(L.a, L.a.c[c], k, L.val, L.inv, cst, x, f, out, omega); break;
+          case 3: lat_node<2, 1, 1, 0, MODE, UNI, T>(L.a, L.a.c[c], k, L.val, L.inv, cst, x, f, out, omega); break;
+          case 4: lat_node<2, 0, 0, 1, MODE, UNI, T>(L.a, L.a.c[c], k, L.val, L.inv, cst, x, f, out, omega); break;
+          case 5: lat_node<2, 1, 0, 1, MODE, UNI, T>(L.a, L.a.c[c], k, L.val, L.inv, cst, x, f, out, omega); break;
+          case 6: lat_node<2, 0, 1, 1, MODE, UNI, T>(L.a, L.a.c[c], k, L.val, L.inv, cst, x, f, out, omega); break;
+          default: lat_node<2, 1, 1, 1, MODE, UNI, T>(L.a, L.a.c[c], k, L.val, L.inv, cst, x, f, out, omega); break;
         }
       }
     }
+    base += chunks;
   }
 }
 
 // UNI: every small level has compact stencils in every class
-template <int P, bool UNI>
-__global__ __launch_bounds__(small_threads<P>()) void lat_small_k(SmallArgs s) {
+template <int P, bool UNI, typename T>
+__global__ __launch_bounds__(small_threads<P>()) void lat_small_k(SmallArgs<T> s) {
+  extern __shared__ double small_lds[];
+  T *const m = (T *)small_lds;
   constexpr int NT = small_threads<P>();
-  float *xs[kSmallMax + 1];
+  int xs[kSmallMax + 1];
+  const int n3 = s.L[s.top].a.nn * s.L[s.top].a.nn * s.L[s.top].a.nn, ftop = s.L[s.top].f;
+  for (int k = threadIdx.x; k < s.words; k += NT) {  // boundary nodes and zero iterates
+    const int e = k - ftop;
+    m[k] = e >= 0 && e < n3 ? s.fin[e] : T(0);
+  }
+  __syncthreads();
   // down: levels top .. 1
   for (int i = s.top; i >= 1; i--) {
-    const SmallLevel &L = s.L[i], &C = s.L[i - 1];
-    float *x = L.lx, *t = L.lt;
+    const SmallLevel<T> &L = s.L[i], &C = s.L[i - 1];
+    int x = L.x, t = L.t;
     for (int k = 0; k < s.pre; k++) {
-      if (k == 0) small_sweep<P, kLJacobiZero, UNI>(L, nullptr, L.lf, t, s.omega);
-      else small_sweep<P, kLJacobi, UNI>(L, x, L.lf, t, s.omega);
-      float *u = x;
+      if (k == 0) small_sweep<P, kLJacobiZero, UNI, T>(L, nullptr, m + L.f, m + t, s.omega);
+      else small_sweep<P, kLJacobi, UNI, T>(L, m + x, m + L.f, m + t, s.omega);
+      const int u = x;
       x = t;
       t = u;
       __syncthreads();
     }
-    if (s.pre == 0) {
-      const long long n3 = (long long)L.a.nn * L.a.nn * L.a.nn;
-      for (long long k = threadIdx.x; k < n3; k += NT) x[k] = 0.f;
-      __syncthreads();
-    }
-    small_sweep<P, kLDefect, UNI>(L, x, L.lf, L.la, 0.f);
+    small_sweep<P, kLDefect, UNI, T>(L, m + x, m + L.f, m + t, T(0));
     __syncthreads();
     for (int c = 0; c < C.a.nclass; c++)
-      for (long long k = threadIdx.x; k < C.a.c[c].nodes; k += NT)
-        restrict_class_node<P>(C.a, c, k, L.a.nn, L.la, C.lf, ZeroSweep{nullptr, nullptr, 0.f});
+      for (int k = threadIdx.x; k < (int)C.a.c[c].nodes; k += NT)
+        restrict_class_node<P, T>(C.a, c, k, L.a.nn, m + t, m + C.f, ZeroSweepT<T>{nullptr, nullptr, T(0)});
     xs[i] = x;
     __syncthreads();
   }
   // coarsest: one wavefront per row, the lanes over the columns
   {
     const int lane = threadIdx.x & 63;
+    const T *f0 = m + s.L[0].f;
+    T *x0 = m + s.L[0].x;
     for (int row = threadIdx.x >> 6; row < s.na; row += NT / 64) {
       double v = 0;
-      for (int j = lane; j < s.na; j += 64) v += s.Ainv[(long long)row * s.na + j] * (double)s.L[0].lf[s.dof2node0[j]];
+      for (int j = lane; j < s.na; j += 64) v += s.Ainv[(long long)row * s.na + j] * (double)f0[s.dof2node0[j]];
 #pragma unroll
       for (int o = 32; o > 0; o >>= 1) v += __shfl_xor(v, o, 64);
-      if (lane == 0) s.L[0].lx[s.dof2node0[row]] = (float)(0.0 + v);
+      if (lane == 0) x0[s.dof2node0[row]] = (T)(0.0 + v);
     }
     __syncthreads();
   }
   // up: levels 1 .. top
+  int cx = s.L[0].x;
   for (int i = 1; i <= s.top; i++) {
-    const SmallLevel &L = s.L[i], &C = s.L[i - 1];
-    float *x = xs[i], *t = x == L.lx ? L.lt : L.lx;
+    const SmallLevel<T> &L = s.L[i], &C = s.L[i - 1];
+    int x = xs[i], t = x == L.x ? L.t : L.x;
     const int ncc = (C.a.nn - 1) / P;
-    for (long long c = threadIdx.x; c < (long long)ncc * ncc * ncc * 4 * P * P; c += NT)
-      prolong_row<P>(c, ncc, L.a.nn, C.a.nn, C.lx, x, s.damp);
+    for (int c = threadIdx.x; c < ncc * ncc * ncc * 4 * P * P; c += NT)
+      prolong_row<P, T>(c, ncc, L.a.nn, C.a.nn, m + cx, m + x, s.damp);
     __syncthreads();
     for (int k = 0; k < s.post; k++) {
-      small_sweep<P, kLJacobi, UNI>(L, x, L.lf, t, s.omega);
-      float *u = x;
+      small_sweep<P, kLJacobi, UNI, T>(L, m + x, m + L.f, m + t, s.omega);
+      const int u = x;
       x = t;
       t = u;
       __syncthreads();
     }
-    if (x != L.lx) {
-      const long long n3 = (long long)L.a.nn * L.a.nn * L.a.nn;
-      for (long long k = threadIdx.x; k < n3; k += NT) L.lx[k] = x[k];
-      __syncthreads();
-    }
+    cx = x;
   }
+  for (int k = threadIdx.x; k < n3; k += NT) s.xout[k] = m[cx + k];
 }
 
 __global__ void lat_convert_k(long long n, const int *__restrict__ perm, const double *__restrict__ val,
@@ -2422,37 +2451,74 @@ void kl_cast_f2d(hipStream_t s, int64_t n, const float *a, double *b) {
   cast_f2d_k<<<(int)std::min<int64_t>((n + kB - 1) / kB, 2048), kB, 0, s>>>(n, a, b);
 }
 
-void kl_small_vcycle(hipStream_t st, const DevLevel *levels, int top, int order, int pre, int post, float omega,
-                     float damp, const double *Ainv) {
-  if (top < 1 || top > kSmallMax) return;
-  SmallArgs s{};
+// Levels 0..top in the one-workgroup program: words of LDS it takes (x, t and
+// f of every level, x and f of the coarsest)
+static long long small_words(const DevLevel *levels, int top) {
+  long long w = 0;
+  for (int i = 0; i <= top; i++) w += (i ? 3LL : 2LL) * levels[i].nn * levels[i].nn * levels[i].nn;
+  return w;
+}
+template <typename T>
+bool kl_small_ok(const DevLevel *levels, int top, long long max_nodes) {
+  if (top < 1 || top > kSmallMax) return false;
+  const DevLevel &D = levels[top];
+  const long long nodes = (long long)D.nn * D.nn * D.nn;
+  if (nodes > max_nodes || D.nclass <= 0 || D.lat_affine) return false;
+  if (sizeof(T) == 8 && !D.lat_exact64) return false;  // FP64: compact stencils only
+  if (D.lat_nval > (sizeof(T) == 8 && D.nclass == 8 ? kSmallValues64Q2 : kSmallValues)) return false;
+  return small_words(levels, top) * (long long)sizeof(T) <= kSmallLds;
+}
+template bool kl_small_ok<float>(const DevLevel *, int, long long);
+template bool kl_small_ok<double>(const DevLevel *, int, long long);
+
+template <typename T>
+void kl_small_vcycle(hipStream_t st, const DevLevel *levels, int top, int order, int pre, int post, T omega, T damp,
+                     const double *Ainv, const T *fin, T *xout) {
+  if (!kl_small_ok<T>(levels, top, 1LL << 40)) throw std::logic_error("levels too large for the one-workgroup V-cycle");
+  SmallArgs<T> s{};
+  int w = 0;
   for (int i = 0; i <= top; i++) {
     const DevLevel &D = levels[i];
+    const LatVals<T> v(D);
+    const int n3 = D.nn * D.nn * D.nn;
     s.L[i].a = lat_args(D);
-    s.L[i].val = D.lval;
-    s.L[i].inv = D.linv;
-    s.L[i].cst = D.lcst;
-    s.L[i].lx = D.lx;
-    s.L[i].lt = D.lt;
-    s.L[i].la = D.la;
-    s.L[i].lf = D.lf;
+    s.L[i].val = v.val;
+    s.L[i].inv = v.inv;
+    s.L[i].cst = v.cst;
+    s.L[i].x = w;
+    s.L[i].f = w + n3;
+    s.L[i].t = i ? w + 2 * n3 : w;
+    w += (i ? 3 : 2) * n3;
   }
   s.top = top;
   s.pre = pre;
   s.post = post;
   s.na = levels[0].nact;
+  s.words = w;
   s.omega = omega;
   s.damp = damp;
   s.Ainv = Ainv;
   s.dof2node0 = levels[0].ldof2node;
+  s.fin = fin;
+  s.xout = xout;
   bool uni = true;
   for (int i = 1; i <= top; i++)
     for (int c = 0; c < s.L[i].a.nclass; c++) uni = uni && s.L[i].a.uni[c];
-  if (order == 1 && uni) lat_small_k<1, true><<<1, small_threads<1>(), 0, st>>>(s);
-  else if (order == 1) lat_small_k<1, false><<<1, small_threads<1>(), 0, st>>>(s);
-  else if (uni) lat_small_k<2, true><<<1, small_threads<2>(), 0, st>>>(s);
-  else lat_small_k<2, false><<<1, small_threads<2>(), 0, st>>>(s);
+  const size_t lds = sizeof(T) * w;
+  if constexpr (sizeof(T) == 8) {
+    if (order == 1) lat_small_k<1, true, T><<<1, small_threads<1>(), lds, st>>>(s);
+    else lat_small_k<2, true, T><<<1, small_threads<2>(), lds, st>>>(s);
+  } else {
+    if (order == 1 && uni) lat_small_k<1, true, T><<<1, small_threads<1>(), lds, st>>>(s);
+    else if (order == 1) lat_small_k<1, false, T><<<1, small_threads<1>(), lds, st>>>(s);
+    else if (uni) lat_small_k<2, true, T><<<1, small_threads<2>(), lds, st>>>(s);
+    else lat_small_k<2, false, T><<<1, small_threads<2>(), lds, st>>>(s);
+  }
 }
+template void kl_small_vcycle<float>(hipStream_t, const DevLevel *, int, int, int, int, float, float, const double *,
+                                     const float *, float *);
+template void kl_small_vcycle<double>(hipStream_t, const DevLevel *, int, int, int, int, double, double,
+                                      const double *, const double *, double *);
 
 void kl_clear_boundary(hipStream_t s, const DevLevel &L, double *v, int64_t ld, int count) {
   const int nd = L.ndof - L.nact;

@@ -83,3 +83,28 @@ def test_fp64_lattice_rotating_field_solve(monkeypatch):
     (x1, s1), (x0, s0) = both(monkeypatch, lambda: P.solve(sp))
     assert s1.iterations == s0.iterations and rel(x1, x0) < SOL_TOL
     P.close()
+
+
+# the one-workgroup program for the bottom levels, both value types: the last
+# mesh that takes it and the first that does not, two and three levels in it,
+# no pre-smoothing, odd numbers of sweeps (the iterate ends in the other
+# buffer), per-node stencils; the same node code in the same order, so bitwise
+@pytest.mark.parametrize("order,m,k0,levels,rot,pre,post", [
+    (1, 2, 0, 2, 0, 3, 3), (1, 2, 0, 4, 0, 2, 1), (1, 3, 0, 3, 0, 1, 2), (1, 7, 0, 2, 0, 3, 3), (1, 1, 1, 3, 1, 3, 2),
+    (2, 1, 0, 3, 0, 0, 3), (2, 2, 0, 2, 0, 2, 3), (2, 3, 0, 2, 0, 3, 3), (2, 1, 1, 3, 1, 3, 3), (1, 3, 0, 3, 1, 2, 3)])
+def test_small_program_matches_launches(order, m, k0, levels, rot, pre, post, monkeypatch):
+    P = pm.Problem(order, m, k0, levels, box=(1.0, 0.9, 0.8))
+    P.assemble(pm.coeffs(eps=0.05, b=(1.0, 0.5, 0.25), conv_kind=rot, rot_c=(0.4, 0.6), supg=1, f_val=1.0))
+    i = P.info(levels - 1)
+    r = np.random.default_rng(3).standard_normal(i["ndof"])
+    r[i["nact"]:] = 0.0
+    for prec in (pm.FP64, pm.MIXED):
+        sp = pm.solver_params(omega=0.5, pre=pre, post=post, rel_tol=1e-10, maxit=60, precision=prec)
+        out = []
+        for bound in ("3000", "0"):
+            monkeypatch.setenv("CD3D_SMALL_NODES", bound)
+            x, st = P.solve(sp, check=False)
+            out.append((P.vcycle(sp, r), x, st.iterations, st.status))
+        assert out[0][2:] == out[1][2:]
+        assert np.array_equal(out[0][0], out[1][0]) and np.array_equal(out[0][1], out[1][1])
+    P.close()
