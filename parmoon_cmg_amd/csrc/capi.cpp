@@ -942,9 +942,6 @@ struct Space {
   // precond leaves z in lat_top->lx (z == nullptr) and the product
   // kl_spmv64_f32 reads it there and writes the column
   bool z32 = false;
-  // orthogonalise by the low-synchronisation form of MGS (k_ls_step)
-  // instead of MGS step by step (the FP64 form keeps the reference's MGS)
-  bool lowsync = false;
   // before the iteration, once the Krylov space (R columns) is there
   std::function<void(int)> prepare;
 };
@@ -972,9 +969,6 @@ Space lattice_space(cd3d_problem &P) {
   S.matvec = [&P, &F, p](const double *x, double *y) { kl_spmv64(P.stream, F, p, x, y); };
   // the Krylov vectors vanish on the boundary, as the V-cycle's rhs must
   S.r32 = F.lf;
-  // CD3D_FGMRES_MGS=1: MGS step by step as in the FP64 form
-  const char *em = getenv("CD3D_FGMRES_MGS");
-  S.lowsync = !(em && em[0] == '1');
   S.lat_top = &F;
   S.lat_order = p;
   // CD3D_FGMRES_Z32=0: FP64 columns, written by a cast after each V-cycle
@@ -1052,7 +1046,15 @@ int fgmres_iterate(cd3d_problem &P, const cd3d_solver_params &sp, const Space &S
   float *Z32 = S.z32 ? (float *)Z : nullptr;
   std::vector<double> H((size_t)(R + 1) * R, 0.0), s(R + 1), cs(R + 1), sn(R + 1);
   double *pa = P.red, *pb = P.red + kRedBlocks;
-  const bool lowsync = S.lowsync && R <= k_ls_max() && ld % 2 == 0 && ((uintptr_t)V & 15) == 0 &&
+  // Orthogonalisation: the low-synchronisation form of MGS (k_ls_step: the
+  // MGS column in two passes over the basis, four launches) unless
+  // CD3D_FGMRES_MGS=1 or the restart length exceeds its bound (then MGS vector
+  // by vector, i + 2 launches that read w and two basis vectors each).
+  // FP64 form, assemble + solve Q2 64^3 13.7 -> 12.2 ms; twelve batched Q1
+  // problems 8.3 -> 7.2 ms; mixed time steps of Q2 24^3 in DOF order 30.0 ->
+  // 27.5 ms (5 us per launch of MGS whatever the size).
+  const char *em = getenv("CD3D_FGMRES_MGS");
+  const bool lowsync = !(em && em[0] == '1') && R <= k_ls_max() && ld % 2 == 0 && ((uintptr_t)V & 15) == 0 &&
                        ((uintptr_t)w & 15) == 0;
   if (lowsync) ensure_ls(P, N);
   // the finest lattice level's zero-start sweep written beside each Krylov
@@ -1258,11 +1260,10 @@ static void batch_solve_impl(BatchRun &br, std::vector<BatchState> &st) {
   br.maxblk.assign(NL, 0);
   br.maxn.assign(NL, 0);
   br.maxn_c.assign(NL, 0);
-  // the mixed form orthogonalises in two passes over the basis per Arnoldi
-  // step (kb_ls_step) unless CD3D_FGMRES_MGS=1; the FP64 form keeps MGS
-  // vector by vector
+  // two passes over the basis per Arnoldi step (kb_ls_step) unless
+  // CD3D_FGMRES_MGS=1 (MGS vector by vector), as in fgmres_iterate
   const char *em = getenv("CD3D_FGMRES_MGS");
-  bool lowsync = sp.precision == CD3D_MIXED && R <= k_ls_max() && !(em && em[0] == '1');
+  bool lowsync = R <= k_ls_max() && !(em && em[0] == '1');
   for (int b = 0; b < B; b++) {
     cd3d_problem &P = *br.ps[b];
     coarse_join(P);

@@ -203,7 +203,7 @@ struct Problem {
   double *V = nullptr, *Z = nullptr, *w = nullptr, *xs = nullptr, *bs = nullptr;
   double *red = nullptr;      // reduction partials
   double *dscal = nullptr;    // device scalars: H column at [0, restart], y at [yoff, yoff + restart)
-  // low-synchronisation Gram-Schmidt of the mixed form: dot partials and the
+  // low-synchronisation Gram-Schmidt: dot partials and the
   // strictly lower part of V^T V (allocated on first use)
   double *ls_part = nullptr, *ls_L = nullptr;
   int ls_blocks = 0;          // chunks ls_part holds partials for
@@ -405,7 +405,7 @@ struct BatchProblem {
   double *red = nullptr;          // 2 x kBatchRed reduction partials
   double *scal = nullptr;         // kBatchScal device scalars
   const double *coef = nullptr;   // kBatchCoef host-written coefficients
-  // the mixed form's low-synchronisation Gram-Schmidt: dot partials and L
+  // low-synchronisation Gram-Schmidt: dot partials and L
   double *ls_part = nullptr, *ls_L = nullptr;
 };
 // level kernels: lev = this level's table (B entries); grid sizes from the

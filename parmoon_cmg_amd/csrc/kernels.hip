@@ -563,7 +563,7 @@ __global__ __launch_bounds__(kBlock) void scale_copy2_k(int n, const double *__r
   }
 }
 
-// Low-synchronisation Gram-Schmidt of the mixed form's FGMRES (the
+// Low-synchronisation Gram-Schmidt of FGMRES (the
 // inverse compact WY form of modified Gram-Schmidt: Swirydowicz, Langou,
 // Ananthan, Yang, Thomas, Numer. Linear Algebra Appl. 28 (2021) e2343).
 // At Arnoldi step i, with w = A z_i and the basis V_0 .. V_i, one pass
