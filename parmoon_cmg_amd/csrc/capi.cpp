@@ -434,7 +434,7 @@ static void ensure_slots(cd3d_problem &P, int l) {
 // scratch vector then (default: the level's assembled rhs)
 static int assemble_level(cd3d_problem &P, int l, const cd3d_coeffs &co, int what, double *val, bool csr = true,
                           double *rhs = nullptr) {
-  if (val == P.dl[l].val) P.dl[l].invdiag_ok = false;
+  if (val == P.dl[l].val) P.dl[l].invdiag_ok = P.dl[l].gp_ok = false;
   DevLevel &D = P.dl[l];
   if (!rhs) rhs = D.rhs_asm;
   const AsmParams ap = asm_params(P, D, co, what);
@@ -558,7 +558,7 @@ static long long small_nodes_bound() {
 static void refresh_f32(cd3d_problem &P, bool values = true) {
   for (size_t l = 0; l < P.dl.size(); l++) {
     DevLevel &D = P.dl[l];
-    D.invdiag_ok = false;  // only the FP64 smoother reads it: computed there on first use
+    D.invdiag_ok = D.gp_ok = false;  // only the FP64 smoothers read them: computed there on first use
     if (l == 0) D.lat_fresh = 0;  // the coarsest level has no FP32 stencils
     if (l > 0) {
       auto per_node = [&](bool with_map) {  // per-node FP32 stencils (4 bytes per nonzero), on first need
@@ -678,6 +678,31 @@ static void ensure_mc(cd3d_problem &P, int l) {
 // sweep) of level l on the device (first use)
 static void ensure_gs(cd3d_problem &P, int l, bool backward) {
   DevLevel &D = P.dl[l];
+  if (D.gp_steps) return;
+  // levels that fit a workgroup's LDS: the packed schedule (both directions;
+  // CD3D_GS_LDS=0, read when the schedule is built, keeps the one in memory)
+  const char *e = getenv("CD3D_GS_LDS");
+  if (!(e && e[0] == '0') && !D.gs_rows[0] && D.nact > 0 && k_gs_packed_fits(D.ndof, 1, 32)) {
+    std::vector<int> start, rows, col, pos;
+    const int slots = build_gs_packed(P.hl[l], start, rows, col, pos), steps = (int)start.size() - 1;
+    if (slots && k_gs_packed_fits(D.ndof, steps, slots)) {
+      D.gp_start = dalloc<int>(P, start.size());
+      D.gp_rows = dalloc<int>(P, rows.size());
+      D.gp_col = dalloc<int>(P, col.size());
+      D.gp_pos = dalloc<int>(P, pos.size());
+      D.gp_val = dalloc<double>(P, pos.size());
+      D.gp_inv = dalloc<double>(P, rows.size());
+      upload(P, D.gp_start, start);
+      upload(P, D.gp_rows, rows);
+      upload(P, D.gp_col, col);
+      upload(P, D.gp_pos, pos);
+      HIPCHK(hipStreamSynchronize(P.stream));  // the host vectors end here
+      D.gp_slots = slots;
+      D.gp_steps = steps;
+      D.gp_ok = false;
+      return;
+    }
+  }
   for (int b = 0; b <= (backward ? 1 : 0); b++) {
     if (D.gs_rows[b]) continue;
     std::vector<int> rows, start;
@@ -706,19 +731,32 @@ void cycle64(VC &v, int i, bool zero_start) {
   if (sm == 13 || sm == 2 || sm == 3) {
     if (sm == 13) ensure_mc(P, i);
     else ensure_gs(P, i, sm == 3);
-    auto relax = [&]() {
-      if (sm == 13) k_mcssor(P.stream, L, L.sol, L.rhs, v.sp.omega);
-      else k_gs_sweep(P.stream, L, L.sol, L.rhs, v.sp.omega, sm);
+    const bool packed = sm != 13 && L.gp_steps > 0;
+    if (packed && !L.gp_ok) {
+      k_gs_pack(P.stream, L);
+      L.gp_ok = true;
+    }
+    auto relax = [&](int sweeps, bool zero) {
+      if (sweeps == 0) return;
+      if (packed) {
+        k_gs_packed(P.stream, L, L.sol, L.rhs, v.sp.omega, sm, sweeps, zero);
+        return;
+      }
+      for (int k = 0; k < sweeps; k++) {
+        if (sm == 13) k_mcssor(P.stream, L, L.sol, L.rhs, v.sp.omega);
+        else k_gs_sweep(P.stream, L, L.sol, L.rhs, v.sp.omega, sm);
+      }
     };
-    if (zero_start) HIPCHK(hipMemsetAsync(L.sol, 0, sizeof(double) * L.ndof, P.stream));
-    for (int k = 0; k < v.sp.pre; k++) relax();
+    if (zero_start && !(packed && v.sp.pre > 0))
+      HIPCHK(hipMemsetAsync(L.sol, 0, sizeof(double) * L.ndof, P.stream));
+    relax(v.sp.pre, zero_start);
     if (v.sp.pre == 0 && zero_start) k_copy_range(P.stream, L.nact, L.ndof, L.rhs, L.sol);
     k_defect(P.stream, L, L.sol, L.rhs, L.aux);
     k_restrict(P.stream, L, C, L.aux, C.rhs);
     for (int r = 0; r < v.rec[i]; r++) cycle64(v, i - 1, r == 0);
     if (v.sp.cycle < 1) v.rec[i] = 1;  // F-cycle
     k_prolong_update(P.stream, L, C, C.sol, L.sol, v.sp.gmg_damp);
-    for (int k = 0; k < v.sp.post; k++) relax();
+    relax(v.sp.post, false);
     return;
   }
   double *x = L.sol, *t = L.tmp;
@@ -2173,7 +2211,7 @@ static int tcd_step_impl(cd3d_problem &P, const cd3d_coeffs &co0, const cd3d_sol
     explicit SystemSwap(cd3d_problem &p) : P(p) {}
     void swap_level(int l) {
       std::swap(P.dl[l].val, P.dl[l].aconv);
-      P.dl[l].invdiag_ok = false;
+      P.dl[l].invdiag_ok = P.dl[l].gp_ok = false;
     }
     ~SystemSwap() {
       for (int l : levels) swap_level(l);

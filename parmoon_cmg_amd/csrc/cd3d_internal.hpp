@@ -106,6 +106,15 @@ struct DevLevel {
   // (build_gs_schedule; uploaded on first use)
   int *gs_rows[2] = {nullptr, nullptr}, *gs_start[2] = {nullptr, nullptr};
   int gs_nlev[2] = {0, 0};
+  // the same sweeps with the iterate in LDS (levels whose vectors fit,
+  // build_gs_packed): steps of at most kGsRows rows of one wavefront level,
+  // their rows' off-diagonal entries packed in step order (gp_slots per row),
+  // the entries' CSR positions, and 1/a_ii; gp_ok: gp_val and gp_inv hold the
+  // values of `val`
+  int gp_steps = 0, gp_slots = 0;
+  int *gp_start = nullptr, *gp_rows = nullptr, *gp_col = nullptr, *gp_pos = nullptr;
+  double *gp_val = nullptr, *gp_inv = nullptr;
+  bool gp_ok = false;
   // assembly
   int4 *cells = nullptr;
   int *slots = nullptr;
@@ -244,6 +253,12 @@ void build_colours(HostLevel &L, int order);
 void build_row_blocks(const std::vector<int> &rowptr, int max_nnz, int max_rows, std::vector<int> &blk);
 void build_mc_colours(HostLevel &L, int order);
 void build_gs_schedule(const HostLevel &L, bool backward, std::vector<int> &rows, std::vector<int> &start);
+constexpr int kGsRows = 16;  // rows of one step of the packed schedule
+// the forward schedule cut into steps (start, rows) and the rows' entries
+// without the diagonal, slots per row: columns (padding: the row itself) and
+// CSR positions (padding: -1).  Returns slots (32 or 128), 0 when a row is too long
+int build_gs_packed(const HostLevel &L, std::vector<int> &start, std::vector<int> &rows, std::vector<int> &col,
+                    std::vector<int> &pos);
 void build_lattice(HostLevel &L, int order);
 void basis_tables(int order, std::vector<double> &tab);
 int quad_points_1d(int order);
@@ -295,6 +310,13 @@ void k_ls_step(hipStream_t s, int n, int i, const double *V, int64_t ld, double 
 // one SOR (kind 2) or SSOR (kind 3) sweep in the reference's row order, in
 // place: x_D = f_D, then the wavefront schedule(s) of the level
 void k_gs_sweep(hipStream_t s, const DevLevel &L, double *x, const double *f, double omega, int kind);
+// `sweeps` of them from x (zero: from a zero iterate) in one launch on a level
+// with a packed schedule (gp_steps > 0, gp_ok): k_gs_pack refreshes its values
+void k_gs_packed(hipStream_t s, const DevLevel &L, double *x, const double *f, double omega, int kind, int sweeps,
+                 bool zero);
+void k_gs_pack(hipStream_t s, const DevLevel &L);
+// the packed sweep fits a workgroup's LDS on the current device
+bool k_gs_packed_fits(int ndof, int steps, int slots);
 void k_invdiag(hipStream_t s, const DevLevel &L);
 void k_restrict(hipStream_t s, const DevLevel &F, const DevLevel &C, const double *fine, double *coarse);
 void k_prolong_update(hipStream_t s, const DevLevel &F, const DevLevel &C, const double *coarse, double *x,

@@ -1381,7 +1381,7 @@ __device__ inline unsigned gj_key(double x) {
 // (uniform); every lane takes part
 template <int CTRL>
 __device__ inline unsigned dpp_max(unsigned v) {
-  const unsigned o = (unsigned)__builtin_amdgcn_update_dpp((int)v, (int)v, CTRL, 0xf, 0xf, false);
+  const unsigned o = (unsigned)__builtin_amdgcn_update_dpp(0, (int)v, CTRL, 0xf, 0xf, true);
   return v > o ? v : o;
 }
 __device__ inline unsigned row16_max(unsigned v) {
@@ -1781,7 +1781,7 @@ __global__ void dirichlet_rows_k(int n, int nact, const int *__restrict__ rp, do
 // levels hold a handful of rows (about 8 on the 32^3-cell Q2 level).  Only
 // the gather of x depends on the previous level, so each wave fetches its
 // row of the next level (index, extent, the first 128 entries, f_i, x_i)
-// while it works on the current one.
+// while it works on the current one.  (Levels that fit in LDS: gs_packed_k.)
 constexpr int kGsBlock = 1024;
 struct GsRow {
   int i, b, e, c0, c1;
@@ -1850,6 +1850,132 @@ __global__ __launch_bounds__(kGsBlock) void gs_sweep_k(int nlev, const int *__re
   }
 }
 
+// The same sweeps on a level whose iterate and rhs fit the LDS of one CU (up
+// to about 10000 unknowns), any number of them in one launch.  The schedule
+// comes packed: steps of at most kGsRows independent rows, 16 lanes to a row
+// with EPL entries each, so nothing but the gather of x (LDS), a sum over 16
+// lanes (DPP) and one barrier lies between two steps; the entries of the step
+// four ahead are requested while a step runs (the barrier orders LDS only and
+// leaves them in flight).  The backward sweep takes the steps in reverse: a
+// row's later-numbered neighbours are in later wavefront levels.
+// Bound by that chain, 0.25 us per step (Q1; Q2 0.34): assemble + solve Q1
+// 16^3 cells (3375 rows, 849 levels) with SSOR 3 + 3, 39.8 -> 12.0 ms against
+// gs_sweep_k (x in L2, 1.0 us per level).  Measured and not kept: one wave with steps of 4
+// rows and no barrier (15.9 against 13.3 ms on the same problem at another
+// coefficient).  Levels beyond the LDS keep gs_sweep_k.
+struct LdsFence {
+  static __device__ inline void barrier() {
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup", "local");
+    __builtin_amdgcn_s_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup", "local");
+  }
+};
+template <int CTRL>
+__device__ inline double dpp_add(double v) {
+  const int lo = __double2loint(v), hi = __double2hiint(v);
+  return v + __hiloint2double(__builtin_amdgcn_update_dpp(0, hi, CTRL, 0xf, 0xf, true),
+                              __builtin_amdgcn_update_dpp(0, lo, CTRL, 0xf, 0xf, true));
+}
+template <int EPL>
+struct GsSlot {
+  int i, c[EPL];
+  double v[EPL], inv;
+};
+
+template <int EPL>
+__global__ __launch_bounds__(kBlock) void gs_packed_k(int n, int nact, int nsteps, const int *__restrict__ start,
+                                                      const int *__restrict__ rows, const int *__restrict__ col,
+                                                      const double *__restrict__ val, const double *__restrict__ inv,
+                                                      double *__restrict__ x, const double *__restrict__ f,
+                                                      double omega, int passes, int both, int zero) {
+  static_assert(kBlock == 16 * kGsRows, "16 lanes per row of a step");
+  extern __shared__ double gs_lds[];
+  double *xs = gs_lds, *fs = gs_lds + n;
+  int *st = (int *)(fs + n);
+  for (int i = threadIdx.x; i < n; i += kBlock) {
+    const double fi = f[i];
+    fs[i] = fi;
+    xs[i] = i >= nact ? fi : zero ? 0.0 : x[i];
+  }
+  for (int i = threadIdx.x; i <= nsteps; i += kBlock) st[i] = start[i];
+  __syncthreads();
+  const int g = threadIdx.x >> 4, lane = threadIdx.x & 15;
+  GsSlot<EPL> q[4];
+  // the step to request next, and its extent, read from LDS one step ahead
+  int pu = 0, pp = 0, b, e;
+  auto extent = [&]() {
+    const int step = both && (pp & 1) ? nsteps - 1 - pu : pu;
+    b = st[step];
+    e = st[step + 1];
+    if (pp >= passes) e = b;
+    if (++pu == nsteps) {
+      pu = 0;
+      pp++;
+    }
+  };
+  auto fetch = [&](GsSlot<EPL> &s, int b0, int e0) {
+    const int r = b0 + g;
+    s.i = -1;
+    s.inv = 0.0;
+#pragma unroll
+    for (int k = 0; k < EPL; k++) {
+      s.c[k] = 0;
+      s.v[k] = 0.0;
+    }
+    if (r < e0) {
+      s.i = rows[r];
+      s.inv = inv[r];
+      const unsigned at = ((unsigned)r * 16u + (unsigned)lane) * EPL;  // the packed rows fit 32 bits
+#pragma unroll
+      for (int k = 0; k < EPL; k++) {
+        s.c[k] = col[at + k];
+        s.v[k] = val[at + k];
+      }
+    }
+  };
+  extent();
+#pragma unroll
+  for (int s = 0; s < 3; s++) {
+    const int b0 = b, e0 = e;
+    extent();
+    fetch(q[s], b0, e0);
+  }
+  const int64_t total = (int64_t)passes * nsteps;
+  for (int64_t t = 0; t < total; t += 4) {
+#pragma unroll
+    for (int s = 0; s < 4; s++) {
+      const int i = max(q[s].i, 0);
+      double w[EPL];
+#pragma unroll
+      for (int k = 0; k < EPL; k++) w[k] = xs[q[s].c[k]];
+      const double xi = xs[i], fi = fs[i];
+      // while these are on their way: the slot of the previous step
+      const int b0 = b, e0 = e;
+      extent();
+      fetch(q[(s + 3) & 3], b0, e0);
+      double a = 0.0;
+#pragma unroll
+      for (int k = 0; k < EPL; k++) a = fma(q[s].v[k], w[k], a);
+      a = dpp_add<0x121>(dpp_add<0x122>(dpp_add<0x124>(dpp_add<0x128>(a))));  // row_ror: the 16 lanes of the row
+      if (lane == 0 && q[s].i >= 0) xs[i] = omega * ((fi - a) * q[s].inv - xi) + xi;
+      LdsFence::barrier();
+    }
+  }
+  __syncthreads();
+  for (int i = threadIdx.x; i < n; i += kBlock) x[i] = xs[i];
+}
+
+__global__ __launch_bounds__(kBlock) void gs_pack_k(int64_t nslots, int nact, const int *__restrict__ pos,
+                                                    const int *__restrict__ rows, const int *__restrict__ diag,
+                                                    const double *__restrict__ a, double *__restrict__ val,
+                                                    double *__restrict__ inv) {
+  for (int64_t k = blockIdx.x * (int64_t)kBlock + threadIdx.x; k < nslots; k += (int64_t)gridDim.x * kBlock) {
+    const int p = pos[k];
+    val[k] = p >= 0 ? a[p] : 0.0;
+    if (k < nact) inv[k] = 1.0 / a[diag[rows[k]]];
+  }
+}
+
 }  // namespace
 
 // ---------------------------------------------------------------- launchers
@@ -1913,6 +2039,38 @@ void k_gs_sweep(hipStream_t s, const DevLevel &L, double *x, const double *f, do
   if (kind == 3)
     gs_sweep_k<<<1, kGsBlock, 0, s>>>(L.gs_nlev[1], L.gs_start[1], L.gs_rows[1], L.rowptr, L.col, L.val, x, f,
                                       omega);
+}
+static size_t gs_packed_lds(int ndof, int steps) { return sizeof(double) * 2 * ndof + sizeof(int) * (steps + 1); }
+bool k_gs_packed_fits(int ndof, int steps, int slots) {
+  constexpr size_t kMax = 160 * 1024;
+  if (gs_packed_lds(ndof, steps) > kMax) return false;
+  // more than 64 KiB of LDS wants an opt-in per kernel, once per device; the
+  // serving loop's threads reach this concurrently
+  static std::mutex mu;
+  static signed char ok[2][64];  // 0 unknown, 1 granted, -1 refused
+  int dev = 0;
+  (void)hipGetDevice(&dev);
+  std::lock_guard<std::mutex> g(mu);
+  signed char &o = ok[slots == 32 ? 0 : 1][dev & 63];
+  if (!o) {
+    const void *k = slots == 32 ? (const void *)gs_packed_k<2> : (const void *)gs_packed_k<8>;
+    o = hipFuncSetAttribute(k, hipFuncAttributeMaxDynamicSharedMemorySize, (int)kMax) == hipSuccess ? 1 : -1;
+    if (o < 0) (void)hipGetLastError();
+  }
+  return o > 0 || gs_packed_lds(ndof, steps) <= 65536;
+}
+void k_gs_pack(hipStream_t s, const DevLevel &L) {
+  const int64_t n = (int64_t)L.nact * L.gp_slots;
+  if (n > 0)
+    gs_pack_k<<<grid_for(n), kBlock, 0, s>>>(n, L.nact, L.gp_pos, L.gp_rows, L.diag, L.val, L.gp_val, L.gp_inv);
+}
+void k_gs_packed(hipStream_t s, const DevLevel &L, double *x, const double *f, double omega, int kind, int sweeps,
+                 bool zero) {
+  const size_t lds = gs_packed_lds(L.ndof, L.gp_steps);
+  const int both = kind == 3, passes = both ? 2 * sweeps : sweeps;
+  auto *k = L.gp_slots == 32 ? gs_packed_k<2> : gs_packed_k<8>;
+  k<<<1, kBlock, lds, s>>>(L.ndof, L.nact, L.gp_steps, L.gp_start, L.gp_rows, L.gp_col, L.gp_val, L.gp_inv, x, f, omega,
+                           passes, both, zero);
 }
 void k_restrict(hipStream_t s, const DevLevel &F, const DevLevel &C, const double *fine, double *coarse) {
   launch_rows<kRestrict, double, double>(s, F.r_nnz, C.ndof, C.nact, F.r_rowptr, F.r_col,

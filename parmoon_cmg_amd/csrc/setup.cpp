@@ -320,6 +320,33 @@ void build_gs_schedule(const HostLevel &L, bool backward, std::vector<int> &rows
   for (int i = 0; i < na; i++) rows[pos[lev[i]]++] = i;
 }
 
+int build_gs_packed(const HostLevel &L, std::vector<int> &start, std::vector<int> &rows, std::vector<int> &col,
+                    std::vector<int> &pos) {
+  std::vector<int> lev;
+  build_gs_schedule(L, false, rows, lev);
+  start.assign(1, 0);
+  for (size_t k = 0; k + 1 < lev.size(); k++)
+    for (int b = lev[k]; b < lev[k + 1]; b += kGsRows) start.push_back(std::min(b + kGsRows, lev[k + 1]));
+  int longest = 0;
+  for (int i = 0; i < L.nact; i++) longest = std::max(longest, L.rowptr[i + 1] - L.rowptr[i] - 1);
+  const int slots = longest <= 32 ? 32 : longest <= 128 ? 128 : 0;
+  if (!slots) return 0;
+  col.assign((size_t)L.nact * slots, 0);
+  pos.assign((size_t)L.nact * slots, -1);
+  parallel_for(L.nact, [&](int r) {
+    const int i = rows[r];
+    size_t k = (size_t)r * slots;
+    const size_t end = k + slots;
+    for (int j = L.rowptr[i]; j < L.rowptr[i + 1]; j++)
+      if (L.kcol[j] != i) {
+        col[k] = L.kcol[j];
+        pos[k++] = j;
+      }
+    for (; k < end; k++) col[k] = i;
+  });
+  return slots;
+}
+
 // Grid transfer between coarse level and the next finer one: P(i,k) is the
 // value of coarse basis function k at fine node i -- what Prolongate
 // computes cell by cell with the prolongation matrices and the multiplicity
