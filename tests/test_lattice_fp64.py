@@ -108,3 +108,36 @@ def test_small_program_matches_launches(order, m, k0, levels, rot, pre, post, mo
         assert out[0][2:] == out[1][2:]
         assert np.array_equal(out[0][0], out[1][0]) and np.array_equal(out[0][1], out[1][1])
     P.close()
+
+
+# cd3d_matvec / cd3d_matvec_dev through lattice order (from 5 M nonzeros) against
+# CSR: one product of at most 125 terms per row, 1e-13 of the result's norm.
+# What is not the assembled stencil matrix stays with CSR: the mass matrices
+# after cd3d_tcd_init, and entries set by the caller
+@pytest.mark.parametrize("order,m,k0,levels,rot", [(2, 3, 0, 4, 0), (2, 3, 0, 4, 1), (1, 1, 2, 5, 0), (1, 5, 0, 5, 1)])
+def test_matvec_through_the_lattice(order, m, k0, levels, rot, monkeypatch):
+    P = pm.Problem(order, m, k0, levels, box=(1.0, 0.9, 0.8))
+    co = pm.coeffs(eps=0.05, b=(1.0, 0.5, 0.25), conv_kind=rot, rot_c=(0.4, 0.6), f_val=1.0)
+    P.assemble(co)
+    l = levels - 1
+    assert P.info(l)["nnz"] >= 5000000
+    x = np.random.default_rng(7).standard_normal(P.info(l)["ndof"])
+
+    def products():
+        out = []
+        for on in ("1", "0"):
+            monkeypatch.setenv("CD3D_MATVEC_LATTICE", on)
+            out.append(P.matvec(l, x))
+        return out
+
+    y1, y0 = products()
+    assert not np.array_equal(y1, y0) and rel(y1, y0) < 1e-13
+    e = P.csr(l)[2]
+    P.tcd_init(co, 0.0, x)
+    y1, y0 = products()
+    assert np.array_equal(y1, y0)
+    P.assemble(co)
+    P.set_entries(l, 2 * e)
+    y2, y3 = products()
+    assert np.array_equal(y2, y3)
+    P.close()
