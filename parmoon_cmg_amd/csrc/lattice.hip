@@ -249,6 +249,128 @@ __global__ __launch_bounds__(kB) void lat_aff_sweep_k(LatArgs a, LatAff af, cons
                                    f, out, omega);
 }
 
+// The same sweeps (modes kLJacobi, kLDefect and the product kLSpmv) with ZN
+// nodes of a class per thread, one above the other: the stencil entries depend
+// on (X, Y) only, so each is evaluated once for the column (four LDS values
+// and 3-4 operations per entry, against one product per node), and Q1 keeps
+// the column's (ZN + 2) x 9 values of x in registers.  Each node's sum runs in
+// lat_node_aff's order: bitwise the same.  Blocks bstart[nclass].. (counted in
+// columns) take the Dirichlet rows of the product forms (identity).
+// Bound by the entries' evaluation and the x loads, not by HBM (Q1 129^3 nodes,
+// FP32 sweep 19.0 -> 14.5 us for 25.8 MB, FP64 product 29.5 -> 18.8 us; 97^3
+// 9.6 -> 7.9 and 15.5 -> 11.5; Q2 129^3 FP32 44 -> 33 us, FP64 product 175 -> 57
+// us, where the unrolled 125-entry form spilled: the planes are a rolled loop).
+constexpr int kLSpmv = 3;
+// entries S0, SX, SY, mass of one stencil position side by side in LDS
+template <typename T>
+struct AffEntry {
+  T s0, sx, sy, sm;
+};
+template <int P, int PX, int PY, int PZ, int MODE, int ZN, typename T>
+__device__ inline void lat_aff_col(const LatArgs &a, const LatDev &C, unsigned u, const AffEntry<T> *st, T alpha,
+                                   T alpha_m, int centre, const T *__restrict__ x, const T *__restrict__ f,
+                                   T *__restrict__ out, T omega) {
+  const unsigned c0 = (unsigned)C.cnt[0], c1 = (unsigned)C.cnt[1], r = u / c0, rz = r / c1;
+  const int X = C.lo[0] + C.step * (int)(u - r * c0), Y = C.lo[1] + C.step * (int)(r - rz * c1);
+  const int kz = (int)rz * ZN, nz = min(ZN, C.cnt[2] - kz), Z0 = C.lo[2] + C.step * kz;
+  const long long nn = a.nn, n2 = nn * nn, node = X + nn * (Y + nn * Z0);
+  auto entry = [&](int s) {
+    const AffEntry<T> e = st[s];
+    return affine_at(&e.s0, &e.sx, &e.sy, &e.sm, alpha, alpha_m, 0, X, Y);
+  };
+  T s[ZN], xc[ZN];
+  long long zo[ZN];  // node of the column's z-th member (the last one again past the end)
+#pragma unroll
+  for (int z = 0; z < ZN; z++) {
+    s[z] = 0;
+    zo[z] = node + n2 * C.step * (z < nz ? z : nz - 1);
+    xc[z] = MODE == kLJacobi ? x[zo[z]] : T(0);
+  }
+  int si = 0;
+  if constexpr (P == 1) {
+    T w[ZN + 2][3][3];
+#pragma unroll
+    for (int z = 0; z < ZN + 2; z++) {
+      const T *xp = x + node + n2 * (min(z, nz + 1) - 1);
+#pragma unroll
+      for (int dy = 0; dy < 3; dy++)
+#pragma unroll
+        for (int dx = 0; dx < 3; dx++) w[z][dy][dx] = xp[dx - 1 + nn * (dy - 1)];
+    }
+#pragma unroll
+    for (int dz = 0; dz < 3; dz++)
+#pragma unroll
+      for (int dy = 0; dy < 3; dy++)
+#pragma unroll
+        for (int dx = 0; dx < 3; dx++, si++) {
+          const T v = entry(si);
+#pragma unroll
+          for (int z = 0; z < ZN; z++) s[z] += v * w[z + dz][dy][dx];
+        }
+  } else {
+#pragma unroll 1
+    for (int dz = lo_off<P, PZ>(); dz <= hi_off<P, PZ>(); dz++)
+#pragma unroll
+      for (int dy = lo_off<P, PY>(); dy <= hi_off<P, PY>(); dy++)
+#pragma unroll
+        for (int dx = lo_off<P, PX>(); dx <= hi_off<P, PX>(); dx++, si++) {
+          const T v = entry(si);
+#pragma unroll
+          for (int z = 0; z < ZN; z++) s[z] += v * x[zo[z] + dx + nn * dy + n2 * dz];
+        }
+  }
+  const T di = MODE == kLJacobi ? T(1) / entry(centre) : T(0);
+#pragma unroll
+  for (int z = 0; z < ZN; z++)
+    if (z < nz) {
+      const long long o = zo[z];
+      if (MODE == kLSpmv) out[o] = s[z];
+      else if (MODE == kLDefect) out[o] = f[o] - s[z];
+      else out[o] = xc[z] + omega * (f[o] - s[z]) * di;
+    }
+}
+
+template <int P, int MODE, int ZN, typename T>
+__global__ __launch_bounds__(kB) void lat_aff_col_k(LatArgs a, LatAff af, const T *__restrict__ x,
+                                                    const T *__restrict__ f, T *__restrict__ out, T omega, int nact,
+                                                    int ndof, const int *__restrict__ dof2node) {
+  __shared__ AffEntry<T> st[kCst];
+  const int nb = a.bstart[a.nclass];
+  if ((int)blockIdx.x >= nb) {  // Dirichlet rows
+    const int d = nact + (blockIdx.x - nb) * kB + threadIdx.x;
+    if (d < ndof) {
+      const int node = dof2node[d];
+      out[node] = MODE == kLDefect ? f[node] - x[node] : x[node];
+    }
+    return;
+  }
+  const int c = block_class(a.bstart, a.nclass, (int)blockIdx.x);
+  for (int i = threadIdx.x; i < kCst; i += kB)
+    st[i] = AffEntry<T>{(T)af.st[c * kCst + i], (T)af.st[8 * kCst + 8 + c * kCst + i],
+                        (T)af.st[2 * 8 * kCst + 8 + c * kCst + i], af.stm ? (T)af.stm[c * kCst + i] : T(0)};
+  __syncthreads();
+  const LatDev &C = a.c[c];
+  const unsigned u = (blockIdx.x - a.bstart[c]) * kB + threadIdx.x;
+  if (u >= (unsigned)C.cnt[0] * (unsigned)C.cnt[1] * (unsigned)((C.cnt[2] + ZN - 1) / ZN)) return;
+#define CD3D_COL(PX, PY, PZ) \
+  lat_aff_col<P, PX, PY, PZ, MODE, ZN, T>(a, C, u, st, (T)af.alpha, (T)af.alpha_m, af.centre[c], x, f, out, omega)
+  if (P == 1) {
+    CD3D_COL(0, 0, 0);
+  } else {
+    switch (c) {
+      case 0: CD3D_COL(0, 0, 0); break;
+      case 1: CD3D_COL(1, 0, 0); break;
+      case 2: CD3D_COL(0, 1, 0); break;
+      case 3: CD3D_COL(1, 1, 0); break;
+      case 4: CD3D_COL(0, 0, 1); break;
+      case 5: CD3D_COL(1, 0, 1); break;
+      case 6: CD3D_COL(0, 1, 1); break;
+      default: CD3D_COL(1, 1, 1); break;
+    }
+  }
+#undef CD3D_COL
+}
+
 // Q2 sweeps by vertex/midpoint pairs along X.  A thread takes the nodes
 // X0 = 2 ix (cell vertex in X, class (0, py, pz)) and X0 + 1 (cell midpoint,
 // class (1, py, pz)).  Both have the same Y/Z stencil extent, and together
@@ -1821,80 +1943,6 @@ __global__ __launch_bounds__(kB) void lat64_quad_gk(LatArgs a, const double *__r
   }
 }
 
-// FP64 operator of a rotating-field level: entry s of a node (X, Y) is
-// alpha (S0 + X SX + Y SY) (conv-diff alone, alpha 1) or
-// fma(alpha, S0 + X SX + Y SY, M) (the TCD3D system matrix M + tau th1 A),
-// the exact arithmetic of the CSR values (affine_entry in csr_fill_affine_k,
-// then matadd_into_k), so the lattice FGMRES applies the assembled matrix.
-// Class-blocked; blocks bstart[nclass].. take the Dirichlet rows (identity).
-template <int P, int PX, int PY, int PZ, int MODE>
-__host__ __device__ inline void lat64_aff_node(const LatArgs &a, const LatDev &C, long long k, const double *s0,
-                                               const double *sx, const double *sy, const double *sm, double alpha,
-                                               const double *__restrict__ x, const double *__restrict__ f,
-                                               double *__restrict__ out) {
-  int kx, ky, kz;
-  class_coords(C, k, kx, ky, kz);
-  const int X = C.lo[0] + C.step * kx, Y = C.lo[1] + C.step * ky, Z = C.lo[2] + C.step * kz;
-  const long long nn = a.nn, node = X + nn * (Y + nn * Z);
-  double s = 0.0;
-  int si = 0;
-#pragma unroll
-  for (int dz = lo_off<P, PZ>(); dz <= hi_off<P, PZ>(); dz++)
-#pragma unroll
-    for (int dy = lo_off<P, PY>(); dy <= hi_off<P, PY>(); dy++)
-#pragma unroll
-      for (int dx = lo_off<P, PX>(); dx <= hi_off<P, PX>(); dx++, si++) {
-        const double e = fma((double)Y, sy[si], fma((double)X, sx[si], s0[si]));
-        const double v = sm ? fma(alpha, e, sm[si]) : alpha * e;
-        s += v * x[node + dx + nn * (dy + nn * dz)];
-      }
-  out[node] = MODE == kL64Defect ? f[node] - s : s;
-}
-
-template <int P, int MODE>
-__global__ __launch_bounds__(kB) void lat64_aff_k(LatArgs a, LatAff af, const double *__restrict__ x,
-                                                  const double *__restrict__ f, double *__restrict__ out, int nact,
-                                                  int ndof, const int *__restrict__ dof2node) {
-  __shared__ double st[4][kCst];
-  const int nb = a.bstart[a.nclass];
-  if ((int)blockIdx.x >= nb) {  // Dirichlet rows
-    const int d = nact + (blockIdx.x - nb) * kB + threadIdx.x;
-    if (d < ndof) {
-      const int node = dof2node[d];
-      out[node] = MODE == kL64Defect ? f[node] - x[node] : x[node];
-    }
-    return;
-  }
-  const int c = block_class(a.bstart, a.nclass, (int)blockIdx.x);
-  for (int i = threadIdx.x; i < kCst; i += kB) {
-    st[0][i] = af.st[c * kCst + i];
-    st[1][i] = af.st[8 * kCst + 8 + c * kCst + i];
-    st[2][i] = af.st[2 * 8 * kCst + 8 + c * kCst + i];
-    st[3][i] = af.stm ? af.stm[c * kCst + i] : 0.0;
-  }
-  __syncthreads();
-  const long long k = (long long)(blockIdx.x - a.bstart[c]) * kB + threadIdx.x;
-  if (k >= a.c[c].nodes) return;
-  const double *sm = af.stm ? st[3] : nullptr;
-#define CD3D_A64(PX, PY, PZ) \
-  lat64_aff_node<P, PX, PY, PZ, MODE>(a, a.c[c], k, st[0], st[1], st[2], sm, af.alpha, x, f, out)
-  if (P == 1) {
-    CD3D_A64(0, 0, 0);
-  } else {
-    switch (c) {
-      case 0: CD3D_A64(0, 0, 0); break;
-      case 1: CD3D_A64(1, 0, 0); break;
-      case 2: CD3D_A64(0, 1, 0); break;
-      case 3: CD3D_A64(1, 1, 0); break;
-      case 4: CD3D_A64(0, 0, 1); break;
-      case 5: CD3D_A64(1, 0, 1); break;
-      case 6: CD3D_A64(0, 1, 1); break;
-      default: CD3D_A64(1, 1, 1); break;
-    }
-  }
-#undef CD3D_A64
-}
-
 // Dirichlet rows (DOFs nact..ndof-1): identity
 __global__ void lat64_boundary_k(int nact, int ndof, const int *__restrict__ dof2node, const double *__restrict__ x,
                                  const double *__restrict__ f, double *__restrict__ out, int defect) {
@@ -2017,6 +2065,7 @@ static bool lat_quads() {
 // 26.4 / 37.0 us (gmax 2); the 65^3-node level is slower with groups (too
 // few threads).  CD3D_PAIR_GROUP = 1, 2 or 4 forces a size; one that does
 // not divide the pairs per line falls back to 1.
+constexpr long long kAffColNodes = 1 << 19;
 constexpr long long kGroupMinThreads = 1 << 17;
 static int pair_group(const LatArgs &a, int gmax) {
   long long pairs = 0;
@@ -2057,6 +2106,45 @@ static bool all_uni(const LatArgs &a) {
   return true;
 }
 
+// nodes per column of lat_aff_col_k on levels large enough to fill the device
+// with columns: Q1 4 (1 / 2 / 4 per thread, FP32: 129^3 nodes 19.7 / 16.3 / 14.5
+// us, 97^3 9.7 / 8.1 / 7.9, 65^3 4.3 / 4.5 / 4.5), Q2 2 (129^3 45.9 / 33.4 / 37.7,
+// 97^3 22.1 / 17.4 / 22.1, 65^3 7.7 / 9.8 / 11.9).  CD3D_AFF_COL=1|2|4 forces it
+static int aff_col(const LatArgs &a, int order) {
+  long long nodes = 0;
+  for (int c = 0; c < a.nclass; c++) nodes += a.c[c].nodes;
+  const char *e = getenv("CD3D_AFF_COL");
+  return e ? atoi(e) : nodes < kAffColNodes ? 1 : order == 1 ? 4 : 2;
+}
+template <int P, int MODE, int ZN, typename T>
+static void aff_col_launch(hipStream_t s, const DevLevel &L, LatArgs a, const LatAff &af, const T *x, const T *f, T *out,
+                           T omega, int boundary) {
+  int b = 0;
+  for (int c = 0; c < a.nclass; c++) {
+    a.bstart[c] = b;
+    b += (int)(((long long)a.c[c].cnt[0] * a.c[c].cnt[1] * ((a.c[c].cnt[2] + ZN - 1) / ZN) + kB - 1) / kB);
+  }
+  a.bstart[a.nclass] = b;
+  const int g = b + (boundary + kB - 1) / kB;
+  if (g > 0) lat_aff_col_k<P, MODE, ZN, T><<<g, kB, 0, s>>>(a, af, x, f, out, omega, L.nact, L.ndof, L.ldof2node);
+}
+// boundary: Dirichlet rows to apply too (the product forms), 0 for sweeps
+template <int MODE, typename T>
+static void aff_cols(hipStream_t s, const DevLevel &L, int order, const LatAff &af, const T *x, const T *f, T *out,
+                     T omega, int boundary) {
+  const LatArgs a = lat_args(L);
+  const int zn = aff_col(a, order);
+  if (order == 1) {
+    if (zn == 4) aff_col_launch<1, MODE, 4, T>(s, L, a, af, x, f, out, omega, boundary);
+    else if (zn == 2) aff_col_launch<1, MODE, 2, T>(s, L, a, af, x, f, out, omega, boundary);
+    else aff_col_launch<1, MODE, 1, T>(s, L, a, af, x, f, out, omega, boundary);
+  } else {
+    if (zn == 4) aff_col_launch<2, MODE, 4, T>(s, L, a, af, x, f, out, omega, boundary);
+    else if (zn == 2) aff_col_launch<2, MODE, 2, T>(s, L, a, af, x, f, out, omega, boundary);
+    else aff_col_launch<2, MODE, 1, T>(s, L, a, af, x, f, out, omega, boundary);
+  }
+}
+
 // the per-class and per-node values of a level for sweeps of value type T
 template <typename T>
 struct LatVals;
@@ -2083,6 +2171,12 @@ void lat_sweep(hipStream_t s, const DevLevel &L, int order, const T *x, const T 
   if (grid <= 0) return;
   if (v.affine) {
     const LatAff af = lat_aff(L);
+    if constexpr (MODE != kLJacobiZero) {
+      if (sizeof(T) == 8 || aff_col(a, order) > 1) {
+        aff_cols<MODE, T>(s, L, order, af, x, f, out, omega, 0);
+        return;
+      }
+    }
     if (order == 1) lat_aff_sweep_k<1, MODE, T><<<grid, kB, 0, s>>>(a, af, x, f, out, omega);
     else lat_aff_sweep_k<2, MODE, T><<<grid, kB, 0, s>>>(a, af, x, f, out, omega);
     return;
@@ -2356,12 +2450,9 @@ void lat64_apply(hipStream_t s, const DevLevel &L, int order, const double *x, c
   const int grid = a.bstart[L.nclass];
   const int nd = L.ndof - L.nact;
   if (L.lat_aff64) {  // rotating field: interior and Dirichlet rows in one launch
-    LatAff af = lat_aff(L);
-    af.alpha = L.lat_alpha;
-    const int g = grid + (nd + kB - 1) / kB;
-    if (g <= 0) return;
-    if (order == 1) lat64_aff_k<1, MODE><<<g, kB, 0, s>>>(a, af, x, f, out, L.nact, L.ndof, L.ldof2node);
-    else lat64_aff_k<2, MODE><<<g, kB, 0, s>>>(a, af, x, f, out, L.nact, L.ndof, L.ldof2node);
+    // entries alpha (S0 + X SX + Y SY), or fma(alpha, that, M) (the TCD3D system
+    // matrix): the arithmetic of the CSR values
+    aff_cols<MODE == kL64Defect ? kLDefect : kLSpmv, double>(s, L, order, lat_aff(L), x, f, out, 0.0, nd);
     return;
   }
   if (order == 2 && grid > 0 && lat_pairs() && L.nn > kPairMinNN) {  // interior and Dirichlet rows in one launch
@@ -2402,14 +2493,11 @@ void lat64_apply(hipStream_t s, const DevLevel &L, int order, const double *x, c
 
 void kl_affine64_apply(hipStream_t s, const DevLevel &L, int order, double alpha, bool with_mass, const double *x,
                        double *y) {
-  const LatArgs a = lat_args(L);
   LatAff af = lat_aff(L);
   af.alpha = alpha;
+  af.alpha_m = with_mass ? 1.0 : 0.0;
   af.stm = with_mass ? L.lst64 + 3 * 8 * kCst + 8 : nullptr;
-  const int g = a.bstart[L.nclass] + (L.ndof - L.nact + kB - 1) / kB;
-  if (g <= 0) return;
-  if (order == 1) lat64_aff_k<1, kL64Spmv><<<g, kB, 0, s>>>(a, af, x, nullptr, y, L.nact, L.ndof, L.ldof2node);
-  else lat64_aff_k<2, kL64Spmv><<<g, kB, 0, s>>>(a, af, x, nullptr, y, L.nact, L.ndof, L.ldof2node);
+  aff_cols<kLSpmv, double>(s, L, order, af, x, nullptr, y, 0.0, L.ndof - L.nact);
 }
 void kl_spmv64(hipStream_t s, const DevLevel &L, int order, const double *x, double *y) {
   lat64_apply<kL64Spmv>(s, L, order, x, nullptr, y);

@@ -141,3 +141,30 @@ def test_matvec_through_the_lattice(order, m, k0, levels, rot, monkeypatch):
     y2, y3 = products()
     assert np.array_equal(y2, y3)
     P.close()
+
+
+# affine stencils (rotating field) with 1, 2 and 4 nodes of a column per thread:
+# each node's sum in the same order, so bitwise; columns that 2 and 4 do not
+# divide, levels that take columns by themselves (97^3 nodes and more)
+@pytest.mark.parametrize("order,m,k0,levels", [(1, 3, 0, 4), (1, 7, 0, 3), (2, 3, 0, 3), (2, 5, 0, 3), (1, 3, 0, 6)])
+def test_affine_columns_match_single_nodes(order, m, k0, levels, monkeypatch):
+    P = pm.Problem(order, m, k0, levels, box=(1.0, 0.9, 0.8))
+    co = pm.coeffs(eps=1e-2, conv_kind=1, rot_c=(0.45, 0.55), pulse_c=(0.3, 0.5, 0.5), f_val=0.5)
+    u0 = P.interp_pulse(levels - 1, co)
+    monkeypatch.setenv("CD3D_SMALL_NODES", "0")
+    for prec in (pm.FP64, pm.MIXED):
+        sp = pm.solver_params(omega=0.5, pre=2, post=1, rel_tol=1e-10, precision=prec)
+        out = []
+        for zn in ("1", "2", "4", None):
+            if zn:
+                monkeypatch.setenv("CD3D_AFF_COL", zn)
+            else:
+                monkeypatch.delenv("CD3D_AFF_COL")
+            P.assemble(co)
+            x, st = P.solve(sp)
+            P.tcd_init(co, 0.1, u0)
+            u, s2 = P.tcd_step(co, sp, 2e-3)
+            out.append((x, u, st.iterations, s2.iterations))
+        for o in out[1:]:
+            assert o[2:] == out[0][2:] and np.array_equal(o[0], out[0][0]) and np.array_equal(o[1], out[0][1])
+    P.close()
