@@ -852,14 +852,38 @@ __host__ __device__ __attribute__((always_inline)) inline void lat_quad_node(con
   }
 }
 
+// Scalar stencil reads go one cache line after the other: a wave asks for all
+// of the 8 KB (8 classes of kCst values) at once, one lane per 128-byte line,
+// so that a cold stencil is fetched from memory once and not line by line.
+// Nothing waits for the value; it is only held until the wave ends.
+// (FP64 product after other work, 127^3 unknowns with the two permutations:
+// 40.8 us without, 38.7 us with it.)
+__device__ __attribute__((always_inline)) inline double st64_touch(const double *st) {
+  static_assert(8 * kCst * sizeof(double) == 64 * 128, "one line per lane");
+  return st[(threadIdx.x & 63) * 16];
+}
+__device__ __attribute__((always_inline)) inline void st64_touched(double v) {
+#ifdef __HIP_DEVICE_COMPILE__
+  asm volatile("" ::"v"(v));
+#endif
+}
+
 template <int G, int MODE, int TB, typename T>
 __global__ __launch_bounds__(TB) void lat_quad_gk(LatArgs a, const T *__restrict__ cst, const T *__restrict__ x,
                                                   const T *__restrict__ f, T *__restrict__ out, T omega, int xcd) {
-  __shared__ T cs[8 * kCst];
-  for (int i = threadIdx.x; i < 8 * kCst; i += TB) cs[i] = cst[i];
-  __syncthreads();
   const int bid = xcd ? xcd_block(blockIdx.x, gridDim.x) : (int)blockIdx.x;
-  lat_quad_node<G, MODE, T>(a, (long long)bid * TB + threadIdx.x, cs, x, f, out, omega);
+  if constexpr (sizeof(T) == 8) {
+    // FP64 stencils as scalar operands: from LDS each coefficient is a read of
+    // 8 bytes per lane for the one product of a pair per line
+    const double touch = st64_touch(cst);
+    lat_quad_node<G, MODE, T>(a, (long long)bid * TB + threadIdx.x, cst, x, f, out, omega);
+    st64_touched(touch);
+  } else {
+    __shared__ T cs[8 * kCst];
+    for (int i = threadIdx.x; i < 8 * kCst; i += TB) cs[i] = cst[i];
+    __syncthreads();
+    lat_quad_node<G, MODE, T>(a, (long long)bid * TB + threadIdx.x, cs, x, f, out, omega);
+  }
 }
 
 template <int P, int MODE, typename T>
@@ -1886,7 +1910,11 @@ __global__ __launch_bounds__(kB) void lat64_pair_gk(LatArgs a, const double *__r
 
 // The FP64 lattice operator by quads of lines (quad_sums over the FP64
 // compact stencils); blocks from nquad on take the Dirichlet rows (identity).
-// Per node the same sums as lat64_pair_group.  TX = float: x is the FP32
+// Per node the same sums as lat64_pair_group.  The stencils are scalar
+// operands: out of LDS each coefficient was 8 bytes per lane for the one
+// product of a pair per line, and LDS reads bound the kernel (FP64 product:
+// 129^3 nodes 21.2 -> 17.4 us, 193^3 55.7 -> 42.0, 97^3 11.4 -> 9.9).
+// TX = float: x is the FP32
 // V-cycle output, converted exactly, and xcopy (when given) receives x at
 // every node written (every lattice node), the FP32 Krylov column z_i.
 template <int G, int MODE, typename TX = double>
@@ -1895,7 +1923,6 @@ __global__ __launch_bounds__(kB) void lat64_quad_gk(LatArgs a, const double *__r
                                                     double *__restrict__ out, int nquad, int nact, int ndof,
                                                     const int *__restrict__ dof2node, int xcd,
                                                     TX *__restrict__ xcopy = nullptr) {
-  __shared__ double cs[8 * kCst];
   const int bid0 = (int)blockIdx.x;
   if (bid0 >= nquad) {
     const int d = nact + (bid0 - nquad) * kB + threadIdx.x;
@@ -1909,14 +1936,14 @@ __global__ __launch_bounds__(kB) void lat64_quad_gk(LatArgs a, const double *__r
     }
     return;
   }
-  for (int i = threadIdx.x; i < 8 * kCst; i += kB) cs[i] = st64[i];
-  __syncthreads();
   const int bid = xcd ? xcd_block(bid0, nquad) : bid0;
   QuadPos p;
   if (!quad_pos<G>(a, (long long)bid * kB + threadIdx.x, p)) return;
   const long long nn = a.nn;
+  const double touch = st64_touch(st64);
   double s0[4][G], s1[4][G], xs[4][2 * G];
-  quad_sums<double, G, TX>(a, p, cs, x, s0, s1, xs);
+  quad_sums<double, G, TX>(a, p, st64, x, s0, s1, xs);  // (scalar operands)
+  st64_touched(touch);
 #pragma unroll
   for (int pc = 0; pc < 4; pc++) {
     const int oy = pc & 1, oz = pc >> 1;
@@ -2459,8 +2486,8 @@ void lat64_apply(hipStream_t s, const DevLevel &L, int order, const double *x, c
     const int G = pair_group(a, 2);
     if (G > 1 && lat_quads()) {
       // measured on the 129^3-node level (FP64 product): quads of one pair
-      // 21.1 us (XCD mapping or not), of two pairs 22.5 (256 VGPRs, one wave
-      // per SIMD), the pair-class kernel 27.0
+      // 17.4 us (21.1 with the stencils in LDS), of two pairs 22.5 (256 VGPRs,
+      // one wave per SIMD), the pair-class kernel 27.0
       const char *ex = getenv("CD3D_QUAD_XCD"), *eg = getenv("CD3D_QUAD64_G");
       const int xcd = ex ? atoi(ex) : 1, gq = eg ? atoi(eg) : 1;
       const long long n = a.c[1].cnt[0];
