@@ -1518,22 +1518,27 @@ __global__ __launch_bounds__(TS *TS) void gj_small_k(int na, const int *__restri
 // panel's new columns and the multipliers of every other column c,
 //   t_rc' = (r a pivot row of the panel ? 0 : t_rc) - sum_j W_rj t_{p_j c}.
 // The other workgroups of the launch apply panel s - 1 to all other columns,
-// from one buffer into the other (a wave takes 64 columns of kGjUpdRows rows:
-// its pivot-row entries stay in registers, W is read as scalars), so the
+// from one buffer into the other, by FP64 matrix products, so the
 // factorisation of a panel, a serial chain of NB pivots in one workgroup, runs
 // beside the update by the one before.  They write panel s + 1's columns to
 // the compact column-major buffer C, which workgroup 0 of the next launch
 // reads with consecutive lanes on consecutive rows (read from the row-major
 // matrix, each lane on its own cache line, a 2197-row panel took 12 us to load
 // and 12 us to bring up to date).  The last launch writes the inverse itself.
-// Bound by the chain of pivots and the launches; per pivot: column keys (DPP
-// maximum), the wave's candidate row to LDS, one barrier, the best candidate.
-// Whole inversion, with separate panel and update launches over na x 2 na
-// before: 343 unknowns 900 -> 509 us, 1331 7.7 -> 4.0 ms, 2197 19.2 -> 10.2 ms
-// (256-thread workgroups with more rows per thread: 17.7 ms).
+// Per pivot: column keys (DPP maximum), one barrier, the best wave stages its
+// row, one barrier, the exchange step.  Bound by that chain and by the
+// instructions a wave issues in it (0.45 us per pivot and 0.035 us per column
+// of the panel at 343 rows: panels of 32 take 588 us where 16 take 394), so at
+// most kGjThreads threads with the rows in registers, and nothing but the
+// step itself outside the one wave that holds the pivot.  From 2197 unknowns
+// on bound by the update's passes over the matrix, hence wide panels there too.
+// Whole inversion with assembly, 1024-thread workgroups in which every wave
+// staged its candidate and panels of 8 above 2048 rows, and now: 343 unknowns
+// 0.55 -> 0.40 ms, 1331 4.0 -> 2.35 ms, 2197 10.3 -> 5.6 ms.
 constexpr int kGjPanel = 16;        // widest panel
-constexpr int kGjBlockedMax = 4096;  // 4 rows per thread of the panel
-constexpr int kGjUpdRows = 8;        // rows per wave of the update
+constexpr int kGjBlockedMax = 4096;  // 8 rows per thread of the panel
+constexpr int kGjUpdBlocks = 255;    // workgroups of the update
+constexpr int kGjThreads = 512;      // of a workgroup at most
 
 __global__ __launch_bounds__(kBlock) void gj_dense_k(int na, const int *__restrict__ rp, const int *__restrict__ col,
                                                      const double *__restrict__ val, double *__restrict__ M,
@@ -1553,142 +1558,211 @@ __global__ __launch_bounds__(kBlock) void gj_dense_k(int na, const int *__restri
 // column of pivot row r or -1.  (The update looks at iperm for panel kp while
 // workgroup 0 sets entries of panel k0: those rows are -1 or >= k0, not of
 // panel kp either way.)  C: the columns of panel k0 or null (then read from
-// M); Cn: receives those of the panel after it.  Wp, iperm are read up to
-// kGjUpdRows entries past their end (scratch).
+// M); Cn: receives those of the panel after it.  W has zero columns from b on.
+// nt: tiles of 16 rows that a wave of the update takes.
 template <int NB, int RPT>
-__global__ __launch_bounds__(1024) void gj_block_k(int na, int kp, int bp, int k0, int b, const double *__restrict__ M,
-                                                   double *__restrict__ Mo, const double *__restrict__ Wp,
-                                                   double *__restrict__ W, const double *__restrict__ C,
-                                                   double *__restrict__ Cn, int *perm, int *iperm,
-                                                   double *__restrict__ inv, int ncb) {
+__global__ __launch_bounds__(kGjThreads) void gj_block_k(int na, int kp, int bp, int k0, int b,
+                                                         const double *__restrict__ M, double *__restrict__ Mo,
+                                                         const double *__restrict__ Wp, double *__restrict__ W,
+                                                         const double *__restrict__ C, double *__restrict__ Cn,
+                                                         int *perm, int *iperm, double *__restrict__ inv, int ncb,
+                                                         int nt) {
   const int t = threadIdx.x, lane = t & 63, wv = __builtin_amdgcn_readfirstlane(t >> 6), nw = blockDim.x >> 6;
   if (blockIdx.x > 0 || b == 0) {
+    // M' = M - W U by FP64 matrix products of 16 x 16 x 4: the wave's 64
+    // columns of U (the pivot rows, four per product) stay in registers, and
+    // the next tile of 16 rows is on its way while one is multiplied
     const int blk = (int)blockIdx.x - (b ? 1 : 0), cb = blk % ncb, rb = blk / ncb;
-    const int c = cb * 64 + lane, r0 = (rb * nw + wv) * kGjUpdRows;
-    if (c >= na || r0 >= na || (c >= k0 && c < k0 + b)) return;
-    const bool own = c >= kp && c < kp + bp;  // a column of the applied panel: its new values are W
-    const int cn = c - (k0 + NB);             // a column of the next panel: 0 <= cn < NB
-    const int oc = b ? c : perm[c];
-    double u[NB], m[kGjUpdRows];
-    int ir[kGjUpdRows];
+    const int l16 = lane & 15, l4 = lane >> 4, c0 = cb * 64 + l16;
+    typedef double d4 __attribute__((ext_vector_type(4)));
+    constexpr int KS = NB / 4;
+    double u[KS][4];
 #pragma unroll
-    for (int j = 0; j < NB; j++) u[j] = j < bp ? M[(int64_t)perm[kp + j] * na + c] : 0.0;
+    for (int ks = 0; ks < KS; ks++) {
+      const int k = 4 * ks + l4;
+      const double *row = M + (int64_t)perm[kp + min(k, bp - 1)] * na;
 #pragma unroll
-    for (int i = 0; i < kGjUpdRows; i++) {
-      m[i] = M[(int64_t)min(r0 + i, na - 1) * na + c];
-      ir[i] = iperm[r0 + i];
+      for (int ct = 0; ct < 4; ct++) u[ks][ct] = row[min(c0 + 16 * ct, na - 1)];
+#pragma unroll
+      for (int ct = 0; ct < 4; ct++) u[ks][ct] = k < bp ? u[ks][ct] : 0.0;
     }
+    d4 m[4];
+    double w[KS];
+    int ir[4];
+    auto load = [&](int r0, d4 *mm, double *ww, int *ii) {
 #pragma unroll
-    for (int i = 0; i < kGjUpdRows; i++) m[i] = ir[i] >= kp && ir[i] < kp + bp ? 0.0 : m[i];
+      for (int i = 0; i < 4; i++) {
+        const int r = min(r0 + 4 * i + l4, na - 1);
+        ii[i] = iperm[r];
 #pragma unroll
-    for (int j = 0; j < NB; j++) {
-      const double *w = Wp + (int64_t)j * na + r0;  // uniform: scalar loads
+        for (int ct = 0; ct < 4; ct++) mm[ct][i] = M[(int64_t)r * na + min(c0 + 16 * ct, na - 1)];
+      }
 #pragma unroll
-      for (int i = 0; i < kGjUpdRows; i++) m[i] = fma(-w[i], u[j], m[i]);
-    }
+      for (int ks = 0; ks < KS; ks++) ww[ks] = Wp[(int64_t)(4 * ks + l4) * na + min(r0 + l16, na - 1)];
+    };
+    int r0 = (rb * nw + wv) * nt * 16;
+    const int re = min(na, r0 + nt * 16);
+    if (r0 < re) load(r0, m, w, ir);
+#pragma unroll 1
+    for (; r0 < re; r0 += 16) {
+      d4 mn[4];
+      double wn[KS];
+      int in[4];
+      load(r0 + 16, mn, wn, in);  // (past the end: the last row again)
 #pragma unroll
-    for (int i = 0; i < kGjUpdRows; i++) {
-      const int r = r0 + i;
-      if (r >= na) break;
-      const double s = own ? Wp[(int64_t)(c - kp) * na + r] : m[i];
-      if (b == 0) inv[(int64_t)ir[i] * na + oc] = s;
-      else if (cn >= 0 && cn < NB) Cn[(int64_t)cn * na + r] = s;
-      else Mo[(int64_t)r * na + c] = s;
+      for (int i = 0; i < 4; i++) {
+        const bool pr = ir[i] >= kp && ir[i] < kp + bp;
+#pragma unroll
+        for (int ct = 0; ct < 4; ct++) m[ct][i] = pr ? 0.0 : m[ct][i];
+      }
+#pragma unroll
+      for (int ks = 0; ks < KS; ks++)
+#pragma unroll
+        for (int ct = 0; ct < 4; ct++)
+          m[ct] = __builtin_amdgcn_mfma_f64_16x16x4f64(-w[ks], u[ks][ct], m[ct], 0, 0, 0);
+#pragma unroll
+      for (int ct = 0; ct < 4; ct++) {
+        const int c = c0 + 16 * ct, cn = c - (k0 + NB);  // 0 <= cn < NB: a column of the next panel
+        if (c >= na || (c >= k0 && c < k0 + b)) continue;
+        const bool own = c >= kp && c < kp + bp;  // a column of the applied panel: its new values are W
+        const int oc = b ? 0 : perm[c];
+#pragma unroll
+        for (int i = 0; i < 4; i++) {
+          const int r = r0 + 4 * i + l4;
+          if (r >= na) break;
+          const double s = own ? Wp[(int64_t)(c - kp) * na + r] : m[ct][i];
+          if (b == 0) inv[(int64_t)ir[i] * na + oc] = s;
+          else if (cn >= 0 && cn < NB) Cn[(int64_t)cn * na + r] = s;
+          else Mo[(int64_t)r * na + c] = s;
+        }
+      }
+#pragma unroll
+      for (int ct = 0; ct < 4; ct++) m[ct] = mn[ct];
+#pragma unroll
+      for (int ks = 0; ks < KS; ks++) w[ks] = wn[ks];
+#pragma unroll
+      for (int i = 0; i < 4; i++) ir[i] = in[i];
     }
     return;
   }
-  __shared__ double srow[2][16][NB + 1], us[NB][NB];
-  __shared__ unsigned sk[2][16];
-  __shared__ int si[2][16], sp[NB];
+  __shared__ double srow[NB + 1], us[NB][NB];
+  __shared__ unsigned sk[16];
+  __shared__ int sp[NB];
   double v[RPT][NB];
-  bool un[RPT];
+  unsigned un[RPT];  // all ones: row not used yet
+  // the panel's columns from C (column-major) or M
+  const double *B = C ? C : M + k0;
+  const int64_t sr = C ? 1 : na, sj = C ? na : 1;
 #pragma unroll
   for (int q = 0; q < RPT; q++) {
-    const int r = t + q * (int)blockDim.x, ir = r < na ? iperm[r] : 0;
-    un[q] = r < na && ir < 0;
-    const bool pr = r >= na || (ir >= kp && ir < kp + bp);
+    const int r = min(t + q * (int)blockDim.x, na - 1);
+    un[q] = (unsigned)iperm[r];
 #pragma unroll
-    for (int j = 0; j < NB; j++)
-      v[q][j] = pr || j >= b ? 0.0 : C ? C[(int64_t)j * na + r] : M[(int64_t)r * na + k0 + j];
+    for (int j = 0; j < NB; j++) v[q][j] = B[r * sr + (j < b ? j : b - 1) * sj];
+  }
+  // the applied panel's pivot rows at the new panel's columns
+  if (bp)
+    for (int e = t; e < NB * NB; e += blockDim.x) {
+      const int i = e / NB, j = e % NB;
+      us[i][j] = i >= bp || j >= b ? 0.0 : B[perm[kp + i] * sr + j * sj];
+    }
+#pragma unroll
+  for (int q = 0; q < RPT; q++) {
+    const int ir = (int)un[q];
+    const bool in = t + q * (int)blockDim.x < na, pr = !in || (ir >= kp && ir < kp + bp);
+    un[q] = in && ir < 0 ? ~0u : 0u;
+#pragma unroll
+    for (int j = 0; j < NB; j++) v[q][j] = pr || j >= b ? 0.0 : v[q][j];
   }
   if (bp) {
-    // the applied panel's pivot rows at the new panel's columns
-    for (int e = t; e < NB * NB; e += blockDim.x) {
-      const int i = e / NB, j = e % NB, p = i < bp ? perm[kp + i] : 0;
-      us[i][j] = i >= bp || j >= b ? 0.0 : C ? C[(int64_t)j * na + p] : M[(int64_t)p * na + k0 + j];
-    }
+    // rank-NB update, the multipliers of the next kCh pivots on their way
+    // while those of kCh are used
+    constexpr int kCh = RPT <= 3 ? 4 : 2;
+    double w[kCh][RPT];
+#pragma unroll
+    for (int i = 0; i < kCh; i++)
+#pragma unroll
+      for (int q = 0; q < RPT; q++) w[i][q] = Wp[(int64_t)i * na + min(t + q * (int)blockDim.x, na - 1)];
     __syncthreads();
-#pragma unroll 2
-    for (int i = 0; i < NB; i++) {
-      double w[RPT];
+#pragma unroll 1
+    for (int i0 = 0; i0 < NB; i0 += kCh) {
+      double wn[kCh][RPT];
 #pragma unroll
-      for (int q = 0; q < RPT; q++) {
-        const int r = t + q * (int)blockDim.x;
-        w[q] = r < na ? Wp[(int64_t)i * na + r] : 0.0;
-      }
+      for (int i = 0; i < kCh; i++)
 #pragma unroll
-      for (int j = 0; j < NB; j++) {
-        const double uj = us[i][j];
+        for (int q = 0; q < RPT; q++)
+          wn[i][q] = Wp[(int64_t)min(i0 + kCh + i, NB - 1) * na + min(t + q * (int)blockDim.x, na - 1)];
 #pragma unroll
-        for (int q = 0; q < RPT; q++) v[q][j] = fma(-w[q], uj, v[q][j]);
-      }
+      for (int i = 0; i < kCh; i++)
+#pragma unroll
+        for (int j = 0; j < NB; j++) {
+          const double uj = us[i0 + i][j];
+#pragma unroll
+          for (int q = 0; q < RPT; q++) v[q][j] = fma(-w[i][q], uj, v[q][j]);
+        }
+#pragma unroll
+      for (int i = 0; i < kCh; i++)
+#pragma unroll
+        for (int q = 0; q < RPT; q++) w[i][q] = wn[i][q];
     }
   }
   // The pivot column is always column 0: every step moves the columns one
   // place down and the finished one to the end, so the loop stays rolled with
-  // its columns in registers.
+  // its columns in registers.  Only the wave that holds the pivot row stages
+  // it and treats it apart, by branches that are uniform in the wave.
 #pragma unroll 1
   for (int j = 0; j < b; j++) {
-    const int buf = j & 1;
-    // the wave's best unused row of the column; its lane stages the row
     unsigned key = 0;
     int bq = 0;
-    double bx = 1.0;
 #pragma unroll
     for (int q = 0; q < RPT; q++) {
-      const unsigned kq = un[q] ? gj_key(v[q][0]) : 0u;
-      if (q == 0 || kq > key) {
-        key = kq;
-        bq = q;
-        bx = v[q][0];
-      }
+      const unsigned kq = gj_key(v[q][0]) & un[q];
+      if (q > 0) bq = kq > key ? q : bq;
+      key = kq > key ? kq : key;
     }
-    const double bi = 1.0 / bx;  // beside the search
     const unsigned wb = wave_max(key);
     const int wl = __ffsll(__ballot(key == wb)) - 1;
-    if (lane == wl) {
-      sk[buf][wv] = wb;
-      si[buf][wv] = t + bq * (int)blockDim.x;
-      srow[buf][wv][NB] = bi;
-#pragma unroll
-      for (int q = 0; q < RPT; q++)
-        if (q == bq)
-#pragma unroll
-          for (int jj = 0; jj < NB; jj++) srow[buf][wv][jj] = v[q][jj];
-    }
+    const int wq = RPT > 1 ? __builtin_amdgcn_readlane(bq, wl) : 0;
+    if (lane == 0) sk[wv] = wb;
     __syncthreads();
-    const unsigned gk = lane < nw ? sk[buf][lane] : 0u;
+    const unsigned gk = lane < nw ? sk[lane] : 0u;
     const unsigned gb = (unsigned)__builtin_amdgcn_readlane((int)row16_max(gk), 0);  // nw <= 16: the first row of lanes
     const int ps = __ffsll(__ballot(gk == gb)) - 1;
-    const double *g = srow[buf][ps];
-    const int p = si[buf][ps];
-    const double dinv = g[NB];
-    if (t == 0) sp[j] = p;  // (a global store here would be waited for at the next barrier)
+    if (wv == ps) {
+#pragma unroll
+      for (int q = 0; q < RPT; q++)
+        if (q == wq) {
+          const double d = 1.0 / v[q][0];
+          if (lane == wl) {
+            srow[NB] = d;
+            sp[j] = t + q * (int)blockDim.x;  // (a global store here would be waited for at the next barrier)
+#pragma unroll
+            for (int jj = 1; jj < NB; jj++) srow[jj] = v[q][jj];
+          }
+        }
+    }
+    __syncthreads();
+    const double dinv = srow[NB];
     double f[RPT];
 #pragma unroll
-    for (int q = 0; q < RPT; q++) {
+    for (int q = 0; q < RPT; q++) f[q] = v[q][0] * dinv;
+    if (wv == ps) {
       // row p: t_pj' = -g_j / d, the others t_ij - f g_j
-      const bool pr = t + q * (int)blockDim.x == p;
-      f[q] = pr ? dinv : v[q][0] * dinv;
-      if (pr) {
-        un[q] = false;
+      const bool pr = lane == wl;
 #pragma unroll
-        for (int jj = 1; jj < NB; jj++) v[q][jj] = 0.0;
-      }
+      for (int q = 0; q < RPT; q++)
+        if (q == wq) {
+          if (pr) {
+            f[q] = dinv;
+            un[q] = 0u;
+#pragma unroll
+            for (int jj = 1; jj < NB; jj++) v[q][jj] = 0.0;
+          }
+        }
     }
 #pragma unroll
     for (int jj = 1; jj < NB; jj++) {
-      const double gj = g[jj];
+      const double gj = srow[jj];
 #pragma unroll
       for (int q = 0; q < RPT; q++) v[q][jj - 1] = fma(-f[q], gj, v[q][jj]);
     }
@@ -2245,8 +2319,12 @@ void k_hconv_geo(hipStream_t s, const DevLevel &L, const double *tab, const AsmP
 template <int NB, int RPT>
 void gj_blocked(hipStream_t s, int na, double *M, double *M1, double *W, double *W1, double *C, double *C1, int *perm,
                 int *iperm, double *inv) {
-  const int bd = RPT == 1 ? (na + 63) / 64 * 64 : 1024, ncb = (na + 63) / 64;
-  const int nrb = (na + bd / 64 * kGjUpdRows - 1) / (bd / 64 * kGjUpdRows), upd = ncb * nrb;
+  const int bd = ((na + RPT - 1) / RPT + 63) / 64 * 64, ncb = (na + 63) / 64;
+  // tiles of 16 rows per wave so that the update is resident at once
+  const int nw = bd / 64, rows = (na + 15) / 16;
+  int nt = 1;
+  while (ncb * ((rows + nw * nt - 1) / (nw * nt)) > kGjUpdBlocks && nt < rows) nt++;
+  const int upd = ncb * ((rows + nw * nt - 1) / (nw * nt));
   const double *Mi = M;
   double *Mo = M1, *Wi = W1, *Wo = W, *Ci = C1, *Co = C;
   int kp = 0, bp = 0, step = 0;
@@ -2254,7 +2332,7 @@ void gj_blocked(hipStream_t s, int na, double *M, double *M1, double *W, double 
     const int b = std::min(NB, na - k0);
     // the first two panels are still unchanged in M
     gj_block_k<NB, RPT><<<bp ? 1 + upd : 1, bd, 0, s>>>(na, kp, bp, k0, b, Mi, Mo, Wi, Wo, step > 1 ? Ci : nullptr, Co,
-                                                        perm, iperm, inv, ncb);
+                                                        perm, iperm, inv, ncb, nt);
     if (bp) {
       double *o = Mo;
       Mo = o == M1 ? M : M1;
@@ -2265,7 +2343,8 @@ void gj_blocked(hipStream_t s, int na, double *M, double *M1, double *W, double 
     kp = k0;
     bp = b;
   }
-  gj_block_k<NB, RPT><<<upd, bd, 0, s>>>(na, kp, bp, na, 0, Mi, Mo, Wi, Wo, nullptr, nullptr, perm, iperm, inv, ncb);
+  gj_block_k<NB, RPT><<<upd, bd, 0, s>>>(na, kp, bp, na, 0, Mi, Mo, Wi, Wo, nullptr, nullptr, perm, iperm, inv, ncb,
+                                         nt);
 }
 
 // CD3D_GJ_UNBLOCKED=1: one launch per pivot also for large blocks (comparison runs)
@@ -2294,11 +2373,16 @@ void k_invert_active(hipStream_t s, const DevLevel &L, double *scratch, double *
     double *M = scratch, *M1 = M + na2, *W = M1 + na2, *W1 = W + pn, *C = W1 + pn, *C1 = C + pn;
     int *perm = (int *)(C1 + pn), *iperm = perm + na;
     gj_dense_k<<<nblk, kBlock, 0, s>>>(na, L.rowptr, L.col, L.val, M, iperm);
-    const int rpt = (na + 1023) / 1024;
-    if (rpt == 1) gj_blocked<16, 1>(s, na, M, M1, W, W1, C, C1, perm, iperm, inv);
-    else if (rpt == 2) gj_blocked<16, 2>(s, na, M, M1, W, W1, C, C1, perm, iperm, inv);
-    else if (rpt == 3) gj_blocked<8, 3>(s, na, M, M1, W, W1, C, C1, perm, iperm, inv);
-    else gj_blocked<8, 4>(s, na, M, M1, W, W1, C, C1, perm, iperm, inv);
+    auto run = [&](auto f) { f(s, na, M, M1, W, W1, C, C1, perm, iperm, inv); };
+    // as few threads as hold the rows; 16 columns of more than five rows do not
+    // fit the 256 registers of a thread
+    const int rpt = (na + kGjThreads - 1) / kGjThreads;
+    if (rpt == 1) run(gj_blocked<16, 1>);
+    else if (rpt == 2) run(gj_blocked<16, 2>);
+    else if (rpt == 3) run(gj_blocked<16, 3>);
+    else if (rpt == 4) run(gj_blocked<16, 4>);
+    else if (rpt == 5) run(gj_blocked<16, 5>);
+    else run(gj_blocked<8, 8>);
     return;
   }
   // scratch: M (2 na^2 doubles), two partial (value, index) buffers, used[na], perm[na]

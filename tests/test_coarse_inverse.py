@@ -53,3 +53,20 @@ def test_coarse_inverse_sizes(order, m, na):
         # an explicit inverse's residual grows with the condition number; partial pivoting adds a growth factor
         assert res < 1e-13 * na * cond
     P.close()
+
+
+@pytest.mark.parametrize("order,m,na", [(1, 9, 512), (2, 6, 1331), (1, 15, 2744)])
+def test_coarse_inverse_rows_per_thread(order, m, na):
+    """Panels with one row per thread and every thread used, with three, and
+    the narrow ones of more than five; bound as above."""
+    P = pm.Problem(order, m, 0, 1, box=(1.0, 0.8, 0.6))
+    i = P.info(0)
+    assert i["nact"] == na
+    P.assemble(pm.coeffs(eps=1e-3, b=(1.0, -0.4, 0.3), c=0.5, supg=1, f_val=1.0))
+    r = np.random.default_rng(5).standard_normal(i["ndof"])
+    r[na:] = 0.0
+    z = P.vcycle(pm.solver_params(coarse_smoother=17), r)
+    res = np.linalg.norm(P.matvec(0, z) - r) / np.linalg.norm(r)
+    print(f"[gpu] coarse inverse na={na}: |A z - r| / |r| = {res:.2e}", flush=True)
+    assert res < 1e-12
+    P.close()
