@@ -937,6 +937,28 @@ __device__ inline double hconv_brick(const double *h, double b0, double b1, doub
   return 2 * nb / den;
 }
 
+// physical point of a brick cell at the reference coordinates r
+__device__ inline void brick_point(const AsmParams &ap, int P, const int4 &cg, const int *dax, const int *sg,
+                                   const double *r, double *X) {
+  const int O[3] = {cg.x, cg.y, cg.z};
+#pragma unroll
+  for (int a = 0; a < 3; a++) {
+    const double xa = ap.dn[dax[a]] * (O[dax[a]] + P * sg[a] * (r[a] + 1) * 0.5);
+    X[0] = dax[a] == 0 ? xa : X[0];
+    X[1] = dax[a] == 1 ? xa : X[1];
+    X[2] = dax[a] == 2 ? xa : X[2];
+  }
+}
+// the source of the manufactured solution sin(pi x) sin(pi y) sin(pi z)
+__device__ inline double manufactured_f(const AsmParams &ap, const double *X, double b0, double b1, double b2) {
+  const double sx = sin(M_PI * X[0]), sy = sin(M_PI * X[1]), sz = sin(M_PI * X[2]);
+  const double cx = cos(M_PI * X[0]), cy = cos(M_PI * X[1]), cz = cos(M_PI * X[2]), u = sx * sy * sz;
+  return ap.eps * 3 * M_PI * M_PI * u + b0 * M_PI * cx * sy * sz + b1 * M_PI * sx * cy * sz + b2 * M_PI * sx * sy * cz +
+         ap.c * u;
+}
+// cells that the kBlock consecutive rows of a block can touch
+constexpr int cells_of_block(int NB) { return (kBlock + NB - 2) / NB + 1; }
+
 // One thread per (cell, local row i); the NB rows of a cell are consecutive
 // threads of a flat index (cells may straddle wavefronts: threads share
 // nothing).  Per quadrature point the thread evaluates the coefficients at
@@ -957,8 +979,13 @@ __device__ inline double hconv_brick(const double *h, double b0, double b1, doub
 // LDS_TAB: the per-thread operands (phi_i and its gradient at every q) are
 // read from an LDS copy of the basis table made at the start of the block;
 // otherwise from the table in global memory.  VAR: coefficients that vary
-// over the cell (rotating convection, manufactured source); without it the
-// kernel carries none of their code (and none of its registers).
+// over the cell (rotating convection, manufactured source, the caller's
+// values); without it the kernel carries none of their code (and none of its
+// registers).  The block first evaluates beta, the SUPG delta (a tanh, three
+// divisions) and the source once per point of its cells into LDS; evaluated by
+// each of a cell's NB rows they were most of the kernel (rotating field with
+// SUPG, Q2 24^3 and its three coarser levels 883 -> 476 us; manufactured
+// source, Q1 16^3, 143 -> 81 us).
 template <int P, bool LDS_TAB, bool VAR>
 __global__ __launch_bounds__(kBlock) void assemble_k(int ncells, const int *__restrict__ list,
                                                      const int4 *__restrict__ cells, const int *__restrict__ slots,
@@ -975,13 +1002,66 @@ __global__ __launch_bounds__(kBlock) void assemble_k(int ncells, const int *__re
     __syncthreads();
   }
   const int64_t gid = (int64_t)blockIdx.x * kBlock + threadIdx.x;
+  const double nu = 1.0 / P;
+  // VAR: beta, the SUPG delta and the source at the points of the block's cells
+  constexpr int MC = cells_of_block(NB);
+  __shared__ double s_hc[VAR ? MC : 1], s_pt[VAR ? MC * NQ : 1][VAR ? 5 : 1];
+  const int c_lo = (int)((int64_t)blockIdx.x * kBlock / NB);
+  if constexpr (VAR) {
+    const int nc = min(ncells - c_lo, (int)(((int64_t)(blockIdx.x + 1) * kBlock - 1) / NB) - c_lo + 1);
+    const bool vary = ap.qp || ap.conv_kind == 1;
+    auto conv = [&](int c, int q, const int4 &cg, const int *dax, const int *sg, double *X, double *b) {
+      if (ap.conv_kind == 1 || ap.f_kind == 1) brick_point(ap, P, cg, dax, sg, tab + q * STRIDE + 1, X);
+      if (ap.qp) {
+        const double *cq = ap.qp + ((int64_t)c * NQ + q) * 6;
+        for (int d = 0; d < 3; d++) b[d] = cq[1 + d];
+      } else if (ap.conv_kind == 1) {
+        b[0] = -(X[1] - ap.rot_c[1]);
+        b[1] = X[0] - ap.rot_c[0];
+        b[2] = 0.1 * ap.sin2pit;
+      } else {
+        for (int d = 0; d < 3; d++) b[d] = ap.b[d];
+      }
+    };
+    if (vary && ap.supg) {  // mesh size in convection direction, b at the first point
+      for (int e = threadIdx.x; e < nc; e += kBlock) {
+        const int c = list ? list[c_lo + e] : c_lo + e;
+        const int4 cg = cells[c];
+        int dax[3], sg[3];
+        decode_frame(cg.w, dax, sg);
+        double X[3] = {0, 0, 0}, b[3];
+        conv(c, 0, cg, dax, sg, X, b);
+        s_hc[e] = hconv_brick(ap.h, b[0], b[1], b[2]);
+      }
+      __syncthreads();
+    }
+    for (int e = threadIdx.x; e < nc * NQ; e += kBlock) {
+      const int lc = e / NQ, q = e % NQ, c = list ? list[c_lo + lc] : c_lo + lc;
+      const int4 cg = cells[c];
+      int dax[3], sg[3];
+      decode_frame(cg.w, dax, sg);
+      double X[3] = {0, 0, 0}, b[3];
+      conv(c, q, cg, dax, sg, X, b);
+      if (vary) {
+#pragma unroll
+        for (int a = 0; a < 3; a++) {
+          const double h = dax[a] == 0 ? ap.h[0] : dax[a] == 1 ? ap.h[1] : ap.h[2];
+          s_pt[e][a] = sg[a] * (dax[a] == 0 ? b[0] : dax[a] == 1 ? b[1] : b[2]) * (2.0 / h);
+        }
+        if (ap.supg)
+          s_pt[e][3] = sdfem_delta(s_hc[lc], ap.qp ? ap.qp[((int64_t)c * NQ + q) * 6] : ap.eps,
+                                   sqrt(b[0] * b[0] + b[1] * b[1] + b[2] * b[2]), nu);
+      }
+      if (!ap.qp && ap.f_kind == 1) s_pt[e][4] = manufactured_f(ap, X, b[0], b[1], b[2]);
+    }
+    __syncthreads();
+  }
   if (gid >= (int64_t)ncells * NB) return;
   const int ci = (int)(gid / NB), i = (int)(gid % NB);
   const int c = list ? list[ci] : ci;
   const int4 cg = cells[c];
   int dax[3], sg[3];
   decode_frame(cg.w, dax, sg);
-  const int O[3] = {cg.x, cg.y, cg.z};
   const double detj = (ap.h[0] / 2) * (ap.h[1] / 2) * (ap.h[2] / 2);
   // per local axis a: 2 / h along the physical axis dax[a] (J^-T of the brick)
   double ih[3], kap[3];
@@ -991,7 +1071,6 @@ __global__ __launch_bounds__(kBlock) void assemble_k(int ncells, const int *__re
     ih[a] = 2.0 / h;
     kap[a] = ap.eps * 4.0 / (h * h);
   }
-  const double nu = 1.0 / P;
   // constant convection: beta and delta are the same at every point
   double beta[3] = {0, 0, 0};
   if (ap.conv_kind == 0) {
@@ -1005,60 +1084,31 @@ __global__ __launch_bounds__(kBlock) void assemble_k(int ncells, const int *__re
 #pragma unroll
   for (int j = 0; j < NB; j++) acc[j] = 0;
   double racc = 0;
-  double hconv = -1;
   for (int q = 0; q < NQ; q++) {
     const double *T = tab + q * STRIDE;
     const double *Ti = LDS_TAB ? s_tab + (q * NB + i) * 4 : T + 4 + 4 * i;
     const double w = T[0] * detj;
     const double phi_i = Ti[0], g0 = Ti[1], g1 = Ti[2], g2 = Ti[3];
-    // physical quadrature point (only variable coefficients need it)
-    double X[3] = {0, 0, 0};
-    if (VAR && (ap.conv_kind == 1 || ap.f_kind == 1)) {
-#pragma unroll
-      for (int a = 0; a < 3; a++) {
-        const double xa = ap.dn[dax[a]] * (O[dax[a]] + P * sg[a] * (T[1 + a] + 1) * 0.5);
-        X[0] = dax[a] == 0 ? xa : X[0];
-        X[1] = dax[a] == 1 ? xa : X[1];
-        X[2] = dax[a] == 2 ? xa : X[2];
-      }
-    }
-    double b0 = ap.b[0], b1 = ap.b[1], b2 = ap.b[2], cr = ap.c;
+    double cr = ap.c, f = ap.f_val;
     double delta = ap.supg ? ap.delta_const : 0.0;
-    double f = ap.f_val;
-    if (VAR && ap.qp) {
-      // the caller's CoeffFct3D values at this point
-      const double *cq = ap.qp + ((int64_t)c * NQ + q) * 6;
-      const double eps = cq[0];
-      b0 = cq[1];
-      b1 = cq[2];
-      b2 = cq[3];
-      cr = cq[4];
-      f = cq[5];
+    if constexpr (VAR) {
+      const double *pt = s_pt[(ci - c_lo) * NQ + q];
+      if (ap.qp) {
+        // the caller's CoeffFct3D values at this point
+        const double *cq = ap.qp + ((int64_t)c * NQ + q) * 6;
+        const double eps = cq[0];
+        cr = cq[4];
+        f = cq[5];
 #pragma unroll
-      for (int a = 0; a < 3; a++) {
-        kap[a] = eps * ih[a] * ih[a];
-        beta[a] = sg[a] * (dax[a] == 0 ? b0 : dax[a] == 1 ? b1 : b2) * ih[a];
+        for (int a = 0; a < 3; a++) kap[a] = eps * ih[a] * ih[a];
+      } else if (ap.f_kind == 1) {
+        f = pt[4];
       }
-      if (ap.supg) {
-        if (hconv < 0) hconv = hconv_brick(ap.h, b0, b1, b2);
-        delta = sdfem_delta(hconv, eps, sqrt(b0 * b0 + b1 * b1 + b2 * b2), nu);
-      }
-    } else if (VAR && ap.conv_kind == 1) {
-      b0 = -(X[1] - ap.rot_c[1]);
-      b1 = X[0] - ap.rot_c[0];
-      b2 = 0.1 * ap.sin2pit;
+      if (ap.qp || ap.conv_kind == 1) {
 #pragma unroll
-      for (int a = 0; a < 3; a++) beta[a] = sg[a] * (dax[a] == 0 ? b0 : dax[a] == 1 ? b1 : b2) * ih[a];
-      if (ap.supg) {
-        if (hconv < 0) hconv = hconv_brick(ap.h, b0, b1, b2);
-        delta = sdfem_delta(hconv, ap.eps, sqrt(b0 * b0 + b1 * b1 + b2 * b2), nu);
+        for (int a = 0; a < 3; a++) beta[a] = pt[a];
+        if (ap.supg) delta = pt[3];
       }
-    }
-    if (VAR && !ap.qp && ap.f_kind == 1) {
-      const double sx = sin(M_PI * X[0]), sy = sin(M_PI * X[1]), sz = sin(M_PI * X[2]);
-      const double cx = cos(M_PI * X[0]), cy = cos(M_PI * X[1]), cz = cos(M_PI * X[2]), u = sx * sy * sz;
-      f = ap.eps * 3 * M_PI * M_PI * u + b0 * M_PI * cx * sy * sz + b1 * M_PI * sx * cy * sz +
-          b2 * M_PI * sx * sy * cz + ap.c * u;
     }
     const double bg = beta[0] * g0 + beta[1] * g1 + beta[2] * g2;
     const double ti = phi_i + delta * bg;
@@ -1107,7 +1157,9 @@ __global__ __launch_bounds__(kBlock) void assemble_k(int ncells, const int *__re
 // so a_i = w |det| (eps K^T (K g_i) + t_i beta), beta = K^T b,
 // t_i = phi_i + delta beta . g_i keep the brick kernel's form
 // A_ij += a_i . g_j + c_i phi_j.  The SUPG delta uses the cell's mesh size in
-// convection direction from hconv[c] (hconv_geo_k, run before).
+// convection direction from hconv[c] (hconv_geo_k, run before).  The geometry
+// is evaluated once per point of the block's cells, a chunk of points at a
+// time, into LDS (by each of a cell's rows: Q2 48^3 2.83 ms, so 2.20 ms).
 template <int P, bool VAR>
 __global__ __launch_bounds__(kBlock) void assemble_geo_k(int ncells, const int *__restrict__ list,
                                                          const int4 *__restrict__ cells, const int *__restrict__ slots,
@@ -1118,63 +1170,95 @@ __global__ __launch_bounds__(kBlock) void assemble_geo_k(int ncells, const int *
   constexpr int N1 = P + 2;
   constexpr int NQ = N1 * N1 * N1;
   constexpr int STRIDE = 4 + 4 * NB;
+  // K, w, beta (and, VAR, delta and f) at QC points at a time of the block's cells
+  constexpr int MC = cells_of_block(NB), QC = P == 1 ? 9 : 16, NV = VAR ? 15 : 13;
+  static_assert(NQ % QC == 0, "whole chunks of points");
+  __shared__ double s_pt[MC * QC][NV];
   const int64_t gid = (int64_t)blockIdx.x * kBlock + threadIdx.x;
-  if (gid >= (int64_t)ncells * NB) return;
-  const int ci = (int)(gid / NB), i = (int)(gid % NB);
+  const int c_lo = (int)((int64_t)blockIdx.x * kBlock / NB);
+  const int nc = min(ncells - c_lo, (int)(((int64_t)(blockIdx.x + 1) * kBlock - 1) / NB) - c_lo + 1);
+  const bool row_on = gid < (int64_t)ncells * NB;  // (the other threads only help with the points)
+  const int ci = row_on ? (int)(gid / NB) : c_lo, i = (int)(gid % NB);
   const int c = list ? list[ci] : ci;
-  TriMap M;
-  tri_load(ap.vx, ap.nv, cells[c], P, M);
   const double nu = 1.0 / P;
-  const double hc = ap.supg ? ap.hconv[c] : 0.0;
   // constant coefficients: one delta per cell
   double delta_c = 0.0;
   if (!VAR && ap.supg)
-    delta_c = sdfem_delta(hc, ap.eps, sqrt(ap.b[0] * ap.b[0] + ap.b[1] * ap.b[1] + ap.b[2] * ap.b[2]), nu);
+    delta_c = sdfem_delta(ap.hconv[c], ap.eps, sqrt(ap.b[0] * ap.b[0] + ap.b[1] * ap.b[1] + ap.b[2] * ap.b[2]), nu);
   double acc[NB];
 #pragma unroll
   for (int j = 0; j < NB; j++) acc[j] = 0;
   double racc = 0;
+  auto points = [&](int q0) {
+    for (int e = threadIdx.x; e < nc * QC; e += kBlock) {
+      const int lc = e / QC, q = q0 + e % QC, cp = list ? list[c_lo + lc] : c_lo + lc;
+      const double *T = tab + q * STRIDE;
+      TriMap M;
+      tri_load(ap.vx, ap.nv, cells[cp], P, M);
+      double b0 = ap.b[0], b1 = ap.b[1], b2 = ap.b[2];
+      if (VAR) {
+        double X[3] = {0, 0, 0}, eps = ap.eps;
+        if (ap.conv_kind == 1 || ap.f_kind == 1) tri_point(M, T[1], T[2], T[3], X);
+        if (ap.qp) {
+          const double *cq = ap.qp + ((int64_t)cp * NQ + q) * 6;
+          eps = cq[0];
+          b0 = cq[1];
+          b1 = cq[2];
+          b2 = cq[3];
+        } else if (ap.conv_kind == 1) {
+          b0 = -(X[1] - ap.rot_c[1]);
+          b1 = X[0] - ap.rot_c[0];
+          b2 = 0.1 * ap.sin2pit;
+        }
+        if (!ap.qp && ap.f_kind == 1) s_pt[e][NV - 1] = manufactured_f(ap, X, b0, b1, b2);
+        if (ap.supg) s_pt[e][NV - 2] = sdfem_delta(ap.hconv[cp], eps, sqrt(b0 * b0 + b1 * b1 + b2 * b2), nu);
+      }
+      double K[3][3];
+      const double det = tri_jac(M, T[1], T[2], T[3], K);
+      const double rd = 1.0 / det;
+#pragma unroll
+      for (int d = 0; d < 3; d++)
+#pragma unroll
+        for (int x = 0; x < 3; x++) {
+          K[d][x] *= rd;
+          s_pt[e][3 * d + x] = K[d][x];
+        }
+      s_pt[e][9] = T[0] * fabs(det);
+#pragma unroll
+      for (int x = 0; x < 3; x++) s_pt[e][10 + x] = b0 * K[0][x] + b1 * K[1][x] + b2 * K[2][x];
+    }
+  };
   for (int q = 0; q < NQ; q++) {
+    if (q % QC == 0) {
+      __syncthreads();
+      points(q);
+      __syncthreads();
+    }
+    const double *pt = s_pt[(ci - c_lo) * QC + q % QC];
     const double *T = tab + q * STRIDE;
     const double *Ti = T + 4 + 4 * i;
     const double phi_i = Ti[0], g0 = Ti[1], g1 = Ti[2], g2 = Ti[3];
-    double eps = ap.eps, b0 = ap.b[0], b1 = ap.b[1], b2 = ap.b[2], cr = ap.c, f = ap.f_val;
+    double eps = ap.eps, cr = ap.c, f = ap.f_val;
     double delta = delta_c;
     if (VAR) {
-      double X[3] = {0, 0, 0};
-      if (ap.conv_kind == 1 || ap.f_kind == 1) tri_point(M, T[1], T[2], T[3], X);
       if (ap.qp) {
         const double *cq = ap.qp + ((int64_t)c * NQ + q) * 6;
         eps = cq[0];
-        b0 = cq[1];
-        b1 = cq[2];
-        b2 = cq[3];
         cr = cq[4];
         f = cq[5];
-      } else if (ap.conv_kind == 1) {
-        b0 = -(X[1] - ap.rot_c[1]);
-        b1 = X[0] - ap.rot_c[0];
-        b2 = 0.1 * ap.sin2pit;
+      } else if (ap.f_kind == 1) {
+        f = pt[NV - 1];
       }
-      if (!ap.qp && ap.f_kind == 1) {
-        const double sx = sin(M_PI * X[0]), sy = sin(M_PI * X[1]), sz = sin(M_PI * X[2]);
-        const double cx = cos(M_PI * X[0]), cy = cos(M_PI * X[1]), cz = cos(M_PI * X[2]), u = sx * sy * sz;
-        f = ap.eps * 3 * M_PI * M_PI * u + b0 * M_PI * cx * sy * sz + b1 * M_PI * sx * cy * sz +
-            b2 * M_PI * sx * sy * cz + ap.c * u;
-      }
-      if (ap.supg) delta = sdfem_delta(hc, eps, sqrt(b0 * b0 + b1 * b1 + b2 * b2), nu);
+      if (ap.supg) delta = pt[NV - 2];
     }
-    double K[3][3];
-    const double det = tri_jac(M, T[1], T[2], T[3], K);
-    const double rd = 1.0 / det;
+    double K[3][3], beta[3];
 #pragma unroll
     for (int d = 0; d < 3; d++)
 #pragma unroll
-      for (int a = 0; a < 3; a++) K[d][a] *= rd;
-    const double w = T[0] * fabs(det);
-    double beta[3];
+      for (int a = 0; a < 3; a++) K[d][a] = pt[3 * d + a];
+    const double w = pt[9];
 #pragma unroll
-    for (int a = 0; a < 3; a++) beta[a] = b0 * K[0][a] + b1 * K[1][a] + b2 * K[2][a];
+    for (int a = 0; a < 3; a++) beta[a] = pt[10 + a];
     const double bg = beta[0] * g0 + beta[1] * g1 + beta[2] * g2;
     const double ti = phi_i + delta * bg;
     if (ap.what == 1) {  // mass; rhs with the SUPG test function
@@ -1202,6 +1286,7 @@ __global__ __launch_bounds__(kBlock) void assemble_geo_k(int ncells, const int *
       acc[j] = fma(a[0], T[5 + 4 * j], fma(a[1], T[6 + 4 * j], fma(a[2], T[7 + 4 * j], fma(cc, T[4 + 4 * j], acc[j]))));
     racc += w * f * ti;
   }
+  if (!row_on) return;
   if (ap.E) {  // two-pass assembly: the element row, contiguously
     const int64_t row = (int64_t)c * NB + i;
 #pragma unroll
