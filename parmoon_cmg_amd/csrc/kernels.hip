@@ -956,13 +956,70 @@ __device__ inline double manufactured_f(const AsmParams &ap, const double *X, do
   return ap.eps * 3 * M_PI * M_PI * u + b0 * M_PI * cx * sy * sz + b1 * M_PI * sx * cy * sz + b2 * M_PI * sx * sy * cz +
          ap.c * u;
 }
-// cells that the kBlock consecutive rows of a block can touch
-constexpr int cells_of_block(int NB) { return (kBlock + NB - 2) / NB + 1; }
+// A block takes kElemRows consecutive element rows, one per lane; its waves
+// share the quadrature points (point q: wave q mod kElemWaves)
+constexpr int kElemRows = 64, kElemWaves = kBlock / 64;
+// cells that they can touch
+constexpr int cells_of_block(int NB) { return (kElemRows + NB - 2) / NB + 1; }
+static_assert(kElemWaves == 4, "element_rows_out adds four waves");
+// LDS doubles of element_rows_out, and of a block with pt of them for its points
+constexpr int elem_lds(int NB, int pt) {
+  return pt > 2 * (NB + 1) * (kElemRows + 1) ? pt : 2 * (NB + 1) * (kElemRows + 1);
+}
 
-// One thread per (cell, local row i); the NB rows of a cell are consecutive
-// threads of a flat index (cells may straddle wavefronts: threads share
-// nothing).  Per quadrature point the thread evaluates the coefficients at
-// the point and forms, in the cell's reference frame,
+// The sum of the four waves' rows, ((0 + 2) + (1 + 3)), then the rows into the
+// element-row buffers (in order: whole lines) or through the slot map into CSR.
+template <int NB>
+__device__ __forceinline__ void element_rows_out(double *acc, double racc, int wv, int lane, int64_t row_lo,
+                                                 int64_t nrows, const int *__restrict__ list,
+                                                 const int *__restrict__ slots, const int *__restrict__ gn, int nact,
+                                                 const AsmParams &ap, double *__restrict__ val,
+                                                 double *__restrict__ rhs, double *lds) {
+  double(*red)[NB + 1][kElemRows + 1] = (double(*)[NB + 1][kElemRows + 1]) lds;
+  __syncthreads();  // the points in the same LDS are read
+  auto put = [&](int b) {
+#pragma unroll
+    for (int j = 0; j < NB; j++) red[b][j][lane] = acc[j];
+    red[b][NB][lane] = racc;
+  };
+  auto add = [&](int b) {
+#pragma unroll
+    for (int j = 0; j < NB; j++) acc[j] += red[b][j][lane];
+    racc += red[b][NB][lane];
+  };
+  if (wv >= 2) put(wv - 2);
+  __syncthreads();
+  if (wv < 2) add(wv);
+  if (wv == 1) put(1);
+  __syncthreads();
+  if (wv == 0) {
+    add(1);
+    put(0);
+  }
+  __syncthreads();
+  for (int e = threadIdx.x; e < kElemRows * NB; e += kBlock) {
+    const int lr = e / NB, j = e % NB;
+    const int64_t gid = row_lo + lr;
+    if (gid >= nrows) break;
+    const int ci = (int)(gid / NB), i = (int)(gid % NB);
+    const int64_t row = (int64_t)(list ? list[ci] : ci) * NB + i;
+    const double v = red[0][j][lr];
+    if (ap.E) {  // two-pass assembly
+      ap.E[row * NB + j] = v;
+      if (j == 0) ap.Er[row] = red[0][NB][lr];
+    } else {
+      const int r = gn[row];
+      if (r >= nact) continue;
+      val[slots[row * NB + j]] += v;
+      if (j == 0) rhs[r] += red[0][NB][lr];
+    }
+  }
+}
+
+// One lane per (cell, local row i); the NB rows of a cell are consecutive
+// lanes of a flat index (cells may straddle wavefronts), and each wave of a
+// block takes every fourth point.  Per quadrature point the thread forms, in
+// the cell's reference frame,
 //   t_i = phi_i + delta beta.grad phi_i     (test function with the SUPG term)
 //   a_i = w (kappa .* grad phi_i + t_i beta),  c_i = w t_i c
 // so that row i of the local matrix of BilinearAssemble_SD / BilinearAssemble
@@ -974,19 +1031,21 @@ constexpr int cells_of_block(int NB) { return (kBlock + NB - 2) / NB + 1; }
 // physical gradients J^-T grad phi of THexaAffin (the cell frames are signed
 // axis permutations of the brick).  The mass matrix (what 1) is
 // A_ij += (w phi_i) phi_j with the rhs w f t_i, and the SUPG time-derivative
-// matrix (what 2) A_ij += (w delta beta.grad phi_i) phi_j.  Then the row is added into the CSR values through
-// the slot map (cells of one colour share no DOF).
-// LDS_TAB: the per-thread operands (phi_i and its gradient at every q) are
-// read from an LDS copy of the basis table made at the start of the block;
-// otherwise from the table in global memory.  VAR: coefficients that vary
-// over the cell (rotating convection, manufactured source, the caller's
-// values); without it the kernel carries none of their code (and none of its
-// registers).  The block first evaluates beta, the SUPG delta (a tanh, three
+// matrix (what 2) A_ij += (w delta beta.grad phi_i) phi_j.  Then the row goes
+// to the element-row buffer, or into the CSR values through the slot map
+// (cells of one colour share no DOF).
+// VAR: coefficients that vary over the cell (rotating convection, manufactured
+// source, the caller's values); without it the kernel carries none of their
+// code (and none of its registers).  The block first evaluates beta, the SUPG delta (a tanh, three
 // divisions) and the source once per point of its cells into LDS; evaluated by
 // each of a cell's NB rows they were most of the kernel (rotating field with
-// SUPG, Q2 24^3 and its three coarser levels 883 -> 476 us; manufactured
-// source, Q1 16^3, 143 -> 81 us).
-template <int P, bool LDS_TAB, bool VAR>
+// SUPG, Q2 24^3 and its three coarser levels 883 -> 476 us).  What is left is
+// the latency of the table reads point after point, so four waves share a
+// block's points (one wave through all 64: the coarse levels took 90 us each;
+// now 25-38, the four levels 303 us; manufactured source, Q1 16^3 143 -> 31
+// us).  A form with FP64 matrix products per 16 rows needs each row's operands
+// in four lanes and was slower (four levels 461 us, general hexahedra 2.8 ms).
+template <int P, bool VAR>
 __global__ __launch_bounds__(kBlock) void assemble_k(int ncells, const int *__restrict__ list,
                                                      const int4 *__restrict__ cells, const int *__restrict__ slots,
                                                      const int *__restrict__ gn, int nact,
@@ -996,19 +1055,16 @@ __global__ __launch_bounds__(kBlock) void assemble_k(int ncells, const int *__re
   constexpr int N1 = P + 2;
   constexpr int NQ = N1 * N1 * N1;
   constexpr int STRIDE = 4 + 4 * NB;
-  __shared__ double s_tab[LDS_TAB ? NQ * NB * 4 : 1];
-  if (LDS_TAB) {
-    for (int k = threadIdx.x; k < NQ * NB * 4; k += kBlock) s_tab[k] = tab[(k / (4 * NB)) * STRIDE + 4 + k % (4 * NB)];
-    __syncthreads();
-  }
-  const int64_t gid = (int64_t)blockIdx.x * kBlock + threadIdx.x;
+  const int lane = threadIdx.x & 63, wv = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int64_t row_lo = (int64_t)blockIdx.x * kElemRows, gid = row_lo + lane;
   const double nu = 1.0 / P;
   // VAR: beta, the SUPG delta and the source at the points of the block's cells
   constexpr int MC = cells_of_block(NB);
-  __shared__ double s_hc[VAR ? MC : 1], s_pt[VAR ? MC * NQ : 1][VAR ? 5 : 1];
-  const int c_lo = (int)((int64_t)blockIdx.x * kBlock / NB);
+  __shared__ double s_hc[VAR ? MC : 1], lds[elem_lds(NB, VAR ? MC * NQ * 5 : 0)];
+  double(*s_pt)[5] = (double(*)[5])lds;
+  const int c_lo = (int)(row_lo / NB);
   if constexpr (VAR) {
-    const int nc = min(ncells - c_lo, (int)(((int64_t)(blockIdx.x + 1) * kBlock - 1) / NB) - c_lo + 1);
+    const int nc = min(ncells - c_lo, (int)((row_lo + kElemRows - 1) / NB) - c_lo + 1);
     const bool vary = ap.qp || ap.conv_kind == 1;
     auto conv = [&](int c, int q, const int4 &cg, const int *dax, const int *sg, double *X, double *b) {
       if (ap.conv_kind == 1 || ap.f_kind == 1) brick_point(ap, P, cg, dax, sg, tab + q * STRIDE + 1, X);
@@ -1056,8 +1112,8 @@ __global__ __launch_bounds__(kBlock) void assemble_k(int ncells, const int *__re
     }
     __syncthreads();
   }
-  if (gid >= (int64_t)ncells * NB) return;
-  const int ci = (int)(gid / NB), i = (int)(gid % NB);
+  const bool row_on = gid < (int64_t)ncells * NB;
+  const int ci = row_on ? (int)(gid / NB) : c_lo, i = (int)(gid % NB);
   const int c = list ? list[ci] : ci;
   const int4 cg = cells[c];
   int dax[3], sg[3];
@@ -1084,11 +1140,15 @@ __global__ __launch_bounds__(kBlock) void assemble_k(int ncells, const int *__re
 #pragma unroll
   for (int j = 0; j < NB; j++) acc[j] = 0;
   double racc = 0;
-  for (int q = 0; q < NQ; q++) {
+  // the row's own operands one point ahead
+  const double *Tn = tab + wv * STRIDE + 4 + 4 * i;
+  double n0 = Tn[0], n1 = Tn[1], n2 = Tn[2], n3 = Tn[3];
+  for (int q = wv; q < NQ; q += kElemWaves) {
     const double *T = tab + q * STRIDE;
-    const double *Ti = LDS_TAB ? s_tab + (q * NB + i) * 4 : T + 4 + 4 * i;
     const double w = T[0] * detj;
-    const double phi_i = Ti[0], g0 = Ti[1], g1 = Ti[2], g2 = Ti[3];
+    const double phi_i = n0, g0 = n1, g1 = n2, g2 = n3;
+    Tn = tab + (q + kElemWaves < NQ ? q + kElemWaves : q) * STRIDE + 4 + 4 * i;
+    n0 = Tn[0], n1 = Tn[1], n2 = Tn[2], n3 = Tn[3];
     double cr = ap.c, f = ap.f_val;
     double delta = ap.supg ? ap.delta_const : 0.0;
     if constexpr (VAR) {
@@ -1112,41 +1172,20 @@ __global__ __launch_bounds__(kBlock) void assemble_k(int ncells, const int *__re
     }
     const double bg = beta[0] * g0 + beta[1] * g1 + beta[2] * g2;
     const double ti = phi_i + delta * bg;
-    if (ap.what == 1) {  // mass; rhs with the SUPG test function (MatrixMRhsAssemble_SUPG, TCD3D.C:48)
-      const double bw = w * phi_i;
-#pragma unroll
-      for (int j = 0; j < NB; j++) acc[j] = fma(bw, T[4 + 4 * j], acc[j]);
-      racc += w * f * ti;
-      continue;
-    }
-    if (ap.what == 2) {  // SUPG time-derivative matrix K (MatricesAKRhsAssemble_SUPG, TCD3D.C:102)
-      const double kw = w * (delta * bg);
-#pragma unroll
-      for (int j = 0; j < NB; j++) acc[j] = fma(kw, T[4 + 4 * j], acc[j]);
-      continue;
-    }
-    const double a0 = w * (kap[0] * g0 + ti * beta[0]);
-    const double a1 = w * (kap[1] * g1 + ti * beta[1]);
-    const double a2 = w * (kap[2] * g2 + ti * beta[2]);
-    const double cc = w * (ti * cr);
+    // mass: w phi_i phi_j, rhs with the SUPG test function
+    // (MatrixMRhsAssemble_SUPG, TCD3D.C:48); SUPG time-derivative matrix K
+    // (MatricesAKRhsAssemble_SUPG, TCD3D.C:102)
+    const bool full = ap.what == 0;
+    const double a0 = full ? w * (kap[0] * g0 + ti * beta[0]) : 0.0;
+    const double a1 = full ? w * (kap[1] * g1 + ti * beta[1]) : 0.0;
+    const double a2 = full ? w * (kap[2] * g2 + ti * beta[2]) : 0.0;
+    const double cc = full ? w * (ti * cr) : ap.what == 1 ? w * phi_i : w * (delta * bg);
 #pragma unroll
     for (int j = 0; j < NB; j++)
       acc[j] = fma(a0, T[5 + 4 * j], fma(a1, T[6 + 4 * j], fma(a2, T[7 + 4 * j], fma(cc, T[4 + 4 * j], acc[j]))));
     racc += w * f * ti;
   }
-  if (ap.E) {  // two-pass assembly: the element row, contiguously
-    const int64_t row = (int64_t)c * NB + i;
-#pragma unroll
-    for (int j = 0; j < NB; j++) ap.E[row * NB + j] = acc[j];
-    ap.Er[row] = racc;
-    return;
-  }
-  const int r = gn[c * NB + i];
-  if (r >= nact) return;
-  const int *sl = slots + ((int64_t)c * NB + i) * NB;
-#pragma unroll
-  for (int j = 0; j < NB; j++) val[sl[j]] += acc[j];
-  rhs[r] += racc;
+  element_rows_out<NB>(acc, racc, wv, lane, row_lo, (int64_t)ncells * NB, list, slots, gn, nact, ap, val, rhs, lds);
 }
 
 // The element kernel on general hexahedra (mapped hierarchies): the same
@@ -1158,8 +1197,8 @@ __global__ __launch_bounds__(kBlock) void assemble_k(int ncells, const int *__re
 // t_i = phi_i + delta beta . g_i keep the brick kernel's form
 // A_ij += a_i . g_j + c_i phi_j.  The SUPG delta uses the cell's mesh size in
 // convection direction from hconv[c] (hconv_geo_k, run before).  The geometry
-// is evaluated once per point of the block's cells, a chunk of points at a
-// time, into LDS (by each of a cell's rows: Q2 48^3 2.83 ms, so 2.20 ms).
+// is evaluated once per point of the block's cells into LDS (Q2 48^3 and
+// coarser levels: by each of a cell's rows 2.83 ms, so 1.76 ms).
 template <int P, bool VAR>
 __global__ __launch_bounds__(kBlock) void assemble_geo_k(int ncells, const int *__restrict__ list,
                                                          const int4 *__restrict__ cells, const int *__restrict__ slots,
@@ -1170,14 +1209,15 @@ __global__ __launch_bounds__(kBlock) void assemble_geo_k(int ncells, const int *
   constexpr int N1 = P + 2;
   constexpr int NQ = N1 * N1 * N1;
   constexpr int STRIDE = 4 + 4 * NB;
-  // K, w, beta (and, VAR, delta and f) at QC points at a time of the block's cells
-  constexpr int MC = cells_of_block(NB), QC = P == 1 ? 9 : 16, NV = VAR ? 15 : 13;
-  static_assert(NQ % QC == 0, "whole chunks of points");
-  __shared__ double s_pt[MC * QC][NV];
-  const int64_t gid = (int64_t)blockIdx.x * kBlock + threadIdx.x;
-  const int c_lo = (int)((int64_t)blockIdx.x * kBlock / NB);
-  const int nc = min(ncells - c_lo, (int)(((int64_t)(blockIdx.x + 1) * kBlock - 1) / NB) - c_lo + 1);
-  const bool row_on = gid < (int64_t)ncells * NB;  // (the other threads only help with the points)
+  // K, w, beta (and, VAR, delta and f) at the points of the block's cells
+  constexpr int MC = cells_of_block(NB), NV = VAR ? 15 : 13;
+  __shared__ double lds[elem_lds(NB, MC * NQ * NV)];
+  double(*s_pt)[NV] = (double(*)[NV])lds;
+  const int lane = threadIdx.x & 63, wv = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int64_t row_lo = (int64_t)blockIdx.x * kElemRows, gid = row_lo + lane;
+  const int c_lo = (int)(row_lo / NB);
+  const int nc = min(ncells - c_lo, (int)((row_lo + kElemRows - 1) / NB) - c_lo + 1);
+  const bool row_on = gid < (int64_t)ncells * NB;
   const int ci = row_on ? (int)(gid / NB) : c_lo, i = (int)(gid % NB);
   const int c = list ? list[ci] : ci;
   const double nu = 1.0 / P;
@@ -1189,9 +1229,9 @@ __global__ __launch_bounds__(kBlock) void assemble_geo_k(int ncells, const int *
 #pragma unroll
   for (int j = 0; j < NB; j++) acc[j] = 0;
   double racc = 0;
-  auto points = [&](int q0) {
-    for (int e = threadIdx.x; e < nc * QC; e += kBlock) {
-      const int lc = e / QC, q = q0 + e % QC, cp = list ? list[c_lo + lc] : c_lo + lc;
+  {
+    for (int e = threadIdx.x; e < nc * NQ; e += kBlock) {
+      const int lc = e / NQ, q = e % NQ, cp = list ? list[c_lo + lc] : c_lo + lc;
       const double *T = tab + q * STRIDE;
       TriMap M;
       tri_load(ap.vx, ap.nv, cells[cp], P, M);
@@ -1227,17 +1267,17 @@ __global__ __launch_bounds__(kBlock) void assemble_geo_k(int ncells, const int *
 #pragma unroll
       for (int x = 0; x < 3; x++) s_pt[e][10 + x] = b0 * K[0][x] + b1 * K[1][x] + b2 * K[2][x];
     }
-  };
-  for (int q = 0; q < NQ; q++) {
-    if (q % QC == 0) {
-      __syncthreads();
-      points(q);
-      __syncthreads();
-    }
-    const double *pt = s_pt[(ci - c_lo) * QC + q % QC];
+    __syncthreads();
+  }
+  // the row's own operands one point ahead
+  const double *Tn = tab + wv * STRIDE + 4 + 4 * i;
+  double n0 = Tn[0], n1 = Tn[1], n2 = Tn[2], n3 = Tn[3];
+  for (int q = wv; q < NQ; q += kElemWaves) {
+    const double *pt = s_pt[(ci - c_lo) * NQ + q];
     const double *T = tab + q * STRIDE;
-    const double *Ti = T + 4 + 4 * i;
-    const double phi_i = Ti[0], g0 = Ti[1], g1 = Ti[2], g2 = Ti[3];
+    const double phi_i = n0, g0 = n1, g1 = n2, g2 = n3;
+    Tn = tab + (q + kElemWaves < NQ ? q + kElemWaves : q) * STRIDE + 4 + 4 * i;
+    n0 = Tn[0], n1 = Tn[1], n2 = Tn[2], n3 = Tn[3];
     double eps = ap.eps, cr = ap.c, f = ap.f_val;
     double delta = delta_c;
     if (VAR) {
@@ -1261,45 +1301,21 @@ __global__ __launch_bounds__(kBlock) void assemble_geo_k(int ncells, const int *
     for (int a = 0; a < 3; a++) beta[a] = pt[10 + a];
     const double bg = beta[0] * g0 + beta[1] * g1 + beta[2] * g2;
     const double ti = phi_i + delta * bg;
-    if (ap.what == 1) {  // mass; rhs with the SUPG test function
-      const double bw = w * phi_i;
-#pragma unroll
-      for (int j = 0; j < NB; j++) acc[j] = fma(bw, T[4 + 4 * j], acc[j]);
-      racc += w * f * ti;
-      continue;
-    }
-    if (ap.what == 2) {  // SUPG time-derivative matrix K
-      const double kw = w * (delta * bg);
-#pragma unroll
-      for (int j = 0; j < NB; j++) acc[j] = fma(kw, T[4 + 4 * j], acc[j]);
-      continue;
-    }
     double G[3];  // physical gradient of phi_i
 #pragma unroll
     for (int d = 0; d < 3; d++) G[d] = K[d][0] * g0 + K[d][1] * g1 + K[d][2] * g2;
     double a[3];
 #pragma unroll
     for (int ax = 0; ax < 3; ax++) a[ax] = w * (eps * (K[0][ax] * G[0] + K[1][ax] * G[1] + K[2][ax] * G[2]) + ti * beta[ax]);
-    const double cc = w * (ti * cr);
+    if (ap.what != 0) a[0] = a[1] = a[2] = 0.0;
+    // mass, rhs with the SUPG test function; SUPG time-derivative matrix K
+    const double cc = ap.what == 0 ? w * (ti * cr) : ap.what == 1 ? w * phi_i : w * (delta * bg);
 #pragma unroll
     for (int j = 0; j < NB; j++)
       acc[j] = fma(a[0], T[5 + 4 * j], fma(a[1], T[6 + 4 * j], fma(a[2], T[7 + 4 * j], fma(cc, T[4 + 4 * j], acc[j]))));
     racc += w * f * ti;
   }
-  if (!row_on) return;
-  if (ap.E) {  // two-pass assembly: the element row, contiguously
-    const int64_t row = (int64_t)c * NB + i;
-#pragma unroll
-    for (int j = 0; j < NB; j++) ap.E[row * NB + j] = acc[j];
-    ap.Er[row] = racc;
-    return;
-  }
-  const int r = gn[c * NB + i];
-  if (r >= nact) return;
-  const int *sl = slots + ((int64_t)c * NB + i) * NB;
-#pragma unroll
-  for (int j = 0; j < NB; j++) val[sl[j]] += acc[j];
-  rhs[r] += racc;
+  element_rows_out<NB>(acc, racc, wv, lane, row_lo, (int64_t)ncells * NB, list, slots, gn, nact, ap, val, rhs, lds);
 }
 
 // per cell of a mapped level: the SUPG mesh size in convection direction,
@@ -2308,41 +2324,29 @@ void k_coarse_smooth(hipStream_t s, const DevLevel &L, double *x, const double *
   coarse_smooth_k<<<1, 64, sizeof(double) * L.ndof, s>>>(L.ndof, L.nact, L.rowptr, L.col, L.val, x, f, d, smoother,
                                                          omega, maxit, red);
 }
+// the element kernel of the order and the kind of cells
+static void launch_elements(hipStream_t s, bool var, int n, const int *list, const DevLevel &L, const double *tab,
+                            const AsmParams &ap, double *val, double *rhs) {
+  const int64_t rows = (int64_t)n * (ap.order == 1 ? 8 : 27);
+  const int grid = (int)((rows + kElemRows - 1) / kElemRows);
+  auto run = [&](auto kernel) {
+    kernel<<<grid, kBlock, 0, s>>>(n, list, L.cells, L.slots, L.gn, L.nact, tab, ap, val, rhs);
+  };
+  if (ap.order == 1) {
+    if (ap.vx) var ? run(assemble_geo_k<1, true>) : run(assemble_geo_k<1, false>);
+    else var ? run(assemble_k<1, true>) : run(assemble_k<1, false>);
+  } else {
+    if (ap.vx) var ? run(assemble_geo_k<2, true>) : run(assemble_geo_k<2, false>);
+    else var ? run(assemble_k<2, true>) : run(assemble_k<2, false>);
+  }
+}
+
 void k_assemble(hipStream_t s, const DevLevel &L, const double *tab, const AsmParams &ap, double *val, double *rhs,
                 int colour_begin, int colour_count) {
   if (colour_count <= 0) return;
   const int *list = L.colour_cells + colour_begin;
-  // CD3D_ASM_LDS_TAB=1: per-thread table operands from an LDS copy of the
-  // table (measured on the 64^3 Q2 level, constant SUPG coefficients: 9.3 ms
-  // per assembly against 6.7 ms from global memory: the 55 KB copy limits a
-  // CU to two workgroups and costs a staging pass per workgroup)
-  static const int lds_tab = [] {
-    const char *e = getenv("CD3D_ASM_LDS_TAB");
-    return e ? atoi(e) : 0;
-  }();
   const bool var = ap.conv_kind != 0 || ap.f_kind != 0 || ap.qp != nullptr;
-  const int64_t threads = (int64_t)colour_count * (ap.order == 1 ? 8 : 27);
-  const int grid = (int)((threads + kBlock - 1) / kBlock);
-  if (ap.vx) {  // general hexahedra
-    if (ap.order == 1) {
-      if (var) assemble_geo_k<1, true><<<grid, kBlock, 0, s>>>(colour_count, list, L.cells, L.slots, L.gn, L.nact, tab, ap, val, rhs);
-      else assemble_geo_k<1, false><<<grid, kBlock, 0, s>>>(colour_count, list, L.cells, L.slots, L.gn, L.nact, tab, ap, val, rhs);
-    } else {
-      if (var) assemble_geo_k<2, true><<<grid, kBlock, 0, s>>>(colour_count, list, L.cells, L.slots, L.gn, L.nact, tab, ap, val, rhs);
-      else assemble_geo_k<2, false><<<grid, kBlock, 0, s>>>(colour_count, list, L.cells, L.slots, L.gn, L.nact, tab, ap, val, rhs);
-    }
-    return;
-  }
-#define CD3D_ASM(P_, LDS_, VAR_) \
-  assemble_k<P_, LDS_, VAR_><<<grid, kBlock, 0, s>>>(colour_count, list, L.cells, L.slots, L.gn, L.nact, tab, ap, val, rhs)
-  if (ap.order == 1) {
-    if (lds_tab) { if (var) CD3D_ASM(1, true, true); else CD3D_ASM(1, true, false); }
-    else { if (var) CD3D_ASM(1, false, true); else CD3D_ASM(1, false, false); }
-  } else {
-    if (lds_tab) { if (var) CD3D_ASM(2, true, true); else CD3D_ASM(2, true, false); }
-    else { if (var) CD3D_ASM(2, false, true); else CD3D_ASM(2, false, false); }
-  }
-#undef CD3D_ASM
+  launch_elements(s, var, colour_count, list, L, tab, ap, val, rhs);
 }
 // CSR entry e of an active row: the sum of its element-row contributions in
 // colour order (gather lists of build_gather); active rhs entries likewise
@@ -2357,31 +2361,8 @@ __global__ __launch_bounds__(kBlock) void gather_entries_k(int64_t n, const int 
 }
 
 void k_assemble_rows(hipStream_t s, const DevLevel &L, const double *tab, const AsmParams &ap) {
-  const int nb = ap.order == 1 ? 8 : 27;
-  const int64_t threads = (int64_t)L.ncell * nb;
-  const int grid = (int)((threads + kBlock - 1) / kBlock);
-  if (ap.vx) {
-    if (ap.order == 1) {
-      if (ap.conv_kind != 0 || ap.f_kind != 0 || ap.qp)
-        assemble_geo_k<1, true><<<grid, kBlock, 0, s>>>(L.ncell, nullptr, L.cells, nullptr, L.gn, L.nact, tab, ap, nullptr, nullptr);
-      else
-        assemble_geo_k<1, false><<<grid, kBlock, 0, s>>>(L.ncell, nullptr, L.cells, nullptr, L.gn, L.nact, tab, ap, nullptr, nullptr);
-    } else {
-      if (ap.conv_kind != 0 || ap.f_kind != 0 || ap.qp)
-        assemble_geo_k<2, true><<<grid, kBlock, 0, s>>>(L.ncell, nullptr, L.cells, nullptr, L.gn, L.nact, tab, ap, nullptr, nullptr);
-      else
-        assemble_geo_k<2, false><<<grid, kBlock, 0, s>>>(L.ncell, nullptr, L.cells, nullptr, L.gn, L.nact, tab, ap, nullptr, nullptr);
-    }
-    return;
-  }
   const bool var = ap.conv_kind != 0 || ap.f_kind != 0 || ap.qp != nullptr;
-  if (ap.order == 1) {
-    if (var) assemble_k<1, false, true><<<grid, kBlock, 0, s>>>(L.ncell, nullptr, L.cells, nullptr, L.gn, L.nact, tab, ap, nullptr, nullptr);
-    else assemble_k<1, false, false><<<grid, kBlock, 0, s>>>(L.ncell, nullptr, L.cells, nullptr, L.gn, L.nact, tab, ap, nullptr, nullptr);
-  } else {
-    if (var) assemble_k<2, false, true><<<grid, kBlock, 0, s>>>(L.ncell, nullptr, L.cells, nullptr, L.gn, L.nact, tab, ap, nullptr, nullptr);
-    else assemble_k<2, false, false><<<grid, kBlock, 0, s>>>(L.ncell, nullptr, L.cells, nullptr, L.gn, L.nact, tab, ap, nullptr, nullptr);
-  }
+  launch_elements(s, var, L.ncell, nullptr, L, tab, ap, nullptr, nullptr);
 }
 
 void k_gather_assembly(hipStream_t s, const DevLevel &L, int64_t nnz_act, double *val, double *rhs) {
