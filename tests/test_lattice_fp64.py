@@ -168,3 +168,24 @@ def test_affine_columns_match_single_nodes(order, m, k0, levels, monkeypatch):
         for o in out[1:]:
             assert o[2:] == out[0][2:] and np.array_equal(o[0], out[0][0]) and np.array_equal(o[1], out[0][1])
     P.close()
+
+
+@pytest.mark.parametrize("order,m,k0,levels,prec,conv", [
+    (2, 3, 0, 3, "FP64", 0), (2, 3, 0, 3, "MIXED", 0), (1, 5, 0, 3, "FP64", 1),
+    (1, 5, 0, 3, "MIXED", 1), (2, 2, 0, 2, "MIXED", 1)])
+def test_reported_residual_is_the_csr_residual(order, m, k0, levels, prec, conv):
+    """rfinal from the class stencils against b - A x from the assembled CSR
+    matrix: both round at most 127 terms per row."""
+    P = pm.Problem(order, m, k0, levels, box=(1.0, 0.7, 0.5))
+    P.assemble(pm.coeffs(eps=0.05, b=(1.0, 0.5, 0.25), c=0.3, conv_kind=conv, f_val=1.0))
+    l = levels - 1
+    x, st = P.solve(pm.solver_params(precision=getattr(pm, prec), rel_tol=1e-6))
+    b = P.rhs(l)
+    rp, kc, e = P.csr(l)
+    row = np.repeat(np.arange(len(rp) - 1), np.diff(rp))
+    r = b - np.bincount(row, e * x[kc], len(rp) - 1)
+    mag = np.abs(b) + np.bincount(row, np.abs(e * x[kc]), len(rp) - 1)
+    tol = 2 * 127 * np.finfo(float).eps * np.linalg.norm(mag)
+    print(f"[gpu] rfinal {st.rfinal:.6e}, CSR {np.linalg.norm(r):.6e}, bound {tol:.1e}", flush=True)
+    assert abs(st.rfinal - np.linalg.norm(r)) < tol
+    P.close()
