@@ -562,14 +562,10 @@ static void refresh_f32(cd3d_problem &P, bool values = true) {
     D.invdiag_ok = D.gp_ok = false;  // only the FP64 smoothers read them: computed there on first use
     if (l == 0) D.lat_fresh = 0;  // the coarsest level has no FP32 stencils
     if (l > 0) {
-      auto per_node = [&](bool with_map) {  // per-node FP32 stencils (4 bytes per nonzero), on first need
+      auto per_node = [&]() {  // per-node FP32 stencils (4 bytes per nonzero), on first need
         if (!D.lval) {
           D.lval = dalloc<float>(P, (size_t)D.lat_nval);
           D.linv = dalloc<float>(P, (size_t)D.lat_nint);
-        }
-        if (with_map && !D.lperm) {
-          D.lperm = dalloc<int>(P, P.hl[l].lat_perm.size());
-          upload(P, D.lperm, P.hl[l].lat_perm);
         }
       };
       const long long nn = D.nn;
@@ -582,7 +578,7 @@ static void refresh_f32(cd3d_problem &P, bool values = true) {
         D.lat_exact64 = false;
         D.lat_aff64 = D.lat_alpha_m == 0.0 || D.lat_alpha_m == 1.0;
       } else if (D.lat_fresh == 2) {  // straight from the affine class stencils
-        per_node(false);
+        per_node();
         HIPCHK(kl_fill_lattice_affine(P.stream, D, D.lat_alpha_m, D.lat_alpha));
         D.lat_fresh = 0;
         D.lat_exact64 = false;
@@ -593,7 +589,7 @@ static void refresh_f32(cd3d_problem &P, bool values = true) {
         bool all_uniform = false;
         HIPCHK(kl_detect_uniform(P.stream, D, P.hflag, &all_uniform));
         if (!all_uniform) {
-          per_node(true);
+          per_node();
           HIPCHK(kl_convert(P.stream, D));
         }
       }

@@ -139,7 +139,6 @@ struct DevLevel {
   LatClass cls[8];
   int64_t lat_nval = 0, lat_nint = 0;
   float *lval = nullptr;       // stencil values f32
-  int *lperm = nullptr;        // CSR position of each stencil value (per-node FP32 path only)
   uint16_t *lsid = nullptr;    // stencil id of each active-row CSR entry
   int *lfirst = nullptr;       // CSR positions of each class's first node (8 x 128)
   float *linv = nullptr;       // 1/a_ii per interior node (class numbering)

@@ -1390,10 +1390,37 @@ __global__ __launch_bounds__(small_threads<P>()) void lat_small_k(SmallArgs<T> s
   for (int k = threadIdx.x; k < n3; k += NT) s.xout[k] = m[cx + k];
 }
 
-__global__ void lat_convert_k(long long n, const int *__restrict__ perm, const double *__restrict__ val,
-                              float *__restrict__ out) {
-  for (long long i = (long long)blockIdx.x * kB + threadIdx.x; i < n; i += (long long)gridDim.x * kB)
-    out[i] = (float)val[perm[i]];
+// CSR values to per-node FP32 stencils (class by class, stencil entry by
+// entry, nodes contiguous): a block transposes the rows of kConvNodes nodes of
+// one class through LDS, reading each row in CSR order with the stencil ids of
+// its entries.  Memory-bound (14 bytes per nonzero).  Read through the CSR
+// position of each stencil value, every lane took its 8 bytes from another
+// cache line (Q2 48^3 general hexahedra, 56 M values: 1.05 ms, so 0.27).
+constexpr int kConvNodes = 64;
+struct ConvTiles {
+  int start[9];  // first block of each class
+};
+__global__ __launch_bounds__(kB) void lat_convert_k(LatArgs a, ConvTiles tl, const int *__restrict__ node2dof,
+                                                    const int *__restrict__ rowptr,
+                                                    const uint16_t *__restrict__ sid, const double *__restrict__ val,
+                                                    float *__restrict__ out) {
+  __shared__ float v[(kCst - 1) * (kConvNodes + 1)];
+  int c = 0;
+  while (c + 1 < a.nclass && (int)blockIdx.x >= tl.start[c + 1]) c++;
+  const LatDev &C = a.c[c];
+  const long long k0 = (long long)((int)blockIdx.x - tl.start[c]) * kConvNodes;
+  const int nk = (int)(C.nodes - k0 < kConvNodes ? C.nodes - k0 : kConvNodes);
+  const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
+  const int rp = lane < nk ? rowptr[node2dof[C.first + k0 + lane]] : 0;
+#pragma unroll 4
+  for (int n = wv; n < kConvNodes; n += kB / 64) {
+    if (n >= nk) break;
+    const int b = __shfl(rp, n);
+    for (int e = lane; e < C.nsten; e += 64) v[(sid[b + e] & 127) * (kConvNodes + 1) + n] = (float)val[b + e];
+  }
+  __syncthreads();
+  if (lane < nk)
+    for (int s = wv; s < C.nsten; s += kB / 64) out[C.off + s * C.nodes + k0 + lane] = v[s * (kConvNodes + 1) + lane];
 }
 
 // Per class: the largest |a| of the first node's stencil (the scale of the
@@ -2380,7 +2407,11 @@ hipError_t kl_detect_uniform(hipStream_t s, DevLevel &L, int *flag_host, bool *a
 }
 
 hipError_t kl_convert(hipStream_t s, const DevLevel &L) {
-  lat_convert_k<<<2048, kB, 0, s>>>(L.lat_nval, L.lperm, L.val, L.lval);
+  const LatArgs a = lat_args(L);
+  ConvTiles tl{};
+  for (int c = 0; c < L.nclass; c++) tl.start[c + 1] = tl.start[c] + (int)((a.c[c].nodes + kConvNodes - 1) / kConvNodes);
+  if (tl.start[L.nclass] > 0)
+    lat_convert_k<<<tl.start[L.nclass], kB, 0, s>>>(a, tl, L.lnode2dof, L.rowptr, L.lsid, L.val, L.lval);
   lat_invdiag_k<<<(int)((L.lat_nint + kB - 1) / kB), kB, 0, s>>>(L.lat_nint, L.lnode2dof, L.diag, L.val, L.linv);
   return hipGetLastError();
 }
