@@ -494,9 +494,9 @@ def main():
     roof = roofline_entry(table, 1, "dominant kernel of the mixed step (with the Gram-Schmidt passes, "
                                     "lowsync_gs_step): the fine-level FP32 Jacobi sweep (algorithmic bytes: x, f "
                                     "and the result once, 12 bytes per node)")
-    mgs = roofline_entry(table, 7, "fused modified Gram-Schmidt step of the FP64 form's FGMRES on the fine level "
-                         "(32 bytes per unknown; the reference's Gram-Schmidt, one launch per basis vector)")
-    lowsync = roofline_entry(table, 9, "the mixed form's low-synchronisation Gram-Schmidt step at i = 10 on the "
+    mgs = roofline_entry(table, 7, "fused modified Gram-Schmidt step on the fine level (32 bytes per unknown; the "
+                         "reference's Gram-Schmidt, one launch per basis vector: restart lengths above 32)")
+    lowsync = roofline_entry(table, 9, "the low-synchronisation Gram-Schmidt step of FGMRES at i = 10 on the "
                              "fine level: one pass for the dots, one for w -= V h and |w|^2 ((2 i + 5) 8 bytes "
                              "per unknown)")
     asm = flop_roofline_entry(table, 8, "per-element quadrature (Gauss4, 64 points) of the Q2 SUPG element "
@@ -504,7 +504,7 @@ def main():
                               "gathered from its contributions; algorithmic flops n_cells n_q 8 n_b^2 per "
                               "assembly (the path for variable coefficients and general hexahedra)")
     spmv = roofline_entry(table, 0, "FP64 CSR SpMV of the fine level (12 nnz + 20 N bytes); the FP64 form's "
-                                    "smoother, defect and FGMRES product")
+                                    "smoother, defect and FGMRES product on levels without class stencils")
     extra = {}
     if not args.no_extra:
         log("[bench] 64^3 Q2 SUPG on general hexahedra (deformed 4^3 macro mesh)")

@@ -284,7 +284,7 @@ cd3d_status cd3d_write_matrix(cd3d_problem *p, int level, const char *path);
  * of the level with the coefficients of the last assembly, element rows
  * written out and gathered into a scratch CSR value array (CD3D_ASM_SCATTER=1:
  * the 8 colour-by-colour scatters): *bytes_per_launch then holds the
- * algorithmic FP64 flops of one pass, n_cells n_q 8 n_b^2; 9 the mixed form's
+ * algorithmic FP64 flops of one pass, n_cells n_q 8 n_b^2; 9 the
  * low-synchronisation Gram-Schmidt step at i = 10 on the finest level (dot
  * pass, coefficients, update pass: (2 i + 5) 8 N bytes).
  * Needs an assembled problem; the level vectors are overwritten. */

@@ -1851,8 +1851,11 @@ static void host_vec_op(cd3d_problem *p, int level, const double *in, double *ou
 // y = A x on device vectors in DOF order.  Where the assembled matrix is
 // exactly its class stencils the product goes through lattice order: x put in
 // order, the stencil product (16 bytes per unknown instead of 12 per nonzero),
-// the result put back.  Measured, CSR against lattice: MVFIGS
-// CD3D_MATVEC_LATTICE=0 keeps CSR.
+// the result put back.  Measured, CSR against lattice: Q2 24^3 (6.6 M nonzeros)
+// 19.8 against 12.4 us (rotating field 15.3), 48^3 141 against 28 (40), 64^3
+// 332 against 33-44 (84); Q1 64^3 (6.8 M) 19.3 against 15.3, 128^3 147 against
+// 50.  Below the line (Q2 20^3, 3.7 M: CSR 14.6 us) the two permutations and
+// three launches take what the product saves.  CD3D_MATVEC_LATTICE=0 keeps CSR.
 constexpr int64_t kLatMatvecMinNnz = 5000000;
 static void level_matvec(cd3d_problem &P, int level, const double *x, double *y) {
   DevLevel &L = P.dl[level];
