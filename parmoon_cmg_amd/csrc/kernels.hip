@@ -2354,8 +2354,20 @@ __global__ __launch_bounds__(kBlock) void gather_entries_k(int64_t n, const int 
                                                            const int *__restrict__ gidx,
                                                            const double *__restrict__ E, double *__restrict__ val) {
   for (int64_t e = (int64_t)blockIdx.x * kBlock + threadIdx.x; e < n; e += (int64_t)gridDim.x * kBlock) {
+    // at most 8 cells share an entry: the positions, then the values, all on
+    // their way before the first is added, in the same order (one after the
+    // other the values were waited for in turn: general hexahedra, Q2 48^3 and
+    // coarser levels 722 us, so 475)
+    const int k0 = gptr[e], m = gptr[e + 1] - k0;
+    int id[8];
+    double v[8];
+#pragma unroll
+    for (int u = 0; u < 8; u++) id[u] = u < m ? gidx[k0 + u] : -1;
+#pragma unroll
+    for (int u = 0; u < 8; u++) v[u] = id[u] >= 0 ? E[id[u]] : 0.0;
     double s = 0.0;
-    for (int k = gptr[e]; k < gptr[e + 1]; k++) s += E[gidx[k]];
+#pragma unroll
+    for (int u = 0; u < 8; u++) s = u < m ? s + v[u] : s;
     val[e] = s;
   }
 }
