@@ -1292,37 +1292,52 @@ struct SmallArgs {
 };
 static_assert(sizeof(SmallArgs<double>) <= 4096, "kernel arguments are limited to 4 KiB");
 
-// UNI: every class of the level has compact stencils (else per-node values)
+// node k of class c of a program's level, compact or per-node
+template <int P, int MODE, bool CMP, typename T>
+__host__ __device__ __attribute__((always_inline)) inline void small_class_node(const SmallLevel<T> &L, int c, int k,
+                                                                                const T *x, const T *f, T *out,
+                                                                                T omega) {
+  const T *cst = L.cst + c * kCst;
+  if (P == 1) {
+    lat_node<1, 0, 0, 0, MODE, CMP, T>(L.a, L.a.c[c], k, L.val, L.inv, cst, x, f, out, omega);
+  } else {
+    switch (c) {
+      case 0: lat_node<2, 0, 0, 0, MODE, CMP, T>(L.a, L.a.c[c], k, L.val, L.inv, cst, x, f, out, omega); break;
+      case 1: lat_node<2, 1, 0, 0, MODE, CMP, T>(L.a, L.a.c[c], k, L.val, L.inv, cst, x, f, out, omega); break;
+      case 2: lat_node<2, 0, 1, 0, MODE, CMP, T>(L.a, L.a.c[c], k, L.val, L.inv, cst, x, f, out, omega); break;
+      case 3: lat_node<2, 1, 1, 0, MODE, CMP, T>(L.a, L.a.c[c], k, L.val, L.inv, cst, x, f, out, omega); break;
+      case 4: lat_node<2, 0, 0, 1, MODE, CMP, T>(L.a, L.a.c[c], k, L.val, L.inv, cst, x, f, out, omega); break;
+      case 5: lat_node<2, 1, 0, 1, MODE, CMP, T>(L.a, L.a.c[c], k, L.val, L.inv, cst, x, f, out, omega); break;
+      case 6: lat_node<2, 0, 1, 1, MODE, CMP, T>(L.a, L.a.c[c], k, L.val, L.inv, cst, x, f, out, omega); break;
+      default: lat_node<2, 1, 1, 1, MODE, CMP, T>(L.a, L.a.c[c], k, L.val, L.inv, cst, x, f, out, omega); break;
+    }
+  }
+}
+// UNI: every class of every level of the program has a compact stencil; else
+// class by class, as the launched sweeps take it: only a level with a class
+// that varies has per-node values, and a program may hold levels of both
+// kinds (the one interior node of a 3^3-node level always counts as uniform)
+template <int P, int MODE, bool UNI, typename T>
+__host__ __device__ __attribute__((always_inline)) inline void small_node(const SmallLevel<T> &L, int c, int k,
+                                                                          const T *x, const T *f, T *out, T omega) {
+  if (UNI || L.a.uni[c]) small_class_node<P, MODE, true, T>(L, c, k, x, f, out, omega);
+  else small_class_node<P, MODE, false, T>(L, c, k, x, f, out, omega);
+}
+
 template <int P, int MODE, bool UNI, typename T>
 __device__ inline void small_sweep(const SmallLevel<T> &L, const T *x, const T *f, T *out, T omega) {
   const int lane = threadIdx.x & 63;
   int item = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), base = 0;
   for (int c = 0; c < L.a.nclass; c++) {
     const int nodes = (int)L.a.c[c].nodes, chunks = (nodes + 63) / 64;
-    const T *cst = L.cst + c * kCst;
     for (; item < base + chunks; item += small_threads<P>() / 64) {
       const int k = (item - base) * 64 + lane;
-      if (k >= nodes) continue;
-      if (P == 1) {
-        lat_node<1, 0, 0, 0, MODE, UNI, T>(L.a, L.a.c[c], k, L.val, L.inv, cst, x, f, out, omega);
-      } else {
-        switch (c) {
-          case 0: lat_node<2, 0, 0, 0, MODE, UNI, T>(L.a, L.a.c[c], k, L.val, L.inv, cst, x, f, out, omega); break;
-          case 1: lat_node<2, 1, 0, 0, MODE, UNI, T>(L.a, L.a.c[c], k, L.val, L.inv, cst, x, f, out, omega); break;
-          case 2: lat_node<2, 0, 1, 0, MODE, UNI, T>(L.a, L.a.c[c], k, L.val, L.inv, cst, x, f, out, omega); break;
-          case 3: lat_node<2, 1, 1, 0, MODE, UNI, T>(L.a, L.a.c[c], k, L.val, L.inv, cst, x, f, out, omega); break;
-          case 4: lat_node<2, 0, 0, 1, MODE, UNI, T>(L.a, L.a.c[c], k, L.val, L.inv, cst, x, f, out, omega); break;
-          case 5: lat_node<2, 1, 0, 1, MODE, UNI, T>(L.a, L.a.c[c], k, L.val, L.inv, cst, x, f, out, omega); break;
-          case 6: lat_node<2, 0, 1, 1, MODE, UNI, T>(L.a, L.a.c[c], k, L.val, L.inv, cst, x, f, out, omega); break;
-          default: lat_node<2, 1, 1, 1, MODE, UNI, T>(L.a, L.a.c[c], k, L.val, L.inv, cst, x, f, out, omega); break;
-        }
-      }
+      if (k < nodes) small_node<P, MODE, UNI, T>(L, c, k, x, f, out, omega);
     }
     base += chunks;
   }
 }
 
-// UNI: every small level has compact stencils in every class
 template <int P, bool UNI, typename T>
 __global__ __launch_bounds__(small_threads<P>()) void lat_small_k(SmallArgs<T> s) {
   extern __shared__ double small_lds[];
@@ -2617,11 +2632,11 @@ bool kl_small_ok(const DevLevel *levels, int top, long long max_nodes) {
 template bool kl_small_ok<float>(const DevLevel *, int, long long);
 template bool kl_small_ok<double>(const DevLevel *, int, long long);
 
+// the levels' part of the program's arguments; returns whether every class of
+// every level has a compact stencil
 template <typename T>
-void kl_small_vcycle(hipStream_t st, const DevLevel *levels, int top, int order, int pre, int post, T omega, T damp,
-                     const double *Ainv, const T *fin, T *xout) {
-  if (!kl_small_ok<T>(levels, top, 1LL << 40)) throw std::logic_error("levels too large for the one-workgroup V-cycle");
-  SmallArgs<T> s{};
+static bool small_levels(const DevLevel *levels, int top, SmallArgs<T> &s) {
+  bool uni = true;
   int w = 0;
   for (int i = 0; i <= top; i++) {
     const DevLevel &D = levels[i];
@@ -2635,22 +2650,29 @@ void kl_small_vcycle(hipStream_t st, const DevLevel *levels, int top, int order,
     s.L[i].f = w + n3;
     s.L[i].t = i ? w + 2 * n3 : w;
     w += (i ? 3 : 2) * n3;
+    for (int c = 0; i > 0 && c < D.nclass; c++) uni = uni && s.L[i].a.uni[c];
   }
   s.top = top;
+  s.words = w;
+  return uni;
+}
+
+template <typename T>
+void kl_small_vcycle(hipStream_t st, const DevLevel *levels, int top, int order, int pre, int post, T omega, T damp,
+                     const double *Ainv, const T *fin, T *xout) {
+  if (!kl_small_ok<T>(levels, top, 1LL << 40)) throw std::logic_error("levels too large for the one-workgroup V-cycle");
+  SmallArgs<T> s{};
+  const bool uni = small_levels<T>(levels, top, s);
   s.pre = pre;
   s.post = post;
   s.na = levels[0].nact;
-  s.words = w;
   s.omega = omega;
   s.damp = damp;
   s.Ainv = Ainv;
   s.dof2node0 = levels[0].ldof2node;
   s.fin = fin;
   s.xout = xout;
-  bool uni = true;
-  for (int i = 1; i <= top; i++)
-    for (int c = 0; c < s.L[i].a.nclass; c++) uni = uni && s.L[i].a.uni[c];
-  const size_t lds = sizeof(T) * w;
+  const size_t lds = sizeof(T) * s.words;
   if constexpr (sizeof(T) == 8) {
     if (order == 1) lat_small_k<1, true, T><<<1, small_threads<1>(), lds, st>>>(s);
     else lat_small_k<2, true, T><<<1, small_threads<2>(), lds, st>>>(s);
