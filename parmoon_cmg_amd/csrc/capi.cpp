@@ -1798,6 +1798,7 @@ cd3d_status cd3d_set_entries(cd3d_problem *p, int level, const double *entries) 
   return run(p, [&]() {
     HIPCHK(hipMemcpyAsync(p->dl[level].val, entries, sizeof(double) * p->dl[level].nnz, hipMemcpyHostToDevice,
                           p->stream));
+    p->dl[level].tcd_mass_uniform = false;  // a mass matrix of the caller's: time steps take it from CSR
     refresh_coarse_and_f32(*p);
     HIPCHK(hipStreamSynchronize(p->stream));
   });
