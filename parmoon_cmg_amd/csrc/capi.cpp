@@ -2178,7 +2178,9 @@ static int tcd_step_impl(cd3d_problem &P, const cd3d_coeffs &co0, const cd3d_sol
   // keeps its CSR system matrix for the exact coarse solve.
   const bool affine_asm = co.conv_kind == 1 && co.f_kind == 0 && !co.supg && !uniform_assembly_off(P);
   bool lattice = (sp.precision == CD3D_MIXED || fp64_lattice_on()) && Lf > 0 && affine_asm && sp.smoother == 1;
-  for (int l = 1; l <= Lf; l++) lattice = lattice && P.dl[l].tcd_mass_uniform && P.dl[l].nclass > 0;
+  // (per-point coefficients, also set after cd3d_tcd_init, are assembled cell by cell)
+  for (int l = 1; l <= Lf; l++)
+    lattice = lattice && P.dl[l].tcd_mass_uniform && P.dl[l].nclass > 0 && !P.dl[l].qp;
   // AssembleARhs at t_new (SystemTCD3D.C:204-226); with SUPG the A and rhs of
   // MatricesAKRhsAssemble_SUPG (TCD3D.C:102) and its time-derivative matrix
   // K, kept as M + K: the reference adds K to M for the rhs product and the

@@ -52,3 +52,24 @@ def test_mass_matrix_set_by_the_caller(order, m, levels, which, monkeypatch):
     if levels - 1 in which:
         assert rel(plain, ref) > 1e-4  # the change is seen
     assert rel(u64, ref) < 1e-8 and rel(u32, ref) < 1e-8
+
+
+# the values of a callback at the quadrature points, set after cd3d_tcd_init on
+# every level, on the finest alone, on the coarsest alone
+@pytest.mark.parametrize("order,m,levels,which", [(1, 2, 3, (0, 1, 2)), (1, 3, 2, (1,)), (2, 2, 2, (0, 1)), (2, 2, 3, (0,))])
+def test_point_coefficients_set_by_the_caller(order, m, levels, which, monkeypatch):
+    def change(P):
+        for l in which:
+            x = P.quad_points(l)
+            q = np.zeros(x.shape[:-1] + (6,))
+            q[..., 0] = 2e-3
+            q[..., 1] = -(x[..., 1] - 0.45)
+            q[..., 2] = x[..., 0] - 0.55
+            q[..., 3] = 0.3 * x[..., 2]
+            q[..., 4] = 0.5 * x[..., 0]
+            q[..., 5] = 1.0 + x[..., 1]
+            P.set_coeffs_qp(l, q)
+
+    ref, u64, u32 = states(order, m, levels, change, monkeypatch)
+    print(f"[gpu] points set on {which}: FP64 {rel(u64, ref):.1e}, mixed {rel(u32, ref):.1e}", flush=True)
+    assert rel(u64, ref) < 1e-8 and rel(u32, ref) < 1e-8
