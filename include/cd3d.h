@@ -168,7 +168,9 @@ cd3d_status cd3d_assemble(cd3d_problem *p, const cd3d_coeffs *co);
 
 /* MatVect / ScalarDefect on level l (Blas2.C:60,11), host vectors */
 cd3d_status cd3d_matvec(cd3d_problem *p, int level, const double *x_host, double *y_host);
-/* same on device buffers, on the handle's stream (asynchronous) */
+/* same on device buffers, on the handle's stream (asynchronous, without any
+ * allocation; on large levels assembled through class stencils the product is
+ * the stencils', a CSR row's sum in another order) */
 cd3d_status cd3d_matvec_dev(cd3d_problem *p, int level, const double *x_dev, double *y_dev);
 /* cd3d_matvec without any device allocation.  No counterpart in the reference:
  * it is for callers that cannot allocate device memory (tight serving loops,

@@ -128,6 +128,9 @@ static void check_macro_vertices(int m, const double *xyz) {
         }
 }
 
+// nonzeros from which a product goes through lattice order (level_matvec)
+constexpr int64_t kLatMatvecMinNnz = 5000000;
+
 static void setup_problem(cd3d_problem &P, const cd3d_mesh_desc &m, const double *macro_xyz = nullptr) {
   if (m.order != 1 && m.order != 2) throw ArgError("order must be 1 or 2");
   if (m.m < 1 || m.k0 < 0 || m.levels < 1 || m.levels > 12) throw ArgError("invalid mesh hierarchy");
@@ -267,6 +270,16 @@ static void setup_problem(cd3d_problem &P, const cd3d_mesh_desc &m, const double
     for (float **v : {&D.lx, &D.lf, &D.la, &D.lt}) {
       *v = dalloc<float>(P, nn3);  // boundary entries stay zero for good
       HIPCHK(hipMemsetAsync(*v, 0, sizeof(float) * nn3, P.stream));
+    }
+    if (!P.mapped && D.nnz >= kLatMatvecMinNnz) {
+      // the vectors of the caller's products through lattice order
+      // (level_matvec), with the matrix, so that no product allocates; without
+      // them the products keep CSR
+      try {
+        D.mv = dalloc<double>(P, 2 * (size_t)H.ndof);
+      } catch (const std::bad_alloc &) {
+        D.mv = nullptr;
+      }
     }
     HIPCHK(hipStreamSynchronize(P.stream));  // host vectors above go out of scope
   }
@@ -1856,17 +1869,16 @@ static void host_vec_op(cd3d_problem *p, int level, const double *in, double *ou
 // 19.8 against 12.4 us (rotating field 15.3), 48^3 141 against 28 (40), 64^3
 // 332 against 33-44 (84); Q1 64^3 (6.8 M) 19.3 against 15.3, 128^3 147 against
 // 50.  Below the line (Q2 20^3, 3.7 M: CSR 14.6 us) the two permutations and
-// three launches take what the product saves.  CD3D_MATVEC_LATTICE=0 keeps CSR.
-constexpr int64_t kLatMatvecMinNnz = 5000000;
+// three launches take what the product saves: kLatMatvecMinNnz, applied where
+// the vectors L.mv are allocated.  CD3D_MATVEC_LATTICE=0 keeps CSR.
 static void level_matvec(cd3d_problem &P, int level, const double *x, double *y) {
   DevLevel &L = P.dl[level];
   const char *e = getenv("CD3D_MATVEC_LATTICE");
   // (after cd3d_tcd_init the level matrices are not those of the stencils)
-  if (!P.assembled || !(L.lat_exact64 || L.lat_aff64) || L.nnz < kLatMatvecMinNnz || (e && e[0] == '0')) {
+  if (!P.assembled || !(L.lat_exact64 || L.lat_aff64) || !L.mv || (e && e[0] == '0')) {
     k_spmv(P.stream, L, x, y);
     return;
   }
-  if (!L.mv) L.mv = dalloc<double>(P, 2 * (size_t)L.ndof);
   kl_dof_to_lat64(P.stream, L, x, L.mv);
   kl_spmv64(P.stream, L, P.mesh.order, L.mv, L.mv + L.ndof);
   kl_lat64_to_dof(P.stream, L, L.mv + L.ndof, y);

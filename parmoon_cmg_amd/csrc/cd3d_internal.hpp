@@ -169,7 +169,7 @@ struct DevLevel {
   // (alpha (S0 + X SX + Y SY), or fma(alpha, that, M) with lat_alpha_m 1):
   // the FP64 lattice operator can stand for the matrix
   bool lat_aff64 = false;
-  double *mv = nullptr;  // two lattice-ordered vectors of the caller's products (first use)
+  double *mv = nullptr;  // two lattice-ordered vectors of the caller's products (large levels; null: CSR)
   bool tcd_mass_uniform = false;  // TCD3D: the mass class stencils are in lst64 (mass slot)
 };
 
