@@ -1905,8 +1905,7 @@ cd3d_status cd3d_internal_matvec_staged(cd3d_problem *p, int level, const double
   if (!p || !x || !y || !base || level < 0 || level >= (int)p->dl.size()) return CD3D_ERR_ARG;
   std::lock_guard<std::mutex> g(p->mu);
   return run(p, [&]() {
-    const DevLevel &L = p->dl[level];
-    const size_t n = (size_t)L.ndof, ld = (n + 31) / 32 * 32;
+    const size_t n = (size_t)p->dl[level].ndof, ld = (n + 31) / 32 * 32;
     if (2 * ld > capacity) {
       char b[200];
       snprintf(b, sizeof b,
@@ -1916,7 +1915,7 @@ cd3d_status cd3d_internal_matvec_staged(cd3d_problem *p, int level, const double
     }
     double *xd = base, *yd = base + ld;
     HIPCHK(hipMemcpyAsync(xd, x, sizeof(double) * n, hipMemcpyHostToDevice, p->stream));
-    k_spmv(p->stream, L, xd, yd);
+    level_matvec(*p, level, xd, yd);
     HIPCHK(hipGetLastError());
     HIPCHK(hipMemcpyAsync(y, yd, sizeof(double) * n, hipMemcpyDeviceToHost, p->stream));
     HIPCHK(hipStreamSynchronize(p->stream));

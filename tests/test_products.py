@@ -62,3 +62,17 @@ def test_captured_product_replays(large):
         assert np.array_equal(P.solution(), eager) and np.any(eager)
     ok(hip.hipGraphExecDestroy(ex))
     ok(hip.hipGraphDestroy(graph))
+
+
+@pytest.mark.parametrize("state", ["assembled", "entries set", "mass"])
+def test_staged_product_takes_the_same_route(large, state):
+    P = large
+    if state == "entries set":
+        P.set_entries(L, 2 * P.csr(L)[2])
+    if state == "mass":
+        P.tcd_init(pm.coeffs(eps=1e-3, conv_kind=1), 0.0, np.zeros(P.info(L)["ndof"]))
+    x = np.random.default_rng(9).standard_normal(P.info(L)["ndof"])
+    held = P.L.cd3d_device_bytes(P.h)
+    y = P.matvec_noalloc(L, x)
+    assert P.L.cd3d_device_bytes(P.h) == held
+    assert np.array_equal(y, P.matvec(L, x))
