@@ -96,7 +96,8 @@ typedef struct {
   int iterations;
   int status;           /* cd3d_status of the solve */
   double r0;            /* |b - A x0| */
-  double rfinal;        /* |b - A x| recomputed in FP64 after the solve */
+  double rfinal;        /* |b - A x| recomputed in FP64 after the solve: with the assembled CSR matrix (time
+                           steps that form no CSR system matrix: with the class stencils) */
   double ms_assemble;
   double ms_solve;
 } cd3d_stats;
