@@ -295,7 +295,11 @@ cd3d_status cd3d_kernel_bench(cd3d_problem *p, int which, int level, int reps, d
                               double *bytes_per_launch);
 
 /* device pointers of level vectors for timing and zero-copy callers:
- * which 0 = solution, 1 = rhs, 2 = scratch vector, 3 = scratch vector */
+ * which 0 = solution, 1 = rhs, 2 = scratch vector, 3 = scratch vector.
+ * After cd3d_solve vector 0 of the finest level is the solution, after
+ * cd3d_vcycle in the FP64 form vectors 0 and 1 are z and r, in DOF order.
+ * Solves, time steps and V-cycles use every other level vector as work space:
+ * they leave it in no particular state or order (DOF or lattice). */
 cd3d_status cd3d_device_ptr(cd3d_problem *p, int level, int which, double **dev);
 /* the handle's HIP stream (hipStream_t) */
 void *cd3d_stream(cd3d_problem *p);

@@ -935,6 +935,10 @@ void precondition(VC &v, const double *r, double *z, bool rhs_dirichlet_zero) {
     kl_from_dof<double>(P.stream, F, r, F.rhs);
     cycleL<double>(v, top, true);
     kl_to_dof<double>(P.stream, F, F.sol, z);
+    // the finest level's solution and rhs in DOF order, as the CSR form leaves
+    // them for zero-copy callers (solves do not come here: lattice64_space)
+    k_copy(P.stream, F.ndof, z, F.sol);
+    k_copy(P.stream, F.ndof, r, F.rhs);
     return;
   }
   k_copy(P.stream, F.ndof, r, F.rhs);
