@@ -51,6 +51,7 @@ struct ArgError : std::runtime_error {
 template <class T>
 T *dalloc(Problem &P, size_t count) {
   if (count == 0) count = 1;
+  if (P.dev_bytes + count * sizeof(T) > P.alloc_limit) throw std::bad_alloc();
   void *p = nullptr;
   hipError_t e = hipMalloc(&p, count * sizeof(T));
   if (e != hipSuccess) {
@@ -61,6 +62,16 @@ T *dalloc(Problem &P, size_t count) {
   P.alloc_bytes.push_back(count * sizeof(T));
   P.dev_bytes += count * sizeof(T);
   return (T *)p;
+}
+
+// null instead of an exception: buffers that a call can do without
+template <class T>
+T *dalloc_or_null(Problem &P, size_t count) {
+  try {
+    return dalloc<T>(P, count);
+  } catch (const std::bad_alloc &) {
+    return nullptr;
+  }
 }
 
 void dfree(Problem &P, void *ptr) {
@@ -275,11 +286,7 @@ static void setup_problem(cd3d_problem &P, const cd3d_mesh_desc &m, const double
       // the vectors of the caller's products through lattice order
       // (level_matvec), with the matrix, so that no product allocates; without
       // them the products keep CSR
-      try {
-        D.mv = dalloc<double>(P, 2 * (size_t)H.ndof);
-      } catch (const std::bad_alloc &) {
-        D.mv = nullptr;
-      }
+      D.mv = dalloc_or_null<double>(P, 2 * (size_t)H.ndof);
     }
     HIPCHK(hipStreamSynchronize(P.stream));  // host vectors above go out of scope
   }
@@ -296,6 +303,15 @@ static void setup_problem(cd3d_problem &P, const cd3d_mesh_desc &m, const double
 // basis column stride: a multiple of 32 doubles, so that every column is
 // 256-byte aligned (the vector kernels stream 16-byte pairs)
 static int64_t krylov_ld(int64_t N) { return (N + 31) / 32 * 32; }
+
+// the lattice-ordered iterate and rhs of FGMRES (first use); false: no room
+// for them, FGMRES in DOF order needs none
+static bool ensure_lat_vectors(cd3d_problem &P) {
+  const size_t N = (size_t)P.dl.back().ndof;
+  if (!P.xl) P.xl = dalloc_or_null<double>(P, N);
+  if (!P.bl) P.bl = dalloc_or_null<double>(P, N);
+  return P.xl && P.bl;
+}
 
 static void ensure_krylov(cd3d_problem &P, int restart) {
   if (restart <= P.krylov_restart) return;
@@ -696,21 +712,32 @@ static void ensure_gs(cd3d_problem &P, int l, bool backward) {
     std::vector<int> start, rows, col, pos;
     const int slots = build_gs_packed(P.hl[l], start, rows, col, pos), steps = (int)start.size() - 1;
     if (slots && k_gs_packed_fits(D.ndof, steps, slots)) {
-      D.gp_start = dalloc<int>(P, start.size());
-      D.gp_rows = dalloc<int>(P, rows.size());
-      D.gp_col = dalloc<int>(P, col.size());
-      D.gp_pos = dalloc<int>(P, pos.size());
-      D.gp_val = dalloc<double>(P, pos.size());
-      D.gp_inv = dalloc<double>(P, rows.size());
-      upload(P, D.gp_start, start);
-      upload(P, D.gp_rows, rows);
-      upload(P, D.gp_col, col);
-      upload(P, D.gp_pos, pos);
-      HIPCHK(hipStreamSynchronize(P.stream));  // the host vectors end here
-      D.gp_slots = slots;
-      D.gp_steps = steps;
-      D.gp_ok = false;
-      return;
+      D.gp_start = dalloc_or_null<int>(P, start.size());
+      D.gp_rows = dalloc_or_null<int>(P, rows.size());
+      D.gp_col = dalloc_or_null<int>(P, col.size());
+      D.gp_pos = dalloc_or_null<int>(P, pos.size());
+      D.gp_val = dalloc_or_null<double>(P, pos.size());
+      D.gp_inv = dalloc_or_null<double>(P, rows.size());
+      if (D.gp_start && D.gp_rows && D.gp_col && D.gp_pos && D.gp_val && D.gp_inv) {
+        upload(P, D.gp_start, start);
+        upload(P, D.gp_rows, rows);
+        upload(P, D.gp_col, col);
+        upload(P, D.gp_pos, pos);
+        HIPCHK(hipStreamSynchronize(P.stream));  // the host vectors end here
+        D.gp_slots = slots;
+        D.gp_steps = steps;
+        D.gp_ok = false;
+        return;
+      }
+      // no room for up to 2 KB per row: the schedule in memory, 4 bytes per row
+      for (int **q : {&D.gp_start, &D.gp_rows, &D.gp_col, &D.gp_pos}) {
+        dfree(P, *q);
+        *q = nullptr;
+      }
+      for (double **q : {&D.gp_val, &D.gp_inv}) {
+        dfree(P, *q);
+        *q = nullptr;
+      }
     }
   }
   for (int b = 0; b <= (backward ? 1 : 0); b++) {
@@ -936,7 +963,7 @@ void precondition(VC &v, const double *r, double *z, bool rhs_dirichlet_zero) {
     cycleL<double>(v, top, true);
     kl_to_dof<double>(P.stream, F, F.sol, z);
     // the finest level's solution and rhs in DOF order, as the CSR form leaves
-    // them for zero-copy callers (solves do not come here: lattice64_space)
+    // them for zero-copy callers (solves run in lattice64_space)
     k_copy(P.stream, F.ndof, z, F.sol);
     k_copy(P.stream, F.ndof, r, F.rhs);
     return;
@@ -1063,13 +1090,16 @@ Space lattice64_space(cd3d_problem &P) {
 
 int fgmres_iterate(cd3d_problem &P, const cd3d_solver_params &sp, const Space &S, double &r0, cd3d_status &status);
 
-// the buffers of the low-synchronisation Gram-Schmidt step (first use)
-void ensure_ls(cd3d_problem &P, int n) {
-  if (!P.ls_L) P.ls_L = dalloc<double>(P, (size_t)k_ls_max() * k_ls_max());
-  if (P.ls_blocks >= k_ls_blocks(n)) return;
+// the buffers of the low-synchronisation Gram-Schmidt step (first use); false:
+// no room for them, MGS vector by vector needs none
+bool ensure_ls(cd3d_problem &P, int n) {
+  if (!P.ls_L) P.ls_L = dalloc_or_null<double>(P, (size_t)k_ls_max() * k_ls_max());
+  if (!P.ls_L) return false;
+  if (P.ls_blocks >= k_ls_blocks(n)) return true;
   if (P.ls_part) dfree(P, P.ls_part);
-  P.ls_blocks = k_ls_blocks(n);
-  P.ls_part = dalloc<double>(P, (size_t)(2 * k_ls_max() + 1) * P.ls_blocks);
+  P.ls_part = dalloc_or_null<double>(P, (size_t)(2 * k_ls_max() + 1) * k_ls_blocks(n));
+  P.ls_blocks = P.ls_part ? k_ls_blocks(n) : 0;
+  return P.ls_part != nullptr;
 }
 
 // rfinal (optional): |b - A x| recomputed in the space after the iteration
@@ -1107,8 +1137,7 @@ int fgmres_iterate(cd3d_problem &P, const cd3d_solver_params &sp, const Space &S
   // 27.5 ms (5 us per launch of MGS whatever the size).
   const char *em = getenv("CD3D_FGMRES_MGS");
   const bool lowsync = !(em && em[0] == '1') && R <= k_ls_max() && ld % 2 == 0 && ((uintptr_t)V & 15) == 0 &&
-                       ((uintptr_t)w & 15) == 0;
-  if (lowsync) ensure_ls(P, N);
+                       ((uintptr_t)w & 15) == 0 && ensure_ls(P, N);
   // the finest lattice level's zero-start sweep written beside each Krylov
   // vector's FP32 copy (TopZeroSweep); CD3D_FUSE_ZERO_SWEEP=0: launched
   TopZeroSweep zt{};
@@ -1385,10 +1414,10 @@ static void batch_solve_impl(BatchRun &br, std::vector<BatchState> &st) {
     k_copy_range(P.stream, F.nact, F.ndof, P.bs, P.xs);
     HIPCHK(hipStreamSynchronize(P.stream));
   }
+  for (int b = 0; b < B; b++) lowsync = lowsync && ensure_ls(*br.ps[b], hp[b].n);
   if (lowsync)
     for (int b = 0; b < B; b++) {
       cd3d_problem &P = *br.ps[b];
-      ensure_ls(P, hp[b].n);
       hp[b].ls_part = P.ls_part;
       hp[b].ls_L = P.ls_L;
     }
@@ -1899,6 +1928,12 @@ cd3d_status cd3d_matvec(cd3d_problem *p, int level, const double *x, double *y) 
 
 }  // extern "C"
 
+// the handle allocates no more device memory than this (tests of calls that
+// find none)
+extern "C" void cd3d_internal_alloc_limit(cd3d_problem *p, size_t bytes) {
+  if (p) p->alloc_limit = bytes;
+}
+
 int cd3d_internal_device(const cd3d_problem *p) { return p ? p->device : -1; }
 
 // cd3d_matvec staged through a device buffer the caller holds (noalloc.hip):
@@ -2000,12 +2035,9 @@ cd3d_status cd3d_solve(cd3d_problem *p, const cd3d_solver_params *sp, const doub
     int its;
     const int top = (int)p->dl.size() - 1;
     const bool lat64 = lattice64_ok(*p, *sp);
-    if (lat64 ||
-        (sp->precision == CD3D_MIXED && top > 0 && sp->smoother == 1 && (F.lat_exact64 || F.lat_aff64))) {
-      if (!p->xl) {
-        p->xl = dalloc<double>(*p, N);
-        p->bl = dalloc<double>(*p, N);
-      }
+    if ((lat64 ||
+         (sp->precision == CD3D_MIXED && top > 0 && sp->smoother == 1 && (F.lat_exact64 || F.lat_aff64))) &&
+        ensure_lat_vectors(*p)) {
       kl_dof_to_lat64(p->stream, F, p->bs, p->bl);
       kl_dof_to_lat64(p->stream, F, p->xs, p->xl);
       its = fgmres(*p, *sp, lat64 ? lattice64_space(*p) : lattice_space(*p), r0, solve_status);
@@ -2201,6 +2233,7 @@ static int tcd_step_impl(cd3d_problem &P, const cd3d_coeffs &co0, const cd3d_sol
   // (per-point coefficients, also set after cd3d_tcd_init, are assembled cell by cell)
   for (int l = 1; l <= Lf; l++)
     lattice = lattice && P.dl[l].tcd_mass_uniform && P.dl[l].nclass > 0 && !P.dl[l].qp;
+  lattice = lattice && ensure_lat_vectors(P);
   // AssembleARhs at t_new (SystemTCD3D.C:204-226); with SUPG the A and rhs of
   // MatricesAKRhsAssemble_SUPG (TCD3D.C:102) and its time-derivative matrix
   // K, kept as M + K: the reference adds K to M for the rhs product and the
@@ -2232,10 +2265,6 @@ static int tcd_step_impl(cd3d_problem &P, const cd3d_coeffs &co0, const cd3d_sol
   k_axpy(P.stream, NA, tau * th4, F.rhs_asm, P.bs);
   HIPCHK(hipMemsetAsync(P.tcd_def, 0, sizeof(double) * N, P.stream));
   if (lattice) {
-    if (!P.xl) {
-      P.xl = dalloc<double>(P, N);
-      P.bl = dalloc<double>(P, N);
-    }
     kl_dof_to_lat64(P.stream, F, P.tcd_oldsol, P.xl);
     kl_affine64_apply(P.stream, F, P.mesh.order, -tau * th2, true, P.xl, P.bl);
     kl_lat64_to_dof(P.stream, F, P.bl, P.tcd_def);
@@ -2287,11 +2316,8 @@ static int tcd_step_impl(cd3d_problem &P, const cd3d_coeffs &co0, const cd3d_sol
   double r0;
   int its;
   const bool lat64 = lattice64_ok(P, sp);
-  if (lat64 || (sp.precision == CD3D_MIXED && Lf > 0 && sp.smoother == 1 && (F.lat_exact64 || F.lat_aff64))) {
-    if (!P.xl) {
-      P.xl = dalloc<double>(P, N);
-      P.bl = dalloc<double>(P, N);
-    }
+  if ((lat64 || (sp.precision == CD3D_MIXED && Lf > 0 && sp.smoother == 1 && (F.lat_exact64 || F.lat_aff64))) &&
+      ensure_lat_vectors(P)) {
     kl_dof_to_lat64(P.stream, F, P.bs, P.bl);
     kl_dof_to_lat64(P.stream, F, P.xs, P.xl);
     its = fgmres(P, sp, lat64 ? lattice64_space(P) : lattice_space(P), r0, solve_status, rf_out);
@@ -2651,7 +2677,7 @@ cd3d_status cd3d_kernel_bench(cd3d_problem *p, int which, int level, int reps, d
         if (level != (int)p->dl.size() - 1) throw ArgError("the Gram-Schmidt step runs on the finest level");
         constexpr int ii = 10;
         ensure_krylov(*p, 2 * ii);
-        ensure_ls(*p, L.ndof);
+        if (!ensure_ls(*p, L.ndof)) throw std::bad_alloc();
         if (p->krylov_ld % 2) throw std::logic_error("Krylov basis stride not a multiple of 2");
         HIPCHK(hipMemsetAsync(p->V, 0, sizeof(double) * (ii + 1) * p->krylov_ld, p->stream));
         HIPCHK(hipMemsetAsync(p->ls_L, 0, sizeof(double) * k_ls_max() * k_ls_max(), p->stream));

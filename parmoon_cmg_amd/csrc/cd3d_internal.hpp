@@ -196,7 +196,7 @@ struct Problem {
   // queues with other handles' main streams and hold them up)
   bool side_ok = true;
   int device = 0;
-  size_t dev_bytes = 0;
+  size_t dev_bytes = 0, alloc_limit = SIZE_MAX;
   std::vector<void *> allocs;
   std::vector<size_t> alloc_bytes;
   std::string err;
