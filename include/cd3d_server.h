@@ -87,9 +87,12 @@ typedef struct {
 
 void cd3d_server_default_params(cd3d_server_params *p);
 /* device bytes one problem of this mesh needs, as the admission control
- * counts them: hierarchy, lattice form, Krylov space of the given restart;
- * cellwise_assembly: variable coefficients (slot maps, per-node FP32
- * stencils); tcd: the TCD3D matrices and vectors (1 Galerkin, 2 SUPG: also
+ * counts them: hierarchy, lattice form, Krylov space of the given restart, for
+ * solves with the damped Jacobi smoother (a request with another smoother
+ * reserves its row schedules too, one that may be batched in the mixed form the
+ * batch's FP32 vectors);
+ * cellwise_assembly: variable coefficients (element rows and gather lists,
+ * per-node FP32 stencils); tcd: the TCD3D matrices and vectors (1 Galerkin, 2 SUPG: also
  * the time-derivative matrix K) */
 size_t cd3d_estimate_bytes(const cd3d_mesh_desc *mesh, int restart, int cellwise_assembly, int tcd);
 

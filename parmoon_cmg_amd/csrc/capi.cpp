@@ -1662,7 +1662,10 @@ void cd3d_default_solver(cd3d_solver_params *p) {
   p->cycle = 1;
 }
 
-size_t cd3d_estimate_bytes(const cd3d_mesh_desc *mesh, int restart, int cellwise_assembly, int tcd) {
+// smoother: that of the solves (2, 3 and 13 keep row schedules); batch32: the
+// FP32 level vectors of a mixed batch too
+static size_t estimate_bytes(const cd3d_mesh_desc *mesh, int restart, int cellwise_assembly, int tcd, int smoother,
+                             bool batch32) {
   if (!mesh || (mesh->order != 1 && mesh->order != 2) || mesh->m < 1 || mesh->k0 < 0 || mesh->levels < 1 ||
       mesh->levels > 12 || restart < 1)
     return 0;
@@ -1689,6 +1692,16 @@ size_t cd3d_estimate_bytes(const cd3d_mesh_desc *mesh, int restart, int cellwise
       b += 12.0 * nb * nb * ncell + 4 * nact_nnz + 12 * nb * ncell + 4 * N;
       if (l > 0) b += 8 * nact_nnz + 4 * na;          // per-node FP32 stencils and their CSR positions
     }
+    if (nnz >= (double)kLatMatvecMinNnz) b += 2 * 8 * N;  // lattice-ordered vectors of the products
+    if (l > 0 && (smoother == 2 || smoother == 3)) {
+      // rows by wavefront level: packed (build_gs_packed: 12 + 16 slots bytes
+      // per row) where x and the rhs fit a workgroup's LDS, else 4 bytes per
+      // row and direction
+      const double packed = na * (12 + 16.0 * (p == 1 ? 32 : 128)) + 4 * (na + 1);
+      b += 2 * 8 * N <= 160 * 1024 ? packed : (smoother == 3 ? 2 : 1) * 4 * (na + 1);
+    }
+    if (l > 0 && smoother == 13) b += 4 * na;  // rows by colour
+    if (batch32) b += 5 * 4 * N;
     if (tcd) b += 8 * nnz * (tcd == 2 ? 2 : 1);      // conv-diff matrix (and K with SUPG) beside the mass matrix
     total += b + (2 << 20);                         // allocation granularity of ~20 buffers
     if (l == 0) total += 8.0 * na * na + 8.0 * (double)gj_scratch_doubles(na);  // coarse inverse + Gauss-Jordan scratch
@@ -1696,9 +1709,14 @@ size_t cd3d_estimate_bytes(const cd3d_mesh_desc *mesh, int restart, int cellwise
     N_fine = N;
   }
   total += 8.0 * (2.0 * (restart + 1) * krylov_ld(N_fine) + 3.0 * N_fine);  // Krylov basis V, Z and w, xs, bs
+  total += 8.0 * 2.0 * N_fine;                      // FGMRES in lattice order: x and b
+  total += 8.0 * (k_ls_max() * k_ls_max() + (2 * k_ls_max() + 1) * (double)k_ls_blocks((int)N_fine));  // Gram-Schmidt
   if (tcd) total += 3 * 8.0 * N_fine;
   total += 8.0 * (4 * 1024 + 256) + 8.0 * 4096;     // reductions, scalars, basis tables
   return (size_t)total;
+}
+size_t cd3d_estimate_bytes(const cd3d_mesh_desc *mesh, int restart, int cellwise_assembly, int tcd) {
+  return estimate_bytes(mesh, restart, cellwise_assembly, tcd, 1, false);
 }
 
 cd3d_status cd3d_create(const cd3d_mesh_desc *mesh, cd3d_problem **out) {
@@ -1927,6 +1945,12 @@ cd3d_status cd3d_matvec(cd3d_problem *p, int level, const double *x, double *y) 
 }
 
 }  // extern "C"
+
+// cd3d_estimate_bytes for the solver of a served request
+size_t cd3d_internal_estimate_request(const cd3d_mesh_desc *mesh, int restart, int cellwise_assembly, int tcd,
+                                      int smoother, bool batch32) {
+  return estimate_bytes(mesh, restart, cellwise_assembly, tcd, smoother, batch32);
+}
 
 // the handle allocates no more device memory than this (tests of calls that
 // find none)

@@ -4,8 +4,8 @@
 // One scheduler thread admits queued requests in arrival order (a request
 // that does not fit may be overtaken at most max_bypass times) and hands
 // them to worker threads.  Device memory is accounted per hierarchy: an
-// admitted request first reserves the estimate (cd3d_estimate_bytes), and the
-// reservation is replaced by the hierarchy's real size once it has run.  Idle
+// admitted request first reserves the estimate (cd3d_estimate_bytes, for its
+// smoother), and the reservation is replaced by the hierarchy's real size once it has run.  Idle
 // hierarchies stay resident for later requests of the same mesh and are
 // evicted least recently used first when a new one needs room.
 #include <hip/hip_runtime.h>
@@ -27,6 +27,10 @@
 
 // capi.cpp: the handle's coarse inverse stays on its main stream
 void cd3d_internal_serving_handle(cd3d_problem *p);
+// capi.cpp: cd3d_estimate_bytes with the row schedules of smoothers 2, 3 and 13
+// and the vectors of a mixed batch
+size_t cd3d_internal_estimate_request(const cd3d_mesh_desc *mesh, int restart, int cellwise_assembly, int tcd,
+                                      int smoother, bool batch32);
 
 namespace {
 
@@ -99,7 +103,11 @@ struct cd3d_server {
     const bool cellwise = r.coeffs.conv_kind != 0 || r.coeffs.f_kind != 0;
     const int restart = std::max(1, std::min(r.solver.restart, r.solver.maxit));
     const int tcd = r.kind == CD3D_REQ_TCD ? (r.coeffs.supg ? 2 : 1) : 0;
-    return cd3d_estimate_bytes(&r.mesh, restart, cellwise ? 1 : 0, tcd);
+    // a solve that may continue with the multicolour smoother (run_request)
+    const bool robust = tcd == 0 && prm.robust_after > 0 && r.solver.smoother == 1 && r.solver.maxit > prm.robust_after;
+    const bool batch32 = tcd == 0 && prm.max_batch > 1 && r.solver.smoother == 1 && r.solver.precision == CD3D_MIXED;
+    return cd3d_internal_estimate_request(&r.mesh, restart, cellwise ? 1 : 0, tcd, robust ? 13 : r.solver.smoother,
+                                          batch32);
   }
 
   // evict idle hierarchies (least recently used first, never `keep`) until
