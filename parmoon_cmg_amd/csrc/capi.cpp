@@ -1690,7 +1690,7 @@ static size_t estimate_bytes(const cd3d_mesh_desc *mesh, int restart, int cellwi
     if (cellwise_assembly) {
       // two-pass assembly: element rows, their gather list and pointers, rhs lists
       b += 12.0 * nb * nb * ncell + 4 * nact_nnz + 12 * nb * ncell + 4 * N;
-      if (l > 0) b += 8 * nact_nnz + 4 * na;          // per-node FP32 stencils and their CSR positions
+      if (l > 0) b += 4 * nact_nnz + 4 * na;          // per-node FP32 stencils and their 1/a_ii
     }
     if (nnz >= (double)kLatMatvecMinNnz) b += 2 * 8 * N;  // lattice-ordered vectors of the products
     if (l > 0 && (smoother == 2 || smoother == 3)) {

@@ -61,7 +61,8 @@ def test_cellwise_solve_stays_within_the_reservation(mesh, prec):
         P.solve(sp, check=False)
     used, est = P.L.cd3d_device_bytes(P.h), reservation(mesh, co, sp)
     print(f"[gpu] {mesh} {prec}: device bytes {used / 2**20:.1f} MiB, reserved {est / 2**20:.1f}", flush=True)
-    assert used <= est
+    # 2 MiB per level of granularity; nothing that is not there (4 bytes per nonzero are 8 %)
+    assert used <= est <= 1.06 * used + 2 * mesh[3] * 2**20
     P.close()
 
 
