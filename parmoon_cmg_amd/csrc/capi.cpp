@@ -717,8 +717,8 @@ static void ensure_gs(cd3d_problem &P, int l, bool backward) {
       D.gp_col = dalloc_or_null<int>(P, col.size());
       D.gp_pos = dalloc_or_null<int>(P, pos.size());
       D.gp_val = dalloc_or_null<double>(P, pos.size());
-      D.gp_inv = dalloc_or_null<double>(P, rows.size());
-      if (D.gp_start && D.gp_rows && D.gp_col && D.gp_pos && D.gp_val && D.gp_inv) {
+      D.gp_diag = dalloc_or_null<double>(P, rows.size());
+      if (D.gp_start && D.gp_rows && D.gp_col && D.gp_pos && D.gp_val && D.gp_diag) {
         upload(P, D.gp_start, start);
         upload(P, D.gp_rows, rows);
         upload(P, D.gp_col, col);
@@ -734,7 +734,7 @@ static void ensure_gs(cd3d_problem &P, int l, bool backward) {
         dfree(P, *q);
         *q = nullptr;
       }
-      for (double **q : {&D.gp_val, &D.gp_inv}) {
+      for (double **q : {&D.gp_val, &D.gp_diag}) {
         dfree(P, *q);
         *q = nullptr;
       }

@@ -109,11 +109,11 @@ struct DevLevel {
   // the same sweeps with the iterate in LDS (levels whose vectors fit,
   // build_gs_packed): steps of at most kGsRows rows of one wavefront level,
   // their rows' off-diagonal entries packed in step order (gp_slots per row),
-  // the entries' CSR positions, and 1/a_ii; gp_ok: gp_val and gp_inv hold the
+  // the entries' CSR positions, and a_ii; gp_ok: gp_val and gp_diag hold the
   // values of `val`
   int gp_steps = 0, gp_slots = 0;
   int *gp_start = nullptr, *gp_rows = nullptr, *gp_col = nullptr, *gp_pos = nullptr;
-  double *gp_val = nullptr, *gp_inv = nullptr;
+  double *gp_val = nullptr, *gp_diag = nullptr;
   bool gp_ok = false;
   // assembly
   int4 *cells = nullptr;

@@ -2030,7 +2030,7 @@ __global__ __launch_bounds__(kGsBlock) void gs_sweep_k(int nlev, const int *__re
 // comes packed: steps of at most kGsRows independent rows, 16 lanes to a row
 // with EPL entries each, so nothing but the gather of x (LDS), a sum over 16
 // lanes (DPP) and one barrier lies between two steps; the entries of the step
-// four ahead are requested while a step runs (the barrier orders LDS only and
+// three ahead are requested while a step runs (the barrier orders LDS only and
 // leaves them in flight).  The backward sweep takes the steps in reverse: a
 // row's later-numbered neighbours are in later wavefront levels.
 // Bound by that chain, 0.25 us per step (Q1; Q2 0.34): assemble + solve Q1
@@ -2054,13 +2054,13 @@ __device__ inline double dpp_add(double v) {
 template <int EPL>
 struct GsSlot {
   int i, c[EPL];
-  double v[EPL], inv;
+  double v[EPL], d;
 };
 
 template <int EPL>
 __global__ __launch_bounds__(kBlock) void gs_packed_k(int n, int nact, int nsteps, const int *__restrict__ start,
                                                       const int *__restrict__ rows, const int *__restrict__ col,
-                                                      const double *__restrict__ val, const double *__restrict__ inv,
+                                                      const double *__restrict__ val, const double *__restrict__ dia,
                                                       double *__restrict__ x, const double *__restrict__ f,
                                                       double omega, int passes, int both, int zero) {
   static_assert(kBlock == 16 * kGsRows, "16 lanes per row of a step");
@@ -2091,7 +2091,7 @@ __global__ __launch_bounds__(kBlock) void gs_packed_k(int n, int nact, int nstep
   auto fetch = [&](GsSlot<EPL> &s, int b0, int e0) {
     const int r = b0 + g;
     s.i = -1;
-    s.inv = 0.0;
+    s.d = 1.0;
 #pragma unroll
     for (int k = 0; k < EPL; k++) {
       s.c[k] = 0;
@@ -2099,7 +2099,7 @@ __global__ __launch_bounds__(kBlock) void gs_packed_k(int n, int nact, int nstep
     }
     if (r < e0) {
       s.i = rows[r];
-      s.inv = inv[r];
+      s.d = dia[r];
       const unsigned at = ((unsigned)r * 16u + (unsigned)lane) * EPL;  // the packed rows fit 32 bits
 #pragma unroll
       for (int k = 0; k < EPL; k++) {
@@ -2132,7 +2132,7 @@ __global__ __launch_bounds__(kBlock) void gs_packed_k(int n, int nact, int nstep
 #pragma unroll
       for (int k = 0; k < EPL; k++) a = fma(q[s].v[k], w[k], a);
       a = dpp_add<0x121>(dpp_add<0x122>(dpp_add<0x124>(dpp_add<0x128>(a))));  // row_ror: the 16 lanes of the row
-      if (lane == 0 && q[s].i >= 0) xs[i] = omega * ((fi - a) * q[s].inv - xi) + xi;
+      if (lane == 0 && q[s].i >= 0) xs[i] = omega * ((fi - a) / q[s].d - xi) + xi;
       LdsFence::barrier();
     }
   }
@@ -2143,11 +2143,11 @@ __global__ __launch_bounds__(kBlock) void gs_packed_k(int n, int nact, int nstep
 __global__ __launch_bounds__(kBlock) void gs_pack_k(int64_t nslots, int nact, const int *__restrict__ pos,
                                                     const int *__restrict__ rows, const int *__restrict__ diag,
                                                     const double *__restrict__ a, double *__restrict__ val,
-                                                    double *__restrict__ inv) {
+                                                    double *__restrict__ dia) {
   for (int64_t k = blockIdx.x * (int64_t)kBlock + threadIdx.x; k < nslots; k += (int64_t)gridDim.x * kBlock) {
     const int p = pos[k];
     val[k] = p >= 0 ? a[p] : 0.0;
-    if (k < nact) inv[k] = 1.0 / a[diag[rows[k]]];
+    if (k < nact) dia[k] = a[diag[rows[k]]];
   }
 }
 
@@ -2237,14 +2237,14 @@ bool k_gs_packed_fits(int ndof, int steps, int slots) {
 void k_gs_pack(hipStream_t s, const DevLevel &L) {
   const int64_t n = (int64_t)L.nact * L.gp_slots;
   if (n > 0)
-    gs_pack_k<<<grid_for(n), kBlock, 0, s>>>(n, L.nact, L.gp_pos, L.gp_rows, L.diag, L.val, L.gp_val, L.gp_inv);
+    gs_pack_k<<<grid_for(n), kBlock, 0, s>>>(n, L.nact, L.gp_pos, L.gp_rows, L.diag, L.val, L.gp_val, L.gp_diag);
 }
 void k_gs_packed(hipStream_t s, const DevLevel &L, double *x, const double *f, double omega, int kind, int sweeps,
                  bool zero) {
   const size_t lds = gs_packed_lds(L.ndof, L.gp_steps);
   const int both = kind == 3, passes = both ? 2 * sweeps : sweeps;
   auto *k = L.gp_slots == 32 ? gs_packed_k<2> : gs_packed_k<8>;
-  k<<<1, kBlock, lds, s>>>(L.ndof, L.nact, L.gp_steps, L.gp_start, L.gp_rows, L.gp_col, L.gp_val, L.gp_inv, x, f, omega,
+  k<<<1, kBlock, lds, s>>>(L.ndof, L.nact, L.gp_steps, L.gp_start, L.gp_rows, L.gp_col, L.gp_val, L.gp_diag, x, f, omega,
                            passes, both, zero);
 }
 void k_restrict(hipStream_t s, const DevLevel &F, const DevLevel &C, const double *fine, double *coarse) {
