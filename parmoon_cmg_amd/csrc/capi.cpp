@@ -167,7 +167,7 @@ static void setup_problem(cd3d_problem &P, const cd3d_mesh_desc &m, const double
   const int L = m.levels;
   P.hl.resize(L);
   P.dl.resize(L);
-  for (int l = 0; l < L; l++) build_host_level(P.hl[l], m.order, m.m, m.k0 + l);
+  for (int l = 0; l < L; l++) build_host_level(P.hl[l], m.order, m.m, m.k0 + l, false);
   if (P.mapped) {
     std::vector<double> vx(macro_xyz, macro_xyz + 3 * (size_t)(m.m + 1) * (m.m + 1) * (m.m + 1)), t;
     int nv = m.m;

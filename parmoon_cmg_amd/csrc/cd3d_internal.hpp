@@ -67,7 +67,7 @@ struct HostLevel {
   // lattice-stencil form
   std::vector<LatClass> lat;
   int64_t lat_nval = 0;             // sum over classes of nsten * nodes
-  std::vector<int> lat_perm;        // CSR position of every stencil value
+  std::vector<int> lat_perm;        // CSR position of every stencil value (lat_positions only)
   std::vector<uint16_t> lat_sid;    // per active-row CSR entry: class * 128 + stencil entry
   std::vector<int> lat_first;       // CSR position of entry s of class c's first node (c * 128 + s)
   std::vector<int> lat_node2dof;    // interior node (class numbering) -> DOF
@@ -242,7 +242,9 @@ struct Problem {
 };
 
 // ---------------------------------------------------------------- setup (setup.cpp)
-void build_host_level(HostLevel &L, int order, int m, int depth);
+// lat_positions: also lat_perm (4 bytes per active nonzero), which the device
+// side does not use: the lattice map checked entry by entry on the host
+void build_host_level(HostLevel &L, int order, int m, int depth, bool lat_positions = true);
 // one regular refinement of an n^3 vertex lattice (edge, face and cell means)
 void refine_vertices(const std::vector<double> &src, int n, std::vector<double> &dst);
 void build_transfer(HostLevel &fine, const HostLevel &coarse, int order);
@@ -259,7 +261,7 @@ constexpr int kGsRows = 16;  // rows of one step of the packed schedule
 // CSR positions (padding: -1).  Returns slots (32 or 128), 0 when a row is too long
 int build_gs_packed(const HostLevel &L, std::vector<int> &start, std::vector<int> &rows, std::vector<int> &col,
                     std::vector<int> &pos);
-void build_lattice(HostLevel &L, int order);
+void build_lattice(HostLevel &L, int order, bool positions);
 void basis_tables(int order, std::vector<double> &tab);
 int quad_points_1d(int order);
 

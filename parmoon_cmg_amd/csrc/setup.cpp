@@ -107,7 +107,7 @@ void refine_vertices(const std::vector<double> &src, int n, std::vector<double> 
       }
 }
 
-void build_host_level(HostLevel &L, int order, int m, int depth) {
+void build_host_level(HostLevel &L, int order, int m, int depth, bool lat_positions) {
   const int p = order, nb = (p + 1) * (p + 1) * (p + 1);
   L.n = m << depth;
   L.ncell = L.n * L.n * L.n;
@@ -201,13 +201,14 @@ void build_host_level(HostLevel &L, int order, int m, int depth) {
   });
   build_colours(L, order);
   build_row_blocks(L.rowptr, kStreamNnz, kStreamRows, L.blk);
-  build_lattice(L, order);
+  build_lattice(L, order, lat_positions);
 }
 
-// Lattice-stencil form: classes, the CSR position of every stencil value and
-// the interior node -> DOF map.  Stencil entry order within a class: z, y, x
+// Lattice-stencil form: classes, the stencil id of every active CSR entry, the
+// interior node -> DOF map and, with positions, the CSR position of every
+// stencil value.  Stencil entry order within a class: z, y, x
 // offsets ascending (x fastest).
-void build_lattice(HostLevel &L, int order) {
+void build_lattice(HostLevel &L, int order, bool positions) {
   const int p = order, nn = L.nn;
   std::vector<int> node_dof((size_t)nn * nn * nn, -1);
   for (int d = 0; d < L.ndof; d++) node_dof[L.dof_node[d]] = d;
@@ -234,7 +235,7 @@ void build_lattice(HostLevel &L, int order) {
     L.lat.push_back(C);
   }
   L.lat_nval = off;
-  L.lat_perm.assign(off, -1);
+  L.lat_perm.assign(positions ? off : 0, -1);
   L.lat_node2dof.assign(first, -1);
   L.lat_sid.assign(off, 0);
   L.lat_first.assign(8 * 128, 0);
@@ -264,7 +265,7 @@ void build_lattice(HostLevel &L, int order) {
               continue;
             }
             const int pos = (int)(q - &L.kcol[0]);
-            L.lat_perm[C.off + (int64_t)s * C.nodes + k] = pos;
+            if (positions) L.lat_perm[C.off + (int64_t)s * C.nodes + k] = pos;
             L.lat_sid[pos] = (uint16_t)(c * 128 + s);
             if (k == 0) L.lat_first[c * 128 + s] = pos;
           }
