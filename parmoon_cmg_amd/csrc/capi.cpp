@@ -928,8 +928,8 @@ bool fp64_lattice_on() {
 // the rotating field, assembled through class stencils): the same matrices
 // and smoother in FP64, 16-24 bytes per unknown and product instead of 12
 // per nonzero (Q2 64^3 cells, fine level: CSR Jacobi sweep 350 us, 1.6 GB).
-// Assemble + solve Q2 64^3 79.5 -> 13.7 ms, three TCD3D steps Q1 128^3 34.8
-// -> 13.8 ms.  Other levels (per-point coefficients, general hexahedra,
+// Assemble + solve Q2 64^3: 79.6 ms on CSR, 11.2 here; three TCD3D steps Q1
+// 128^3: 34.6 and 10.5 ms.  Other levels (per-point coefficients, general hexahedra,
 // entries set by the caller) and smoothers keep the CSR form.
 bool lattice64_ok(const cd3d_problem &P, const cd3d_solver_params &sp) {
   if (sp.precision != CD3D_FP64 || P.dl.size() < 2 || sp.smoother != 1 || !fp64_lattice_on()) return false;
@@ -1001,9 +1001,9 @@ double dev_norm(cd3d_problem &P, int n, const double *a) {
 
 // TFgmresIte::Iterate, flexible branch (FgmresIte.C:219-595) on the finest
 // level: x (P.xs) and b (P.bs) on the device.  Returns the iteration count.
-// The vector space FGMRES runs in: DOF order with the CSR matrix (the plain
-// form), or node-lattice order with the class stencils (mixed form on a
-// constant-coefficient level); x and b are device vectors of that space.
+// The vector space FGMRES runs in: DOF order with the CSR matrix, or
+// node-lattice order with the class stencils (where the finest matrix is exactly
+// them, in either form); x and b are device vectors of that space.
 struct Space {
   int n;
   double *x, *b;

@@ -2033,10 +2033,13 @@ __global__ __launch_bounds__(kGsBlock) void gs_sweep_k(int nlev, const int *__re
 // three ahead are requested while a step runs (the barrier orders LDS only and
 // leaves them in flight).  The backward sweep takes the steps in reverse: a
 // row's later-numbered neighbours are in later wavefront levels.
-// Bound by that chain, 0.25 us per step (Q1; Q2 0.34): assemble + solve Q1
-// 16^3 cells (3375 rows, 849 levels) with SSOR 3 + 3, 39.8 -> 12.0 ms against
-// gs_sweep_k (x in L2, 1.0 us per level).  Measured and not kept: one wave with steps of 4
-// rows and no barrier (15.9 against 13.3 ms on the same problem at another
+// Bound by that chain, 0.27 us per step (Q1; Q2 0.37; the division is 8 % of
+// it): assemble + solve Q1 16^3 cells (3375 rows, 849 levels) with SSOR 3 + 3,
+// 39.9 -> 10.9 ms against gs_sweep_k (x in L2, 1.0 us per level).  Five
+// iterations with 3 + 3 sweeps, gs_sweep_k / this: SSOR Q1 8^3 cells 0.84 / 0.37
+// ms, 20^3 on 5^3 macro bricks 79 / 17.6; Q2 4^3 13.0 / 4.9, 10^3 on 5^3 101 /
+// 30.5; SOR in the same proportion.  Measured and not kept: one wave with steps
+// of 4 rows and no barrier (15.9 against 13.3 ms on the first problem at another
 // coefficient).  Levels beyond the LDS keep gs_sweep_k.
 struct LdsFence {
   static __device__ inline void barrier() {

@@ -1799,7 +1799,7 @@ __global__ void lat_fill_affine_k(LatArgs a, long long n, const double *__restri
 }
 
 // ------------------------------------------------------------------------
-// FP64 operator in lattice order for the outer FGMRES of the mixed form,
+// FP64 operator in lattice order for the FGMRES of both forms,
 // when the class stencils are exactly the assembled CSR values: interior
 // rows apply the class stencil, boundary (Dirichlet) rows are identity rows.
 
@@ -2266,7 +2266,8 @@ void lat_sweep(hipStream_t s, const DevLevel &L, int order, const T *x, const T 
     const int gq_g = eg ? atoi(eg) : 2, tb = et ? atoi(et) : 256, xcd = ex ? atoi(ex) : 1;
     const long long n = a.c[1].cnt[0];
     if constexpr (sizeof(T) == 8) {
-      // FP64: one pair per line (two pairs take 256 VGPRs, one wave per SIMD)
+      // FP64: one pair per line.  Sweep with one / two pairs, us: 97^3 nodes
+      // 10.9 / 16.4, 129^3 17.5 / 19.2, 161^3 33.3 / 32.7, 193^3 45.7 / 48.3
       lat_quad_gk<1, MODE, 256, T><<<(int)((n * n * n + 255) / 256), 256, 0, s>>>(a, v.cst, x, f, out, omega, xcd);
     } else {
       // G == 4 implies 2 divides the pairs per line too
@@ -2531,9 +2532,10 @@ void lat64_apply(hipStream_t s, const DevLevel &L, int order, const double *x, c
   if (order == 2 && grid > 0 && lat_pairs() && L.nn > kPairMinNN) {  // interior and Dirichlet rows in one launch
     const int G = pair_group(a, 2);
     if (G > 1 && lat_quads()) {
-      // measured on the 129^3-node level (FP64 product): quads of one pair
-      // 17.4 us (21.1 with the stencils in LDS), of two pairs 22.5 (256 VGPRs,
-      // one wave per SIMD), the pair-class kernel 27.0
+      // FP64 product, us: quads of one / two pairs (56 / 127 VGPRs) 97^3 nodes
+      // 10.3 / 15.6, 129^3 17.0 / 18.2, 161^3 29.6 / 28.3, 193^3 42.9 / 41.8: one
+      // pair, up to 4 % behind on the largest levels; 129^3 with the stencils in
+      // LDS 21.1 / 22.5, the pair-class kernel 27.0
       const char *ex = getenv("CD3D_QUAD_XCD"), *eg = getenv("CD3D_QUAD64_G");
       const int xcd = ex ? atoi(ex) : 1, gq = eg ? atoi(eg) : 1;
       const long long n = a.c[1].cnt[0];
