@@ -258,7 +258,7 @@ static void setup_problem(cd3d_problem &P, const cd3d_mesh_desc &m, const double
     D.colour_cells = dalloc<int>(P, H.colour_cells.size());
     upload(P, D.colour_cells, H.colour_cells);
     D.colour_start = H.colour_start;
-    // lattice-stencil form of the mixed-precision V-cycle
+    // lattice-stencil form of the V-cycle
     D.nn = H.nn;
     D.nclass = (int)H.lat.size();
     for (int c = 0; c < D.nclass; c++) D.cls[c] = H.lat[c];
@@ -649,8 +649,8 @@ struct VC {
   const cd3d_solver_params &sp;
   int rec[32];     // mg_recursions (TMultiGrid3D::SetRecursion, MultiGrid3D.C:690-703)
   int small = -1;  // the level whose zero-start visit runs as one launch (lattice V-cycles; 0: none)
-  // mixed V-cycle: bit i set when the restriction into level i also wrote
-  // its first pre-smoothing sweep from zero (into lt); CD3D_FUSE_ZERO_SWEEP=0
+  // lattice V-cycles: bit i set when the restriction into level i also wrote
+  // its first pre-smoothing sweep from zero (into LatVecs::t); CD3D_FUSE_ZERO_SWEEP=0
   // launches that sweep instead
   unsigned zero_ready = 0;
   bool fuse_zero = true;
@@ -1011,8 +1011,8 @@ struct Space {
   std::function<void(const double *, double *)> matvec;
   // precond(v, r, z, r32_state): z = M^-1 r; r32_state 1: r32 already holds
   // (float) r, written by the kernel that produced r; 2: that kernel also
-  // wrote the finest level's first pre-smoothing sweep from zero (into lt);
-  // 0: neither
+  // wrote the finest level's first pre-smoothing sweep from zero (into lt,
+  // FP64: tmp); 0: neither
   std::function<void(VC &, const double *, double *, int)> precond;
   float *r32 = nullptr;  // FP32 copy of the preconditioner input (lattice space)
   DevLevel *lat_top = nullptr;  // the finest level of the lattice V-cycle
@@ -1710,7 +1710,8 @@ static size_t estimate_bytes(const cd3d_mesh_desc *mesh, int restart, int cellwi
   }
   total += 8.0 * (2.0 * (restart + 1) * krylov_ld(N_fine) + 3.0 * N_fine);  // Krylov basis V, Z and w, xs, bs
   total += 8.0 * 2.0 * N_fine;                      // FGMRES in lattice order: x and b
-  total += 8.0 * (k_ls_max() * k_ls_max() + (2 * k_ls_max() + 1) * (double)k_ls_blocks((int)N_fine));  // Gram-Schmidt
+  total += 8.0 * (k_ls_max() * k_ls_max() +        // Gram-Schmidt
+                  (2 * k_ls_max() + 1) * (double)k_ls_blocks((int)std::min(N_fine, 2e9)));
   if (tcd) total += 3 * 8.0 * N_fine;
   total += 8.0 * (4 * 1024 + 256) + 8.0 * 4096;     // reductions, scalars, basis tables
   return (size_t)total;
@@ -2695,7 +2696,7 @@ cd3d_status cd3d_kernel_bench(cd3d_problem *p, int which, int level, int reps, d
         b = 32 * N;
         break;
       case 9: {
-        // the mixed form's low-synchronisation Gram-Schmidt step at i = 10
+        // the low-synchronisation Gram-Schmidt step at i = 10
         // (dot pass, coefficients, update pass) on the finest level, over a
         // zero basis: (i + 2) + (i + 3) vectors of 8 N bytes
         if (level != (int)p->dl.size() - 1) throw ArgError("the Gram-Schmidt step runs on the finest level");

@@ -1,9 +1,10 @@
 // Internal data structures of libcd3d_hip.so.
 //
 // Layout in device memory (HBM), per multigrid level l:
-//   CSR  rowptr int32[N+1], col int32[nnz], val f64[nnz] (+ val32 f32[nnz] for
-//        the mixed-precision V-cycle), diag int32[N] (position of a_ii)
-//   vectors f64[N]: sol, rhs, aux (defect / correction), tmp (Jacobi buffer)
+//   CSR  rowptr int32[N+1], col int32[nnz], val f64[nnz], diag int32[N]
+//        (position of a_ii)
+//   vectors f64[N]: sol, rhs, aux (defect / correction), tmp (Jacobi buffer);
+//            in lattice order inside the FP64 lattice V-cycle
 //            f32[N]: the same four for the mixed-precision V-cycle
 //   transfer from level l-1: P (fine rows, CSR) and R = P^T (coarse rows, CSR)
 //   assembly: cell geometry int4[ncell] (origin in node units + frame code),
@@ -25,7 +26,7 @@
 
 namespace cd3d {
 
-// Lattice-stencil form of a level (mixed-precision V-cycle): interior nodes
+// Lattice-stencil form of a level (V-cycles of both forms): interior nodes
 // of the node lattice split into parity classes; class c holds the box of
 // nodes with X % 2 == px (Q2; one class for Q1), each with the same stencil
 // (per axis offsets -p..p on cell-face planes, the cell's p+1 nodes inside a
@@ -133,7 +134,7 @@ struct DevLevel {
   double *hconv = nullptr;
   double h[3] = {0, 0, 0};   // cell sides
   double dn[3] = {0, 0, 0};  // node spacing
-  // lattice-stencil form (mixed-precision V-cycle)
+  // lattice-stencil form
   int nn = 0;                  // nodes per side
   int nclass = 0;
   LatClass cls[8];
