@@ -259,7 +259,8 @@ cd3d_status cd3d_interpolate(cd3d_problem *p, int level, int fn, const cd3d_coef
  * errors[2] = max |u - fn| at the last cell's points (what the reference
  * leaves in its third entry), errors[3] = max |u - fn| at all points.
  * u_host NULL: the level's current solution on the device (finest level: the
- * last cd3d_solve, or the TCD3D state after cd3d_tcd_init). */
+ * last cd3d_solve, or the TCD3D state after cd3d_tcd_init; coarser levels'
+ * vectors are work space of the solver, see cd3d_device_ptr). */
 cd3d_status cd3d_errors(cd3d_problem *p, int level, const double *u_host, int fn, const cd3d_coeffs *co,
                         double *errors);
 /* TOutput3D::WriteVtk (Output3D.C:1747): legacy ASCII VTK of level l with the
